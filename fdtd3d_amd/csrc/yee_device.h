@@ -101,6 +101,27 @@ __device__ __forceinline__ bool half_cell (const StepArgs<T> &a, int &i, int &j,
   return j < a.run_hi[1] && k >= a.run_lo[2] && k < a.run_hi[2];
 }
 
+// The same for a launch over several boxes: the box whose tile rows hold blockIdx / 8 (a uniform
+// scan of at most 20 records), then its tile in the XCD's band.  A tile may span several planes
+// (a y face is one row high).
+__device__ __forceinline__ bool half_cell_boxes (const HalfBox *box, int nbox, int &i, int &j, int &k)
+{
+  const int b = (int) blockIdx.x;
+  const int r = b >> 3;
+  int s = nbox - 1;
+  while (s > 0 && r < box[s].first) --s;
+  const HalfBox x = box[s];
+  const int u = (b & 7) * x.per_xcd + (r - x.first);
+  if (r - x.first >= x.per_xcd || u >= x.ntile) return false;
+  const int t = u / x.ntx;
+  const int ty = t / x.ntz;
+  const int tid = (int) threadIdx.x, lbx = 8 - x.lbz - x.lby;
+  k = x.tz0 + ((t - ty * x.ntz) << x.lbz) + (tid & ((1 << x.lbz) - 1));
+  j = x.lo[1] + (ty << x.lby) + ((tid >> x.lbz) & ((1 << x.lby) - 1));
+  i = x.lo[0] + ((u - t * x.ntx) << lbx) + (tid >> (x.lbz + x.lby));
+  return i < x.hi[0] && j < x.hi[1] && k >= x.lo[2] && k < x.hi[2];
+}
+
 // Direct-update coefficient cb = dt / (m m0 dx) of computeCaCb (InternalScheme.inc.h:2340-2344).
 // FP64 divides exactly (the reference's operations); FP32 multiplies by the hardware reciprocal
 // (1 ulp), several times cheaper than an IEEE division and far inside the FP32 tolerance.

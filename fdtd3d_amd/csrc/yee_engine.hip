@@ -36,7 +36,8 @@ template <typename T> __global__ void point_source (T *, int64_t, double);
 template <typename T> __global__ void tfsf_mask_kernel (StepArgs<T>, int, int, uint8_t *);
 template <typename T, int COMP, int DIM> __global__ void scattered_kernel (StepArgs<T>, const T *, double *, int, int64_t, int64_t);
 template <typename T, int BY, int MAT, int MAXW> __global__ void step_3d_fused (StepArgs<T>);
-template <typename T> __global__ void tfsf_ztable (StepArgs<T>, double *);
+template <typename T, int MODE> __global__ void e_boxes (StepArgs<T>, const HalfBox *, int, int, double *);
+template <typename T, int MODE> __global__ void h_boxes (StepArgs<T>, const HalfBox *, int);
 template <typename T> __global__ void test_fill (StepArgs<T>, T *, int, int, double, int);
 template <typename T> __global__ void ntff_faces (NtffArgs<T>);
 template <typename T>
@@ -88,6 +89,36 @@ enum ArgRole
   kRoleH,       // H update: new E, old H -> new H
   kRoleFused,   // whole step: old E, old H -> new E, new H
 };
+
+// Hard point-source value of the E (t + 1/2) or H (t + 1) update of step t
+// (performPointSourceCalc, InternalScheme.inc.h:2818-2895), with the C library's sin.
+double source_value (const yee_handle *h, bool e_half, int32_t t)
+{
+  const double ts = e_half ? t + 0.5 : t + 1.0;
+  // the complex build's point source is (sin, cos) of the same argument (InternalScheme.inc.h:2888-2893)
+  const double arg = h->sc.dt * ts * 2 * kPi * h->sc.freq;
+  double v = h->src_kind == 2 ? std::cos (arg) : std::sin (arg);
+  if (h->src_sigma > 0)
+  {
+    const double u = (ts - h->src_t0) / h->src_sigma;
+    v *= std::exp (-u * u);
+  }
+  return v;
+}
+
+// The hard source lies on a cell the half-step kernels update, which then store its value
+// themselves.  (Runs with test functions take the border values and norms between the update
+// and the source, so there it stays a launch of its own.)
+bool source_in_update (const yee_handle *h)
+{
+  if (!(h->cfg.point_source & 0x3fu) || h->fn_any ()) return false;
+  for (int ax = 0; ax < h->dim; ++ax)
+  {
+    const int64_t p = h->cfg.point_source_pos[ax];
+    if (h->lack[ax] ? p != 0 : (p < 1 || p >= h->n[ax] - 1)) return false;
+  }
+  return true;
+}
 
 template <typename T>
 StepArgs<T> make_args (const yee_handle *h, int parity, ArgRole role = kRoleE)
@@ -144,6 +175,12 @@ StepArgs<T> make_args (const yee_handle *h, int parity, ArgRole role = kRoleE)
     else if (h->src_kind == 1) current = std::cos (h->sc.dt * (ts - 1) * 2 * kPi * h->sc.freq);
     else current = -std::sin (h->sc.dt * (ts - 1) * 2 * kPi * h->sc.freq);
     a.cur_val = current * mu0 () / h->sc.dt / 2.0;
+  }
+  if (source_in_update (h))
+  {
+    a.src_mask = h->cfg.point_source & 0x3fu;
+    for (int ax = 0; ax < 3; ++ax) a.src_pos[ax] = ax < h->dim ? (int) h->cfg.point_source_pos[ax] : 0;
+    a.src_val = source_value (h, role != kRoleH, h->t);
   }
   a.sz = 1;
   for (int m = 0; m < 3; ++m)
@@ -207,15 +244,9 @@ StepArgs<T> make_args (const yee_handle *h, int parity, ArgRole role = kRoleE)
 
 
 template <typename T>
-int launch_half (yee_handle *h, bool e_half, int parity, const int64_t *lo = nullptr, const int64_t *hi = nullptr)
+int launch_half (yee_handle *h, bool e_half, int parity)
 {
   StepArgs<T> a = make_args<T> (h, parity, e_half ? kRoleE : kRoleH);
-  if (lo)
-    for (int ax = 0; ax < 3; ++ax)
-    {
-      a.run_lo[ax] = (int) lo[ax];
-      a.run_hi[ax] = (int) hi[ax];
-    }
   if (h->dim == 3)
   {
     const int64_t ext[3] = { a.run_hi[0] - a.run_lo[0], a.run_hi[1] - a.run_lo[1], a.run_hi[2] - a.run_lo[2] };
@@ -288,22 +319,6 @@ int launch_half (yee_handle *h, bool e_half, int parity, const int64_t *lo = nul
   return YEE_OK;
 }
 
-// Hard point-source value of the E (t + 1/2) or H (t + 1) update of step t
-// (performPointSourceCalc, InternalScheme.inc.h:2818-2895), with the C library's sin.
-double source_value (const yee_handle *h, bool e_half, int32_t t)
-{
-  const double ts = e_half ? t + 0.5 : t + 1.0;
-  // the complex build's point source is (sin, cos) of the same argument (InternalScheme.inc.h:2888-2893)
-  const double arg = h->sc.dt * ts * 2 * kPi * h->sc.freq;
-  double v = h->src_kind == 2 ? std::cos (arg) : std::sin (arg);
-  if (h->src_sigma > 0)
-  {
-    const double u = (ts - h->src_t0) / h->src_sigma;
-    v *= std::exp (-u * u);
-  }
-  return v;
-}
-
 // A cell next to an x or y face of the TF/SF box (the kAxFRange / kAxFPlane bits of the fused
 // kernel): inside [L-1, R] on every axis and on one of the planes L-1, R-1, R of x or y.
 bool tfsf_near_host (const yee_handle *h, const int64_t p[3])
@@ -337,11 +352,12 @@ bool source_in_fused_box (const yee_handle *h)
   return (h->cfg.point_source & 0x3fu) && fused_owns_host (h, h->cfg.point_source_pos);
 }
 
-// Point sources as separate one-cell launches into buffer `buf`; with the fused step the
-// sources inside its box are applied by that kernel instead (skip_box).
+// Point sources as separate one-cell launches into buffer `buf`: at t = 0, where no field is
+// updated, and on cells the half-step kernels do not update.
 template <typename T>
-int launch_sources (yee_handle *h, bool e_half, int32_t t, int buf, bool skip_box)
+int launch_sources (yee_handle *h, bool e_half, int32_t t, int buf)
 {
+  if (t > 0 && source_in_update (h)) return YEE_OK;
   const int c0 = e_half ? 0 : 3;
   for (int c = c0; c < c0 + 3; ++c)
   {
@@ -350,7 +366,6 @@ int launch_sources (yee_handle *h, bool e_half, int32_t t, int buf, bool skip_bo
     const int64_t pz = h->dim == 3 ? p[2] : 0;
     // getFieldValueOrNullByAbsolutePos: positions outside the grid are ignored
     if (p[0] < 0 || p[0] >= h->n[0] || p[1] < 0 || p[1] >= h->n[1] || pz < 0 || pz >= h->n[2]) continue;
-    if (skip_box && source_in_fused_box (h)) continue;
     const int64_t q = (p[0] * h->n[1] + p[1]) * h->n[2] + pz;
     hipLaunchKernelGGL ((point_source<T>), dim3 (1), dim3 (64), 0, h->stream, (T *) h->f[buf][c], q,
                        source_value (h, e_half, t));
@@ -459,69 +474,123 @@ int face_boxes (const yee_handle *h, int64_t lo[9][3], int64_t hi[9][3])
   return m;
 }
 
-// One time step (t > 0) with the fused kernel: E of the PML slabs and TF/SF faces, E sources
-// the fused kernel does not own, fused E+H sweep, H of the slabs and faces, H sources; old
-// state in buffer cur, new state in 1 - cur.
-template <typename T>
-int fused_step (yee_handle *h, int32_t t, int prev)
+// The boxes of the half-step launches around the fused kernel: the PML slabs, the TF/SF x / y
+// faces, the Drude box, the cells of the point source and of the current source (the fused kernel
+// leaves them out).  Uploaded once, at yee_prepare.
+int build_boxes (yee_handle *h)
 {
-  int rc;
-  const int dst = 1 - h->cur;
   int64_t lo[20][3], hi[20][3];
-  int nslab = slab_boxes (h, lo, hi);
-  nslab += face_boxes (h, lo + nslab, hi + nslab);
+  int n = slab_boxes (h, lo, hi);
+  n += face_boxes (h, lo + n, hi + n);
   if (h->mode == 2)
   {
     // the Drude box (its cells run the two-stage update with the ADE terms), clipped to the interior
     bool ok = true;
     for (int ax = 0; ax < 3; ++ax)
     {
-      lo[nslab][ax] = std::max<int64_t> (1, h->box_lo[ax]);
-      hi[nslab][ax] = std::min<int64_t> (h->n[ax] - 1, h->box_hi[ax]);
-      ok = ok && hi[nslab][ax] > lo[nslab][ax];
+      lo[n][ax] = std::max<int64_t> (1, h->box_lo[ax]);
+      hi[n][ax] = std::min<int64_t> (h->n[ax] - 1, h->box_hi[ax]);
+      ok = ok && hi[n][ax] > lo[n][ax];
     }
-    if (ok) ++nslab;
+    if (ok) ++n;
   }
+  auto cell = [&] (const int64_t pos[3]) {
+    for (int ax = 0; ax < 3; ++ax)
+    {
+      lo[n][ax] = pos[ax];
+      hi[n][ax] = pos[ax] + 1;
+    }
+    ++n;
+  };
   const bool src_box = source_in_fused_box (h);
-  if (src_box)
+  const int64_t *sp = h->cfg.point_source_pos, *cp = h->cfg.current_source_pos;
+  if (src_box) cell (sp);
+  const bool cur_on_src = src_box && cp[0] == sp[0] && cp[1] == sp[1] && cp[2] == sp[2];
+  if (h->cfg.current_source && !cur_on_src && fused_owns_host (h, cp)) cell (cp);
+  for (int g = 0; g < 2; ++g)
   {
-    // the point-source cell: updated by the half-step kernels, then overwritten by the source
-    // (the fused kernel leaves it out, as it does the TF/SF faces)
-    for (int ax = 0; ax < 3; ++ax)
+    // group 0: the boxes that miss the Drude box (of a Drude run: they take the PML update);
+    // group 1: those that meet it, with the ADE code and its registers
+    std::vector<HalfBox> v;
+    int64_t rows = 0;
+    for (int s = 0; s < n; ++s)
     {
-      lo[nslab][ax] = h->cfg.point_source_pos[ax];
-      hi[nslab][ax] = h->cfg.point_source_pos[ax] + 1;
+      bool meets = h->mode == 2;
+      for (int ax = 0; ax < 3; ++ax) meets = meets && lo[s][ax] < h->box_hi[ax] && h->box_lo[ax] < hi[s][ax];
+      if (meets != (g == 1)) continue;
+      HalfBox b {};
+      int64_t ext[3];
+      for (int ax = 0; ax < 3; ++ax)
+      {
+        b.lo[ax] = (int) lo[s][ax];
+        b.hi[ax] = (int) hi[s][ax];
+        ext[ax] = hi[s][ax] - lo[s][ax];
+      }
+      // 256 threads: 64 z cells (16 or 32 for z slabs), then rows, then planes, so that few idle
+      b.lbz = ext[2] <= 16 ? 4 : (ext[2] <= 32 ? 5 : 6);
+      b.lby = 0;
+      while (b.lby < 8 - b.lbz && (1 << b.lby) < ext[1]) ++b.lby;
+      const int bz = 1 << b.lbz, by = 1 << b.lby, bx = 256 / (bz * by);
+      b.tz0 = ext[2] <= bz ? b.lo[2] : (b.lo[2] & ~(bz - 1));
+      b.ntz = (b.hi[2] - b.tz0 + bz - 1) / bz;
+      b.ntx = (int) ((ext[0] + bx - 1) / bx);
+      const int64_t nt = (int64_t) b.ntz * ((ext[1] + by - 1) / by) * b.ntx;
+      b.per_xcd = (int) ((nt + 7) / 8);
+      b.ntile = (int) nt;
+      b.first = (int) rows;
+      rows += b.per_xcd;
+      if (8 * rows > (int64_t) 1 << 30) return fail (YEE_EINVAL, "half-step box too large for one launch");
+      v.push_back (b);
     }
-    ++nslab;
+    h->nbox[g] = (int) v.size ();
+    h->box_blocks[g] = (int) (8 * rows);
+    if (v.empty ()) continue;
+    if (!h->boxes[g]) HIP_TRY (hipMalloc ((void **) &h->boxes[g], 20 * sizeof (HalfBox)));
+    HIP_TRY (hipMemcpy (h->boxes[g], v.data (), v.size () * sizeof (HalfBox), hipMemcpyHostToDevice));
   }
-  const bool cur_on_src = src_box && h->cfg.current_source_pos[0] == h->cfg.point_source_pos[0]
-                          && h->cfg.current_source_pos[1] == h->cfg.point_source_pos[1]
-                          && h->cfg.current_source_pos[2] == h->cfg.point_source_pos[2];
-  if (h->cfg.current_source && !cur_on_src && fused_owns_host (h, h->cfg.current_source_pos))
+  return YEE_OK;
+}
+
+// E (with the z-face table of the fused kernel) or H of every box, one launch a group.
+template <typename T>
+int launch_boxes (yee_handle *h, bool e_half, int prev)
+{
+  const StepArgs<T> a = make_args<T> (h, prev, e_half ? kRoleE : kRoleH);
+  const int64_t nz = e_half && h->zcorr ? (3 * h->zc_n[0] * h->zc_n[1] + 255) / 256 : 0;
+  for (int g = 0; g < 2; ++g)
   {
-    // the current-source cell: the half-step kernels subtract the current after its curl
-    // update (the fused kernel leaves it out, kAxCur)
-    for (int ax = 0; ax < 3; ++ax)
+    const int nb = h->nbox[g], blk = h->box_blocks[g];
+    const dim3 grid ((unsigned) (blk + (g == 0 ? nz : 0))), block (256);
+    if (grid.x == 0) continue;
+    const HalfBox *box = h->boxes[g];
+    double *zt = (double *) h->zcorr;
+    switch ((g == 1 ? 2 : std::min (h->mode, 1)) * 2 + (e_half ? 0 : 1))
     {
-      lo[nslab][ax] = h->cfg.current_source_pos[ax];
-      hi[nslab][ax] = h->cfg.current_source_pos[ax] + 1;
+      case 0: hipLaunchKernelGGL ((e_boxes<T, 0>), grid, block, 0, h->stream, a, box, nb, blk, zt); break;
+      case 1: hipLaunchKernelGGL ((h_boxes<T, 0>), grid, block, 0, h->stream, a, box, nb); break;
+      case 2: hipLaunchKernelGGL ((e_boxes<T, 1>), grid, block, 0, h->stream, a, box, nb, blk, zt); break;
+      case 3: hipLaunchKernelGGL ((h_boxes<T, 1>), grid, block, 0, h->stream, a, box, nb); break;
+      case 4: hipLaunchKernelGGL ((e_boxes<T, 2>), grid, block, 0, h->stream, a, box, nb, blk, zt); break;
+      default: hipLaunchKernelGGL ((h_boxes<T, 2>), grid, block, 0, h->stream, a, box, nb); break;
     }
-    ++nslab;
-  }
-  {
-    ProfScope ps (h, 1);
-    for (int s = 0; s < nslab; ++s)
-      if ((rc = launch_half<T> (h, true, prev, lo[s], hi[s]))) return rc;
-  }
-  if ((rc = launch_sources<T> (h, true, t, dst, false))) return rc;
-  if (h->zcorr)
-  {
-    StepArgs<T> a = make_args<T> (h, prev);
-    const int64_t n = 3 * h->zc_n[0] * h->zc_n[1];
-    hipLaunchKernelGGL ((tfsf_ztable<T>), dim3 ((unsigned) ((n + 255) / 256)), dim3 (256), 0, h->stream, a,
-                       (double *) h->zcorr);
     HIP_TRY (hipGetLastError ());
   }
+  return YEE_OK;
+}
+
+// One time step (t > 0) with the fused kernel: E of the PML slabs and TF/SF faces, the fused E+H
+// sweep, H of the slabs and faces; old state in buffer cur, new state in 1 - cur.
+template <typename T>
+int fused_step (yee_handle *h, int32_t t, int prev)
+{
+  int rc;
+  const int dst = 1 - h->cur;
+  const bool src_box = source_in_fused_box (h);
+  {
+    ProfScope ps (h, 1);
+    if ((rc = launch_boxes<T> (h, true, prev))) return rc;
+  }
+  if ((rc = launch_sources<T> (h, true, t, dst))) return rc;
   {
     StepArgs<T> a = make_args<T> (h, prev, kRoleFused);
     for (int ax = 0; ax < 3; ++ax)
@@ -531,12 +600,8 @@ int fused_step (yee_handle *h, int32_t t, int prev)
     }
     a.lx = h->fused_lx;
     a.nstrips = h->fused_nstrips;
-    if (src_box)
-    {
-      // excluded from the kernel's cells (axis_bits, kAxSrc)
-      a.src_mask = h->cfg.point_source & 0x3fu;
-      for (int ax = 0; ax < 3; ++ax) a.src_pos[ax] = (int) h->cfg.point_source_pos[ax];
-    }
+    // the source cell is excluded from the kernel's cells (axis_bits, kAxSrc)
+    if (!src_box) a.src_mask = 0;
     ProfScope ps (h, 3);
     const unsigned blocks = (unsigned) (h->fused_nstrips * h->fused_nchunks);
     const dim3 grid (blocks), block ((unsigned) h->fused_threads);
@@ -557,10 +622,9 @@ int fused_step (yee_handle *h, int32_t t, int prev)
   }
   {
     ProfScope ps (h, 2);
-    for (int s = 0; s < nslab; ++s)
-      if ((rc = launch_half<T> (h, false, prev, lo[s], hi[s]))) return rc;
+    if ((rc = launch_boxes<T> (h, false, prev))) return rc;
   }
-  return launch_sources<T> (h, false, t, dst, false);
+  return launch_sources<T> (h, false, t, dst);
 }
 
 // Analytic test problem, after the half step's update of every component and before its point
@@ -645,14 +709,14 @@ int step_once (yee_handle *h)
     if ((rc = launch_half<T> (h, true, prev))) return rc;
   }
   if (h->fn_any () && (rc = test_hooks<T> (h, true))) return rc;
-  if ((rc = launch_sources<T> (h, true, t, h->cur, false))) return rc;
+  if ((rc = launch_sources<T> (h, true, t, h->cur))) return rc;
   if (t > 0)
   {
     ProfScope ps (h, 2);
     if ((rc = launch_half<T> (h, false, prev))) return rc;
   }
   if (h->fn_any () && (rc = test_hooks<T> (h, false))) return rc;
-  if ((rc = launch_sources<T> (h, false, t, h->cur, false))) return rc;
+  if ((rc = launch_sources<T> (h, false, t, h->cur))) return rc;
   h->t++;
   return YEE_OK;
 }
@@ -1241,6 +1305,8 @@ void yee_destroy (yee_handle *h)
   if (h->hinc[1]) (void) hipFree (h->hinc[1]);
   for (hipEvent_t e : h->ev)
     if (e) (void) hipEventDestroy (e);
+  for (yee::HalfBox *b : h->boxes)
+    if (b) (void) hipFree (b);
   if (h->norm_part) (void) hipFree (h->norm_part);
   if (h->ntff_buf) (void) hipFree (h->ntff_buf);
   if (h->stream) (void) hipStreamDestroy (h->stream);
@@ -1350,6 +1416,11 @@ int yee_prepare (yee_handle *h)
     h->tab_len = (int) std::max (h->n[0], std::max (h->n[1], h->n[2]));
     std::vector<double> tab = pml_tables (h->cfg, h->tab_len);
     int rc = upload (h, &h->pml, tab.data (), tab.size ());
+    if (rc) return rc;
+  }
+  if (h->fused)
+  {
+    int rc = build_boxes (h);
     if (rc) return rc;
   }
   if (h->fn_start)

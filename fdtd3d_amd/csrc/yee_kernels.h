@@ -79,6 +79,7 @@ struct StepArgs
   uint32_t src_mask;           // bit c: hard source on component c at flat index src_q
   int64_t src_q;
   int src_pos[3];              // the same position as (x, y, z)
+  double src_val;              // its value of this half step (half-step kernels: stored in place of the update)
   uint32_t cur_mask;           // bit c: current source J (E) / M (H) on component c at cur_pos
   int cur_pos[3];
   double cur_val;              // the current of this half step: sin (dt ts 2 pi f) mu0 / dt / 2
@@ -99,6 +100,16 @@ struct StepArgs
   double exp_k, exp_d, exp_w, exp_t0, exp_m;
   // Yee layout: 0 E_CENTERED, 1 H_CENTERED (component positions of the test problems)
   int layout;
+};
+
+// One box of a half-step launch over several boxes (e_boxes / h_boxes): the cells [lo, hi), tiles
+// of 2^lbz z cells x 2^lby rows x 256 / that planes from (lo[0], lo[1], tz0), their counts, the
+// tiles per XCD band and the first tile row (blockIdx / 8) of the box in the launch.
+struct HalfBox
+{
+  int lo[3], hi[3];
+  int lbz, lby;
+  int tz0, ntz, ntx, ntile, per_xcd, first;
 };
 
 // Near-to-far-field transform (yee_ntff): the complex fields' two parts, the snapshot of H before

@@ -161,7 +161,12 @@ template <typename T, int MODE, int COMP>
 __device__ __forceinline__ void update_cell (const StepArgs<T> &a, int64_t q, const int p[3], T f_old,
                                              const Old<T> &old, T tmp, T mat, bool special, T om, T ga)
 {
-  gst (a.f_n[COMP] + q, cell_value<T, MODE, COMP> (a, q, p, f_old, old, tmp, mat, special, om, ga, true));
+  T v = cell_value<T, MODE, COMP> (a, q, p, f_old, old, tmp, mat, special, om, ga, true);
+  // hard point source (performPointSourceCalc, InternalScheme.inc.h:2818-2895): it replaces the
+  // updated value, so storing it here saves a launch per component and half step
+  if (((a.src_mask >> COMP) & 1u) && p[0] == a.src_pos[0] && p[1] == a.src_pos[1] && p[2] == a.src_pos[2])
+    v = (T) a.src_val;
+  gst (a.f_n[COMP] + q, v);
 }
 
 // Previous value and (special cells) the D/B history of component COMP at q.
@@ -407,6 +412,42 @@ __global__ __launch_bounds__ (256) void h_half_3d_hc (StepArgs<T> a)
   h_half_cell<T, MODE, 1> (a, i, j, k);
 }
 
+// One z-face correction entry (tfsf_ztable_entry below) and the half steps of several boxes in
+// one launch: the PML slabs, the TF/SF x / y faces, the source cells of a fused step.  The boxes
+// do not read one another's results (E reads H before the step, H reads E after it; cells in two
+// boxes have no D / B and get the same value twice), so their order is free.  What bounds these
+// boxes on small and ordinary grids is latency: a launch of a slab takes 6 us however few cells
+// it has, and a step had 24 of them (80^3 FP64 with PML and TF/SF: 194 us a step, 94 us with one
+// launch a half step; 512^3 FP32: 2.61 -> 2.53 ms, where the slabs are bound by HBM instead).
+template <typename T>
+__device__ __forceinline__ void tfsf_ztable_entry (const StepArgs<T> &a, double *out, int64_t u);
+
+template <typename T, int MODE>
+__global__ __launch_bounds__ (256) void e_boxes (StepArgs<T> a, const HalfBox *box, int nbox, int nblk, double *zt)
+{
+  if ((int) blockIdx.x >= nblk)
+  {
+    // the blocks after the boxes' fill the z-face table of the fused kernel
+    tfsf_ztable_entry (a, zt, (int64_t) ((int) blockIdx.x - nblk) * 256 + (int) threadIdx.x);
+    return;
+  }
+  int i, j, k;
+  if (!half_cell_boxes (box, nbox, i, j, k)) return;
+  const int p[3] = { i, j, k };
+  if (MODE == 2 && !in_drude_box (a, p, 3)) e_half_cell<T, 1> (a, i, j, k);
+  else e_half_cell<T, MODE> (a, i, j, k);
+}
+
+template <typename T, int MODE>
+__global__ __launch_bounds__ (256) void h_boxes (StepArgs<T> a, const HalfBox *box, int nbox)
+{
+  int i, j, k;
+  if (!half_cell_boxes (box, nbox, i, j, k)) return;
+  const int p[3] = { i, j, k };
+  if (MODE == 2 && !in_drude_box (a, p, 3)) h_half_cell<T, 1> (a, i, j, k);
+  else h_half_cell<T, MODE> (a, i, j, k);
+}
+
 // ---------------------------------------------------------------------------------------
 // Fused 3D time step: E of step t, then H of step t, in one sweep of the cells it owns.
 //
@@ -522,9 +563,8 @@ __device__ __forceinline__ void zface_apply (const double *c, T &v_lo, T &v_hi)
 // update (Ex pair BACK/FRONT, Ey pair BACK/FRONT), part 1 for the H update (Hx, Hy likewise).
 // The same predicates and incident interpolation as calculateTFSF (tfsf_pair_diff).
 template <typename T>
-__global__ void tfsf_ztable (StepArgs<T> a, double *out)
+__device__ __forceinline__ void tfsf_ztable_entry (const StepArgs<T> &a, double *out, int64_t u)
 {
-  const int64_t u = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t per = (int64_t) a.zc_n[0] * a.zc_n[1];
   if (u >= 3 * per) return;
   const int f = (int) (u / per);
@@ -2082,7 +2122,12 @@ __global__ void tfsf_mask_kernel (StepArgs<T> a, int comp, int dim, uint8_t *out
   template __global__ void step_3d_fused<T, FUSED_BY (T), 1, 12> (StepArgs<T>);            \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 2, 12> (StepArgs<T>);            \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 3, 12> (StepArgs<T>);            \
-  template __global__ void tfsf_ztable<T> (StepArgs<T>, double *);                         \
+  template __global__ void e_boxes<T, 0> (StepArgs<T>, const HalfBox *, int, int, double *); \
+  template __global__ void e_boxes<T, 1> (StepArgs<T>, const HalfBox *, int, int, double *); \
+  template __global__ void e_boxes<T, 2> (StepArgs<T>, const HalfBox *, int, int, double *); \
+  template __global__ void h_boxes<T, 0> (StepArgs<T>, const HalfBox *, int);              \
+  template __global__ void h_boxes<T, 1> (StepArgs<T>, const HalfBox *, int);              \
+  template __global__ void h_boxes<T, 2> (StepArgs<T>, const HalfBox *, int);              \
   template __global__ void point_source<T> (T *, int64_t, double);                         \
   template __global__ void tfsf_mask_kernel<T> (StepArgs<T>, int, int, uint8_t *); \
   template __global__ void test_fill<T> (StepArgs<T>, T *, int, int, double, int); \

@@ -1,0 +1,45 @@
+"""How the work of a time step is cut into launches must not show in its results (needs the GPU).
+
+One launch updates every box around the fused kernel (PML slabs, TF/SF faces, source cells): the
+fields are bit-identical to the half-step kernels over the whole grid (YEE_KERNEL=split), with the
+hard source on a face plane, an edge of two faces, in a slab, inside the fused box and on the grid
+border (never updated: the source alone writes it), and with boxes of one cell along an axis.
+"""
+import numpy as np
+import pytest
+
+from fdtd3d_amd.config import parse_args
+from fdtd3d_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(args, precision, monkeypatch, kernel, eps, steps):
+    monkeypatch.setenv("YEE_KERNEL", kernel)
+    cfg = parse_args(args.split(), precision=precision)
+    eng = Engine(cfg)
+    eng.set_material("eps", eps)
+    eng.prepare()
+    eng.step(steps)
+    names = list(cfg.components) + (["D" + c[1] if c[0] == "E" else "B" + c[1] for c in cfg.components] if cfg.use_pml else [])
+    out = {n: eng.field_raw(n) for n in names}
+    eng.close()
+    return out
+
+
+BOXES = "--3d --size x:19,y:21,z:70 --use-pml --pml-size x:3,y:1,z:4 --use-tfsf --tfsf-size-left x:6,y:5,z:7 " \
+        "--tfsf-size-right x:6,y:5,z:7 --angle-teta 30 --angle-phi 45 --angle-psi 90 --point-source-ez --point-source-hx "
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("pos", ["x:5,y:9,z:30", "x:5,y:4,z:30", "x:9,y:9,z:66", "x:9,y:10,z:31", "x:0,y:9,z:30",
+                                 "x:9,y:20,z:69"])
+def test_boxes_in_one_launch(pos, precision, engine_lib, monkeypatch):
+    args = BOXES + f"--point-source {pos} --time-steps 20"
+    print(f"[gpu] boxes, source {pos}, precision {precision}", flush=True)
+    eps = np.random.default_rng(3).uniform(1.0, 4.0, size=(19, 21, 70))
+    ref = _run(args, precision, monkeypatch, "split", eps, 20)
+    got = _run(args, precision, monkeypatch, "fused", eps, 20)
+    for n, v in ref.items():
+        assert np.array_equal(got[n], v), n
+    assert np.abs(ref["Ez"]).max() > 0
