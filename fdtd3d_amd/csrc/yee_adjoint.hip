@@ -296,7 +296,7 @@ template <typename T>
 AdjArgs<T> adj_args (const yee_handle *h)
 {
   AdjArgs<T> g {};
-  g.a = engine_args<T> (h, 0);
+  g.a = engine_args<T> (h);
   for (int c = 0; c < 6; ++c)
   {
     g.af[c] = (T *) h->adj->af[c];
@@ -365,9 +365,9 @@ int snapshot (yee_handle *h, int k, bool restore)
     if ((rc = move (h->f[h->cur][c], grid))) return rc;
     if ((rc = move (h->d[h->cur][c], grid))) return rc;
   }
-  if ((rc = move (h->einc, inc))) return rc;
-  if ((rc = move (h->hinc[0], inc))) return rc;
-  if ((rc = move (h->hinc[1], inc))) return rc;
+  if (restore) h->inc_t = h->hist_t = h->t;   // the next step restarts the incident rows
+  if ((rc = move (h->einc[h->inc_cur], inc))) return rc;
+  if ((rc = move (h->hinc[h->inc_cur], inc))) return rc;
   return YEE_OK;
 }
 
@@ -443,7 +443,8 @@ int forward_impl (yee_handle *h, const double *design, double *J)
   HIP_TRY (hipEventRecord (h->ev[0], h->stream));
   for (int32_t t = 0; t < s->T; ++t)
   {
-    if ((rc = engine_step_once (h))) return rc;
+    // up to the next snapshot
+    if ((rc = engine_step_once (h, std::min (K == 0 ? s->T : (t + K - 1) / K * K + 1, s->T) - t))) return rc;
     if (K == 0)
     {
       if ((rc = record<T> (h, t))) return rc;
@@ -514,7 +515,7 @@ int backward_impl (yee_handle *h, double dJ, double *grad)
         if ((rc = record<T> (h, 0))) return rc;   // state after step kK
         for (int32_t t = t0 + 1; t <= t1; ++t)
         {
-          if ((rc = engine_step_once (h))) return rc;
+          if ((rc = engine_step_once (h, t1 + 1 - t))) return rc;
           if ((rc = record<T> (h, t - t0))) return rc;
         }
       }
@@ -634,7 +635,7 @@ int yee_adjoint_setup (yee_handle *h, const yee_adjoint_spec *sp)
       if (h->f[0][c]) bytes += grid;
       if (h->d[0][c]) bytes += grid;
     }
-    bytes += 3 * (size_t) h->inc_len * h->wsize;
+    bytes += 2 * (size_t) h->inc_len * h->wsize;
     s->snap_bytes = bytes;
     s->snap.assign (nsnap, nullptr);
     s->snap_t.assign (nsnap, 0);

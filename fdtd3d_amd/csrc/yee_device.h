@@ -289,7 +289,7 @@ __device__ double incident_at (const StepArgs<T> &a, int i, int j, int k, const 
   long long i1 = (long long) c1;
   // the reference asserts d > 0; clamp so a degenerate box can never read out of bounds
   if (i1 < 0) i1 = 0;
-  if (i1 > tg.inc_len - 2) i1 = tg.inc_len - 2;
+  if (i1 > a.inc_len - 2) i1 = a.inc_len - 2;
   const double p2 = d - c1;
   const double p1 = 1 - p2;
   const double v = (double) gld (inc + i1) * p1 + (double) gld (inc + i1 + 1) * p2;
@@ -309,7 +309,7 @@ __device__ __forceinline__ bool tfsf_pair_diff (const StepArgs<T> &a, int i, int
   const bool lo = tfsf_pred<T, COMP, Tab::dir[COMP][2 * PAIR], DIM> (a, i, j, k);
   const bool hi = tfsf_pred<T, COMP, Tab::dir[COMP][2 * PAIR + 1], DIM> (a, i, j, k);
   if (!lo && !hi) return false;
-  const T *inc = h ? a.tg->einc : a.tg->hinc[a.hinc_sel];
+  const T *inc = h ? a.einc : a.hinc;
   const double ddiff = h ? 0.0 : 0.5;
   const bool use_hi_slot = h ? !lo : lo;
   constexpr int s_lo = 2 * PAIR, s_hi = 2 * PAIR + 1;
@@ -339,7 +339,7 @@ __device__ __forceinline__ void tfsf_pair (const StepArgs<T> &a, int i, int j, i
   const bool lo = tfsf_pred<T, COMP, Tab::dir[COMP][2 * PAIR], DIM, LAY> (a, i, j, k);
   const bool hi = tfsf_pred<T, COMP, Tab::dir[COMP][2 * PAIR + 1], DIM, LAY> (a, i, j, k);
   if (!lo && !hi) return;
-  const T *inc = h ? a.tg->einc : a.tg->hinc[a.hinc_sel];
+  const T *inc = h ? a.einc : a.hinc;
   const double ddiff = h ? 0.0 : 0.5;
   // slot 2*PAIR is "lo" (d11 / d21), slot 2*PAIR+1 is "hi" (d12 / d22)
   const bool use_hi_slot = rh ? !lo : lo;

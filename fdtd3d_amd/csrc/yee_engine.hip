@@ -2,7 +2,7 @@
 //
 // One handle = one simulation on one GPU: device state, the HIP stream its work is
 // queued on, and the FP64 set-up tables.  yee_step enqueues per time step:
-//   incident_step (TF/SF only)  ->  E half-step  ->  E point sources  ->  H half-step  ->  H point sources
+//   incident_steps (TF/SF only, once per up to 32 steps)  ->  E half-step  ->  H half-step (each with its point sources)
 // which is the ordering of Scheme::performNStepsForBlock (Source/Scheme/Scheme.inc.h:28-473).
 #include <hip/hip_runtime.h>
 
@@ -31,10 +31,11 @@ template <typename T, int MODE> __global__ void e_half_tmz (StepArgs<T>);
 template <typename T, int MODE> __global__ void h_half_tmz (StepArgs<T>);
 template <typename T, int MODE> __global__ void e_half_tez (StepArgs<T>);
 template <typename T, int MODE> __global__ void h_half_tez (StepArgs<T>);
-template <typename T> __global__ void incident_step (T *, const T *, T *, int64_t, int, double, double, double);
+template <typename T>
+__global__ void incident_steps (const T *, const T *, T *, T *, int64_t, int, double, double, IncidentSource, T *, T *, int64_t);
 template <typename T> __global__ void point_source (T *, int64_t, double);
 template <typename T> __global__ void tfsf_mask_kernel (StepArgs<T>, int, int, uint8_t *);
-template <typename T, int COMP, int DIM> __global__ void scattered_kernel (StepArgs<T>, const T *, double *, int, int64_t, int64_t);
+template <typename T, int COMP, int DIM> __global__ void scattered_kernel (StepArgs<T>, const T *, double *, int64_t, int64_t);
 template <typename T, int BY, int MAT, int MAXW> __global__ void step_3d_fused (StepArgs<T>);
 template <typename T, int MODE> __global__ void e_boxes (StepArgs<T>, const HalfBox *, int, int, double *);
 template <typename T, int MODE> __global__ void h_boxes (StepArgs<T>, const HalfBox *, int);
@@ -121,7 +122,7 @@ bool source_in_update (const yee_handle *h)
 }
 
 template <typename T>
-StepArgs<T> make_args (const yee_handle *h, int parity, ArgRole role = kRoleE)
+StepArgs<T> make_args (const yee_handle *h, ArgRole role = kRoleE)
 {
   StepArgs<T> a {};
   a.nx = (int) h->n[0];
@@ -224,8 +225,14 @@ StepArgs<T> make_args (const yee_handle *h, int parity, ArgRole role = kRoleE)
   a.zcorr = (const double *) h->zcorr;
   a.zc_n[0] = (int) h->zc_n[0];
   a.zc_n[1] = (int) h->zc_n[1];
-  // the E half-step of step t reads HInc after step t-1, kept in buffer (t+1) & 1
-  a.hinc_sel = parity;
+  if (h->use_tfsf ())
+  {
+    // the rows of step t (incident_ahead has made them)
+    const int64_t row = (int64_t) (h->t - h->hist_t) * h->hist_len;
+    a.einc = (const T *) h->hist_e + row;
+    a.hinc = (const T *) h->hist_h + row;
+    a.inc_len = h->hist_len;
+  }
   // analytic test problem: the right side of this half step, at time step t (E) or t + 1/2 (H)
   // (Scheme.inc.h:1062-1098)
   a.rhs_kind = h->fn_rhs;
@@ -244,9 +251,9 @@ StepArgs<T> make_args (const yee_handle *h, int parity, ArgRole role = kRoleE)
 
 
 template <typename T>
-int launch_half (yee_handle *h, bool e_half, int parity)
+int launch_half (yee_handle *h, bool e_half)
 {
-  StepArgs<T> a = make_args<T> (h, parity, e_half ? kRoleE : kRoleH);
+  StepArgs<T> a = make_args<T> (h, e_half ? kRoleE : kRoleH);
   if (h->dim == 3)
   {
     const int64_t ext[3] = { a.run_hi[0] - a.run_lo[0], a.run_hi[1] - a.run_lo[1], a.run_hi[2] - a.run_lo[2] };
@@ -553,9 +560,9 @@ int build_boxes (yee_handle *h)
 
 // E (with the z-face table of the fused kernel) or H of every box, one launch a group.
 template <typename T>
-int launch_boxes (yee_handle *h, bool e_half, int prev)
+int launch_boxes (yee_handle *h, bool e_half)
 {
-  const StepArgs<T> a = make_args<T> (h, prev, e_half ? kRoleE : kRoleH);
+  const StepArgs<T> a = make_args<T> (h, e_half ? kRoleE : kRoleH);
   const int64_t nz = e_half && h->zcorr ? (3 * h->zc_n[0] * h->zc_n[1] + 255) / 256 : 0;
   for (int g = 0; g < 2; ++g)
   {
@@ -581,18 +588,18 @@ int launch_boxes (yee_handle *h, bool e_half, int prev)
 // One time step (t > 0) with the fused kernel: E of the PML slabs and TF/SF faces, the fused E+H
 // sweep, H of the slabs and faces; old state in buffer cur, new state in 1 - cur.
 template <typename T>
-int fused_step (yee_handle *h, int32_t t, int prev)
+int fused_step (yee_handle *h, int32_t t)
 {
   int rc;
   const int dst = 1 - h->cur;
   const bool src_box = source_in_fused_box (h);
   {
     ProfScope ps (h, 1);
-    if ((rc = launch_boxes<T> (h, true, prev))) return rc;
+    if ((rc = launch_boxes<T> (h, true))) return rc;
   }
   if ((rc = launch_sources<T> (h, true, t, dst))) return rc;
   {
-    StepArgs<T> a = make_args<T> (h, prev, kRoleFused);
+    StepArgs<T> a = make_args<T> (h, kRoleFused);
     for (int ax = 0; ax < 3; ++ax)
     {
       a.run_lo[ax] = (int) h->fbox_lo[ax];
@@ -622,7 +629,7 @@ int fused_step (yee_handle *h, int32_t t, int prev)
   }
   {
     ProfScope ps (h, 2);
-    if ((rc = launch_boxes<T> (h, false, prev))) return rc;
+    if ((rc = launch_boxes<T> (h, false))) return rc;
   }
   return launch_sources<T> (h, false, t, dst);
 }
@@ -637,7 +644,7 @@ template <typename T>
 int test_hooks (yee_handle *h, bool e_half)
 {
   const double time = (e_half ? (double) h->t + 0.5 : (double) h->t + 1.0) * h->sc.dt;
-  StepArgs<T> a = make_args<T> (h, 0);
+  StepArgs<T> a = make_args<T> (h);
   const int64_t blocks = std::max<int64_t> (1, std::min<int64_t> ((h->ncell + 255) / 256, 65536));
   for (int c = e_half ? 0 : 3; c < (e_half ? 3 : 6); ++c)
   {
@@ -665,7 +672,7 @@ int test_hooks (yee_handle *h, bool e_half)
 template <typename T>
 int test_start (yee_handle *h)
 {
-  StepArgs<T> a = make_args<T> (h, 0);
+  StepArgs<T> a = make_args<T> (h);
   const int64_t blocks = std::max<int64_t> (1, std::min<int64_t> ((h->ncell + 255) / 256, 65536));
   for (int c = 0; c < 6; ++c)
   {
@@ -678,27 +685,45 @@ int test_start (yee_handle *h)
   return YEE_OK;
 }
 
+// Makes the incident rows of step h->t unless an earlier launch has: one launch advances the
+// incident grid by up to kIncSteps of the `ahead` steps the caller takes in a row, so that its
+// state is that of the last step when the call returns.
 template <typename T>
-int step_once (yee_handle *h)
+int incident_ahead (yee_handle *h, int32_t ahead)
+{
+  if (!h->use_tfsf () || h->t < h->inc_t) return YEE_OK;
+  const int n = (int) std::min<int32_t> (std::max<int32_t> (ahead, 1), kIncSteps);
+  const double modE = h->sc.dt / (h->sc.rel * eps0 () * h->cfg.dx);
+  const double modH = h->sc.dt / (h->sc.rel * mu0 () * h->cfg.dx);
+  IncidentSource src {};
+  for (int s = 0; s < n; ++s)
+  {
+    const double arg = h->sc.dt * (h->t + s) * 2 * kPi * h->sc.freq;
+    src.v[s] = h->src_kind == 2 ? std::cos (arg) : std::sin (arg);   // complex build: (sin, cos)
+  }
+  // cells the wave can have reached, and the rows' length
+  const int64_t cells = std::max (std::min (h->inc_len, (int64_t) h->t + n + 2), h->hist_len);
+  const int b = h->inc_cur;
+  ProfScope ps (h, 0);
+  hipLaunchKernelGGL ((incident_steps<T>), dim3 ((unsigned) ((cells + kIncTile - 1) / kIncTile)), dim3 (256), 0, h->stream,
+                     (const T *) h->einc[b], (const T *) h->hinc[b], (T *) h->einc[1 - b], (T *) h->hinc[1 - b],
+                     h->inc_len, n, modE, modH, src, (T *) h->hist_e, (T *) h->hist_h, h->hist_len);
+  HIP_TRY (hipGetLastError ());
+  h->inc_cur = 1 - b;
+  h->hist_t = h->t;
+  h->inc_t = h->t + n;
+  return YEE_OK;
+}
+
+template <typename T>
+int step_once (yee_handle *h, int32_t ahead)
 {
   const int32_t t = h->t;
-  const int prev = (t + 1) & 1;   // HInc after step t-1
-  const int cur = t & 1;          // HInc after step t
-  if (h->use_tfsf ())
-  {
-    const double modE = h->sc.dt / (h->sc.rel * eps0 () * h->cfg.dx);
-    const double modH = h->sc.dt / (h->sc.rel * mu0 () * h->cfg.dx);
-    const double arg = h->sc.dt * t * 2 * kPi * h->sc.freq;
-    ProfScope ps (h, 0);
-    hipLaunchKernelGGL ((incident_step<T>), dim3 (1), dim3 (1024), 0, h->stream, (T *) h->einc,
-                       (const T *) h->hinc[prev], (T *) h->hinc[cur], h->inc_len, (int) t, modE, modH,
-                       h->src_kind == 2 ? std::cos (arg) : std::sin (arg));   // complex build: (sin, cos)
-    HIP_TRY (hipGetLastError ());
-  }
-  int rc;
+  int rc = incident_ahead<T> (h, ahead);
+  if (rc) return rc;
   if (h->fused && t > 0)
   {
-    if ((rc = fused_step<T> (h, t, prev))) return rc;
+    if ((rc = fused_step<T> (h, t))) return rc;
     h->cur = 1 - h->cur;
     h->t++;
     return YEE_OK;
@@ -706,14 +731,14 @@ int step_once (yee_handle *h)
   if (t > 0)
   {
     ProfScope ps (h, 1);
-    if ((rc = launch_half<T> (h, true, prev))) return rc;
+    if ((rc = launch_half<T> (h, true))) return rc;
   }
   if (h->fn_any () && (rc = test_hooks<T> (h, true))) return rc;
   if ((rc = launch_sources<T> (h, true, t, h->cur))) return rc;
   if (t > 0)
   {
     ProfScope ps (h, 2);
-    if ((rc = launch_half<T> (h, false, prev))) return rc;
+    if ((rc = launch_half<T> (h, false))) return rc;
   }
   if (h->fn_any () && (rc = test_hooks<T> (h, false))) return rc;
   if ((rc = launch_sources<T> (h, false, t, h->cur))) return rc;
@@ -942,10 +967,6 @@ int upload_tfsf_geom (yee_handle *h)
   g.S2 = h->sc.S2;
   g.C2 = h->sc.C2;
   for (int c = 0; c < 6; ++c) g.proj[c] = h->sc.proj[c];
-  g.einc = (const T *) h->einc;
-  g.hinc[0] = (const T *) h->hinc[0];
-  g.hinc[1] = (const T *) h->hinc[1];
-  g.inc_len = h->inc_len;
   if (!h->tg) HIP_TRY (hipMalloc (&h->tg, sizeof g));
   HIP_TRY (hipMemcpy (h->tg, &g, sizeof g, hipMemcpyHostToDevice));
   return YEE_OK;
@@ -1059,9 +1080,9 @@ int set_exact_exp_part (yee_handle *h, int32_t kind, int32_t pair, double border
 
 namespace yee {
 
-int engine_step_once (yee_handle *h)
+int engine_step_once (yee_handle *h, int32_t ahead)
 {
-  return h->fp32 () ? step_once<float> (h) : step_once<double> (h);
+  return h->fp32 () ? step_once<float> (h, ahead) : step_once<double> (h, ahead);
 }
 
 int engine_alloc_grid (yee_handle *h, void **view)
@@ -1070,12 +1091,12 @@ int engine_alloc_grid (yee_handle *h, void **view)
 }
 
 template <typename T>
-StepArgs<T> engine_args (const yee_handle *h, int parity)
+StepArgs<T> engine_args (const yee_handle *h)
 {
-  return make_args<T> (h, parity);
+  return make_args<T> (h);
 }
-template StepArgs<float> engine_args<float> (const yee_handle *, int);
-template StepArgs<double> engine_args<double> (const yee_handle *, int);
+template StepArgs<float> engine_args<float> (const yee_handle *);
+template StepArgs<double> engine_args<double> (const yee_handle *);
 
 int engine_reset (yee_handle *h)
 {
@@ -1087,9 +1108,9 @@ int engine_reset (yee_handle *h)
       for (void *p : ptrs)
         if (p) HIP_TRY (hipMemsetAsync ((char *) p - kPadFront * h->wsize, 0, bytes, h->stream));
     }
-  if (h->einc) HIP_TRY (hipMemsetAsync (h->einc, 0, (size_t) h->inc_len * h->wsize, h->stream));
-  for (void *p : h->hinc)
+  for (void *p : { h->einc[0], h->einc[1], h->hinc[0], h->hinc[1] })
     if (p) HIP_TRY (hipMemsetAsync (p, 0, (size_t) h->inc_len * h->wsize, h->stream));
+  h->inc_t = h->hist_t = 0;
   h->t = 0;
   h->cur = 0;
   return YEE_OK;
@@ -1267,12 +1288,38 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   {
     // allocateGridsInc: 500 * size.x cells (InternalScheme.specific.h:99-107)
     h->inc_len = 500 * h->n[first_active_axis (*cfg)];   // size.get1 () of the scheme's grid
-    if ((rc = alloc_zero (h, &h->einc, h->inc_len * h->wsize))) return bail (rc);
-    if ((rc = alloc_zero (h, &h->hinc[0], h->inc_len * h->wsize))) return bail (rc);
-    if ((rc = alloc_zero (h, &h->hinc[1], h->inc_len * h->wsize))) return bail (rc);
   }
   if (hipStreamSynchronize (h->stream) != hipSuccess) return bail (fail (YEE_EDEVICE, "stream sync failed"));
   h->sc = compute_scalars (h->cfg);
+  if (h->use_tfsf ())
+  {
+    // the furthest incident cell the TF/SF correction reads (incident_at): the distance along the
+    // wave is linear in the coordinates, so it is largest at a corner of the corrected points,
+    // which lie within [L - 2, R + 3] on every axis
+    const double dir[3] = { h->dim == 3 ? h->sc.S1 * h->sc.C2 : h->sc.C2, h->dim == 3 ? h->sc.S1 * h->sc.S2 : h->sc.S2,
+                            h->dim == 3 ? h->sc.C1 : 0.0 };
+    double far = 0;
+    for (int ax = 0; ax < 3; ++ax)
+    {
+      if (!axis_active (h->cfg, ax)) continue;
+      const double lo = (double) cfg->tfsf_left[ax] - 2 - h->sc.zero_inc[ax];
+      const double hi = (double) (h->n[ax] - cfg->tfsf_right[ax]) + 3 - h->sc.zero_inc[ax];
+      far += std::max (dir[ax] * lo, dir[ax] * hi);
+    }
+    h->hist_len = std::min (h->inc_len, (int64_t) std::max (far, 0.0) + 8);
+    // one allocation: EInc and HInc (two buffers each), then the two histories
+    const size_t inc = (size_t) h->inc_len * h->wsize, hist = (size_t) (kIncSteps * h->hist_len) * h->wsize;
+    if ((rc = alloc_zero (h, &h->inc_mem, 4 * inc + 2 * hist))) return bail (rc);
+    char *m = (char *) h->inc_mem;
+    for (int b = 0; b < 2; ++b)
+    {
+      h->einc[b] = m + 2 * b * inc;
+      h->hinc[b] = m + (2 * b + 1) * inc;
+    }
+    h->hist_e = m + 4 * inc;
+    h->hist_h = m + 4 * inc + hist;
+    if (hipStreamSynchronize (h->stream) != hipSuccess) return bail (fail (YEE_EDEVICE, "stream sync failed"));
+  }
   if (h->complex ())
   {
     // complex field values: this handle is the real part; the imaginary part is a second real
@@ -1300,9 +1347,7 @@ void yee_destroy (yee_handle *h)
   if (h->tg) (void) hipFree (h->tg);
   if (h->zcorr) (void) hipFree (h->zcorr);
   if (h->pml) (void) hipFree (h->pml);
-  if (h->einc) (void) hipFree (h->einc);
-  if (h->hinc[0]) (void) hipFree (h->hinc[0]);
-  if (h->hinc[1]) (void) hipFree (h->hinc[1]);
+  if (h->inc_mem) (void) hipFree (h->inc_mem);
   for (hipEvent_t e : h->ev)
     if (e) (void) hipEventDestroy (e);
   for (yee::HalfBox *b : h->boxes)
@@ -1442,10 +1487,10 @@ int yee_step (yee_handle *h, int32_t n)
   if (h->imag) HIP_TRY (hipStreamWaitEvent (h->imag->stream, h->ev[0], 0));
   for (int32_t s = 0; s < n; ++s)
   {
-    int rc = h->fp32 () ? step_once<float> (h) : step_once<double> (h);
+    int rc = engine_step_once (h, n - s);
     if (rc) return rc;
     // complex fields: the imaginary part on its own stream, alongside
-    if (h->imag && (rc = h->fp32 () ? step_once<float> (h->imag) : step_once<double> (h->imag))) return rc;
+    if (h->imag && (rc = engine_step_once (h->imag, n - s))) return rc;
   }
   if (h->imag)
   {
@@ -1760,12 +1805,12 @@ int yee_get_diff_norm_complex (yee_handle *h, int32_t comp, double out[9])
   const double time = (comp >= 3 ? (double) t + 1.0 : (double) t + 0.5) * h->sc.dt;
   double *mpart = h->norm_part + (size_t) (6 + comp) * 2 * kNormBlocks;
   if (h->fp32 ())
-    hipLaunchKernelGGL ((test_norm<float>), dim3 (kNormBlocks), dim3 (256), 0, h->stream, make_args<float> (h, 0),
+    hipLaunchKernelGGL ((test_norm<float>), dim3 (kNormBlocks), dim3 (256), 0, h->stream, make_args<float> (h),
                        (const float *) h->f[h->cur][comp], (const float *) h->imag->f[h->imag->cur][comp], comp,
                        h->fn_exact, time, (int) h->norm_lo[0], (int) h->norm_lo[1], (int) h->norm_lo[2],
                        (int) h->norm_hi[0], (int) h->norm_hi[1], (int) h->norm_hi[2], mpart);
   else
-    hipLaunchKernelGGL ((test_norm<double>), dim3 (kNormBlocks), dim3 (256), 0, h->stream, make_args<double> (h, 0),
+    hipLaunchKernelGGL ((test_norm<double>), dim3 (kNormBlocks), dim3 (256), 0, h->stream, make_args<double> (h),
                        (const double *) h->f[h->cur][comp], (const double *) h->imag->f[h->imag->cur][comp], comp,
                        h->fn_exact, time, (int) h->norm_lo[0], (int) h->norm_lo[1], (int) h->norm_lo[2],
                        (int) h->norm_hi[0], (int) h->norm_hi[1], (int) h->norm_hi[2], mpart);
@@ -1827,29 +1872,31 @@ namespace {
 template <typename T>
 int scattered (yee_handle *h, int comp, double *dev, int64_t q0, int64_t count)
 {
-  const StepArgs<T> a = make_args<T> (h, 0);
+  StepArgs<T> a = make_args<T> (h);
+  a.einc = (const T *) h->einc[h->inc_cur];
+  a.hinc = (const T *) h->hinc[h->inc_cur];
+  a.inc_len = h->inc_len;
   const T *f = (const T *) h->f[h->cur][comp];
-  const int hsel = (h->t + 1) & 1;   // buffer of the newest HInc (yee_get_incident)
   const dim3 grid ((unsigned) ((count + 255) / 256)), block (256);
   if (h->dim == 3)
     switch (comp)
     {
-      case 0: hipLaunchKernelGGL ((scattered_kernel<T, 0, 3>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 1: hipLaunchKernelGGL ((scattered_kernel<T, 1, 3>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 2: hipLaunchKernelGGL ((scattered_kernel<T, 2, 3>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 3: hipLaunchKernelGGL ((scattered_kernel<T, 3, 3>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 4: hipLaunchKernelGGL ((scattered_kernel<T, 4, 3>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      default: hipLaunchKernelGGL ((scattered_kernel<T, 5, 3>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
+      case 0: hipLaunchKernelGGL ((scattered_kernel<T, 0, 3>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 1: hipLaunchKernelGGL ((scattered_kernel<T, 1, 3>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 2: hipLaunchKernelGGL ((scattered_kernel<T, 2, 3>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 3: hipLaunchKernelGGL ((scattered_kernel<T, 3, 3>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 4: hipLaunchKernelGGL ((scattered_kernel<T, 4, 3>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      default: hipLaunchKernelGGL ((scattered_kernel<T, 5, 3>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
     }
   else
     switch (comp)
     {
-      case 0: hipLaunchKernelGGL ((scattered_kernel<T, 0, 2>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 1: hipLaunchKernelGGL ((scattered_kernel<T, 1, 2>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 2: hipLaunchKernelGGL ((scattered_kernel<T, 2, 2>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 3: hipLaunchKernelGGL ((scattered_kernel<T, 3, 2>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      case 4: hipLaunchKernelGGL ((scattered_kernel<T, 4, 2>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
-      default: hipLaunchKernelGGL ((scattered_kernel<T, 5, 2>), grid, block, 0, h->stream, a, f, dev, hsel, q0, count); break;
+      case 0: hipLaunchKernelGGL ((scattered_kernel<T, 0, 2>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 1: hipLaunchKernelGGL ((scattered_kernel<T, 1, 2>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 2: hipLaunchKernelGGL ((scattered_kernel<T, 2, 2>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 3: hipLaunchKernelGGL ((scattered_kernel<T, 3, 2>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      case 4: hipLaunchKernelGGL ((scattered_kernel<T, 4, 2>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
+      default: hipLaunchKernelGGL ((scattered_kernel<T, 5, 2>), grid, block, 0, h->stream, a, f, dev, q0, count); break;
     }
   HIP_TRY (hipGetLastError ());
   return YEE_OK;
@@ -1949,9 +1996,9 @@ int yee_get_mask (yee_handle *h, int32_t kind, int32_t comp, uint8_t *out)
     HIP_TRY (hipMalloc (&dev, (size_t) h->ncell));
     const int grid = (int) std::min<int64_t> (4096, (h->ncell + 255) / 256);
     if (h->fp32 ())
-      hipLaunchKernelGGL ((tfsf_mask_kernel<float>), dim3 (grid), dim3 (256), 0, h->stream, make_args<float> (h, 0), comp, h->dim, dev);
+      hipLaunchKernelGGL ((tfsf_mask_kernel<float>), dim3 (grid), dim3 (256), 0, h->stream, make_args<float> (h), comp, h->dim, dev);
     else
-      hipLaunchKernelGGL ((tfsf_mask_kernel<double>), dim3 (grid), dim3 (256), 0, h->stream, make_args<double> (h, 0), comp, h->dim, dev);
+      hipLaunchKernelGGL ((tfsf_mask_kernel<double>), dim3 (grid), dim3 (256), 0, h->stream, make_args<double> (h), comp, h->dim, dev);
     hipError_t e = hipGetLastError ();
     if (e == hipSuccess) e = hipStreamSynchronize (h->stream);
     if (e == hipSuccess) e = hipMemcpy (out, dev, (size_t) h->ncell, hipMemcpyDeviceToHost);
@@ -1988,9 +2035,7 @@ int yee_get_incident (yee_handle *h, double *einc, double *hinc, int64_t len)
   if (!h->use_tfsf ()) return fail (YEE_EINVAL, "TF/SF is not enabled");
   if (len < 0 || len > h->inc_len) return fail (YEE_EINVAL, "length out of range");
   HIP_TRY (hipStreamSynchronize (h->stream));
-  // newest HInc: written by the last completed step into buffer (t - 1) & 1
-  const int newest = (h->t + 1) & 1;
-  void *srcs[2] = { h->einc, h->hinc[newest] };
+  void *srcs[2] = { h->einc[h->inc_cur], h->hinc[h->inc_cur] };
   double *dsts[2] = { einc, hinc };
   for (int s = 0; s < 2; ++s)
   {

@@ -73,8 +73,15 @@ struct yee_handle
 
   void *pml = nullptr;
   int tab_len = 0;
-  void *einc = nullptr, *hinc[2] = { nullptr, nullptr };
+  // incident 1D grid: two buffers (inc_cur: the newer, after the steps before inc_t), and the rows
+  // of the steps [hist_t, inc_t) that the field updates read (incident_steps)
+  void *einc[2] = { nullptr, nullptr }, *hinc[2] = { nullptr, nullptr };
   int64_t inc_len = 0;
+  int inc_cur = 0;
+  int32_t inc_t = 0, hist_t = 0;
+  void *inc_mem = nullptr;   // the allocation of all of them
+  void *hist_e = nullptr, *hist_h = nullptr;
+  int64_t hist_len = 0;
   yee::Scalars sc {};
   double src_t0 = 0, src_sigma = 0;   // Gaussian envelope of the point source (sigma <= 0: none)
   int32_t t = 0;
@@ -123,15 +130,16 @@ struct yee_handle
 
 namespace yee {
 
-// One time step of the handle (the body of yee_step), enqueued on its stream.
-int engine_step_once (yee_handle *h);
+// One time step of the handle (the body of yee_step), enqueued on its stream; the caller takes
+// `ahead` >= 1 steps in a row before it reads or saves the state.
+int engine_step_once (yee_handle *h, int32_t ahead);
 // Padded, zero-filled grid allocation owned by the handle.
 int engine_alloc_grid (yee_handle *h, void **view);
 // Zeroes every field, auxiliary and incident array and resets the step counter.
 int engine_reset (yee_handle *h);
 // Kernel argument block of the handle's current state (in-place half-step view).
 template <typename T>
-StepArgs<T> engine_args (const yee_handle *h, int parity);
+StepArgs<T> engine_args (const yee_handle *h);
 // Frees the adjoint state (called by yee_destroy).
 void adjoint_free (yee_handle *h);
 // Tile grid of a half-step style launch over a.run_lo .. a.run_hi (fills the tile fields of a;

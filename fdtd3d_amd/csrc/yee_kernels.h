@@ -17,9 +17,6 @@ struct TfsfGeom
   double zinc[3];              // zeroIncCoordFP
   double S1, C1, S2, C2;       // sin / cos of the incidence angles
   double proj[6];              // get<comp>FromIncident factors
-  const T *einc;               // EInc after this step's E update (read by H)
-  const T *hinc[2];            // HInc by step parity (E reads the layer after the previous step)
-  int64_t inc_len;
 };
 
 // Geometry and tables common to every half-step kernel.
@@ -68,7 +65,8 @@ struct StepArgs
   int tfsf;
   int tl[3], tr[3];            // total-field box [tl, tr] in integer coordinates
   const struct TfsfGeom<T> *tg;
-  int hinc_sel;                // HInc buffer holding the layer after the previous step
+  const T *einc, *hinc;        // EInc after this step's update (read by H), HInc before it (read by E)
+  int64_t inc_len;             // values in each (rows of the incident history)
 
   // fused step kernel: work decomposition and the point sources it applies in registers
   int lx;                      // x planes per chunk
@@ -100,6 +98,14 @@ struct StepArgs
   double exp_k, exp_d, exp_w, exp_t0, exp_m;
   // Yee layout: 0 E_CENTERED, 1 H_CENTERED (component positions of the test problems)
   int layout;
+};
+
+// Incident steps of one launch (incident_steps) and the source values sin (dt t 2 pi f) at cell 0.
+constexpr int kIncSteps = 32;
+constexpr int kIncTile = 448;   // cells of a workgroup; with 2 kIncSteps of margin 512, two a thread
+struct IncidentSource
+{
+  double v[kIncSteps];
 };
 
 // One box of a half-step launch over several boxes (e_boxes / h_boxes): the cells [lo, hi), tiles

@@ -1680,31 +1680,67 @@ __global__ void batch_advance (int *state, const int *sims, int n, int k)
 }
 
 // ---------------------------------------------------------------------------------------
-// Incident 1D grid: performPlaneWaveESteps then performPlaneWaveHSteps for step t
-// (InternalScheme.inc.h:3276-3357).  One workgroup; only the cells the wave can have
-// reached (i <= t + 2) are touched, the rest are exactly zero in the reference too.
-// EInc is updated in place; HInc is written to the other buffer so the E half-step of
-// this step can still read HInc of the previous step.  The source value sin(dt t 2 pi f)
-// is computed on the host with the C library.
+// Incident 1D grid: performPlaneWaveESteps then performPlaneWaveHSteps of n <= kIncSteps steps
+// from step t0 (InternalScheme.inc.h:3276-3357) in one launch.
+//
+// A workgroup owns kIncTile cells and keeps them and n more on either side in LDS: a step reaches
+// one cell to each side, so the owned cells are exact after n steps while the margin spoils from
+// its ends inward.  The state goes from e0 / h0 to e1 / h1 (other workgroups still read the old
+// values), and the first hist_len cells of every step, all that the TF/SF box of the grid reads,
+// to row s of hist_h (HInc before step t0 + s, read by its E update) and hist_e (EInc after it, read
+// by its H update).  Cells the wave has not reached are zero and stay so.  The values at cell 0
+// come from the host's C library.
+//
+// One step a launch cost 2.3 - 4.5 us each (and more as the wave grew: one workgroup walked all
+// of it); it is pure latency, two barriers and four LDS accesses a step, about 0.3 us of it.
 // ---------------------------------------------------------------------------------------
 template <typename T>
-__global__ __launch_bounds__ (1024) void incident_step (T *einc, const T *hinc_prev, T *hinc_new, int64_t len,
-                                                        int t, double modE, double modH, double src_value)
+__global__ __launch_bounds__ (256) void incident_steps (const T *e0, const T *h0, T *e1, T *h1, int64_t len, int n,
+                                                        double modE, double modH, IncidentSource src, T *hist_e,
+                                                        T *hist_h, int64_t hist_len)
 {
-  const int64_t lim = min (len, (int64_t) t + 3);
-  for (int64_t i = 1 + threadIdx.x; i < lim; i += blockDim.x)
+  __shared__ T e[kIncTile + 2 * kIncSteps], h[kIncTile + 2 * kIncSteps];
+  const int tid = (int) threadIdx.x;
+  const int L = kIncTile + 2 * n;
+  const int64_t base = (int64_t) blockIdx.x * kIncTile - n;   // cell of LDS index 0
+  for (int l = tid; l < L; l += 256)
   {
-    einc[i] = einc[i] + (hinc_prev[i - 1] - hinc_prev[i]) * (T) modE;
-  }
-  if (threadIdx.x == 0)
-  {
-    einc[0] = (T) src_value;
+    const int64_t i = base + l;
+    const bool in = i >= 0 && i < len;
+    e[l] = in ? gld (e0 + i) : (T) 0;
+    h[l] = in ? gld (h0 + i) : (T) 0;
   }
   __syncthreads ();
-  const int64_t limh = min (len - 1, (int64_t) t + 3);
-  for (int64_t i = threadIdx.x; i < limh; i += blockDim.x)
+  for (int s = 0; s < n; ++s)
   {
-    hinc_new[i] = hinc_prev[i] + (einc[i] - einc[i + 1]) * (T) modH;
+    for (int l = tid; l < L; l += 256)
+    {
+      const int64_t i = base + l;
+      const bool own = l >= n && l < n + kIncTile && i < hist_len;
+      const T hv = h[l];
+      T ev = e[l];
+      if (own) gst (hist_h + s * hist_len + i, hv);
+      if (i == 0) ev = (T) src.v[s];
+      else if (l >= 1 && i >= 1 && i < len) ev = ev + (h[l - 1] - hv) * (T) modE;
+      e[l] = ev;
+      if (own) gst (hist_e + s * hist_len + i, ev);
+    }
+    __syncthreads ();
+    for (int l = tid; l + 1 < L; l += 256)
+    {
+      const int64_t i = base + l;
+      if (i >= 0 && i < len - 1) h[l] = h[l] + (e[l] - e[l + 1]) * (T) modH;
+    }
+    __syncthreads ();
+  }
+  for (int l = n + tid; l < n + kIncTile; l += 256)
+  {
+    const int64_t i = base + l;
+    if (i < len)
+    {
+      gst (e1 + i, e[l]);
+      gst (h1 + i, h[l]);
+    }
   }
 }
 
@@ -2004,7 +2040,7 @@ __global__ __launch_bounds__ (256) void ntff_faces (NtffArgs<T> a)
 // Scattered field of one component (Scheme::makeGridScattered, Scheme.inc.h:4113-4228): the
 // newest field minus the incident plane wave at the component's grid points inside the TF/SF
 // box [L, R] (SchemeHelper::doSkipMakeScattered, SchemeHelper.h:905-911: points outside keep
-// the total field).  E takes EInc, H the newest HInc buffer (hsel), interpolated as the TF/SF
+// the total field).  E takes the newest EInc, H the newest HInc (a.einc, a.hinc), interpolated as the TF/SF
 // correction does.
 // Cells [q0, q0 + count) of the flat grid; out[q - q0] receives the value in the field
 // precision, widened to FP64.
@@ -2020,7 +2056,7 @@ __device__ double scattered_incident (const StepArgs<T> &a, int i, int j, int k,
 }
 
 template <typename T, int COMP, int DIM>
-__global__ void scattered_kernel (StepArgs<T> a, const T *f, double *out, int hsel, int64_t q0, int64_t count)
+__global__ void scattered_kernel (StepArgs<T> a, const T *f, double *out, int64_t q0, int64_t count)
 {
   const int nzz = DIM == 3 ? a.nz : 1;
   const int64_t u = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -2030,7 +2066,7 @@ __global__ void scattered_kernel (StepArgs<T> a, const T *f, double *out, int hs
   const int j = (int) ((q / nzz) % a.ny);
   const int i = (int) (q / ((int64_t) nzz * a.ny));
   double v = (double) f[q];
-  const T *inc = COMP >= 3 ? a.tg->hinc[hsel] : a.tg->einc;
+  const T *inc = COMP >= 3 ? a.hinc : a.einc;
   if (a.layout == 0) v -= scattered_incident<T, COMP, DIM, 0> (a, i, j, k, inc);
   else v -= scattered_incident<T, COMP, DIM, 1> (a, i, j, k, inc);
   out[u] = (double) (T) v;
@@ -2113,7 +2149,7 @@ __global__ void tfsf_mask_kernel (StepArgs<T> a, int comp, int dim, uint8_t *out
   template __global__ void batch_tmz_step<T> (const StepArgs<T> *, const int4 *, int, const int *, const T *, int); \
   template __global__ void batch_tmz_step2<T> (const StepArgs<T> *, const int4 *, int, const int *, const T *, int); \
   template __global__ void batch_tmz_sources<T> (const StepArgs<T> *, int, const int *, const T *, int); \
-  template __global__ void incident_step<T> (T *, const T *, T *, int64_t, int, double, double, double); \
+  template __global__ void incident_steps<T> (const T *, const T *, T *, T *, int64_t, int, double, double, IncidentSource, T *, T *, int64_t); \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 0, 16> (StepArgs<T>);            \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 1, 16> (StepArgs<T>);            \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 2, 16> (StepArgs<T>);            \
@@ -2134,18 +2170,18 @@ __global__ void tfsf_mask_kernel (StepArgs<T> a, int comp, int dim, uint8_t *out
   template __global__ void ntff_faces<T> (NtffArgs<T>); \
   template __global__ void test_norm<T> (StepArgs<T>, const T *, const T *, int, int, double, int, int, int, int, int, int, double *); \
   template __global__ void fine_average<T> (const T *, int64_t, int64_t, int64_t, int, int, int, int, int, T *, T *, T *); \
-  template __global__ void scattered_kernel<T, 0, 3> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 1, 3> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 2, 3> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 3, 3> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 4, 3> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 5, 3> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 0, 2> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 1, 2> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 5, 2> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 2, 2> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 3, 2> (StepArgs<T>, const T *, double *, int, int64_t, int64_t); \
-  template __global__ void scattered_kernel<T, 4, 2> (StepArgs<T>, const T *, double *, int, int64_t, int64_t);
+  template __global__ void scattered_kernel<T, 0, 3> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 1, 3> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 2, 3> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 3, 3> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 4, 3> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 5, 3> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 0, 2> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 1, 2> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 5, 2> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 2, 2> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 3, 2> (StepArgs<T>, const T *, double *, int64_t, int64_t); \
+  template __global__ void scattered_kernel<T, 4, 2> (StepArgs<T>, const T *, double *, int64_t, int64_t);
 
 YEE_INST (float)
 YEE_INST (double)

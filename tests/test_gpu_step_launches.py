@@ -43,3 +43,29 @@ def test_boxes_in_one_launch(pos, precision, engine_lib, monkeypatch):
     for n, v in ref.items():
         assert np.array_equal(got[n], v), n
     assert np.abs(ref["Ez"]).max() > 0
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("args", [
+    "--1d-exhy --size z:40 --use-pml --pml-size z:5 --use-tfsf --tfsf-size-left z:12 --tfsf-size-right z:0 --angle-teta 0 "
+    "--angle-phi 0",
+    "--2d-tmz --size x:40,y:33 --use-tfsf --tfsf-size-left x:8,y:7 --tfsf-size-right x:8,y:7 --angle-teta 90 --angle-phi 30",
+    "--3d --size x:14,y:13,z:15 --use-tfsf --tfsf-size-left x:4,y:4,z:4 --tfsf-size-right x:4,y:4,z:4 --angle-teta 140 "
+    "--angle-phi 200 --angle-psi 10",
+])
+def test_incident_steps_in_groups(args, precision, engine_lib):
+    """The incident grid advances up to 32 steps a launch: calls of 1, 31, 32, 33 and 70 steps give
+    the fields and the exported incident grids of single steps (beyond one workgroup's 448 cells)."""
+    cfg = parse_args((args + " --time-steps 1200").split(), precision=precision)
+    out = []
+    for calls in ([1] * 1167, [1, 31, 32, 33, 70, 1000]):
+        eng = Engine(cfg)
+        eng.prepare()
+        for n in calls:
+            eng.step(n)
+        einc, hinc = eng.incident(500 * cfg.size[cfg.active_axes[0]])
+        assert np.count_nonzero(einc) > 448
+        out.append({"einc": einc, "hinc": hinc, **{c: eng.field_raw(c) for c in cfg.components}})
+        eng.close()
+    for n, v in out[0].items():
+        assert np.array_equal(out[1][n], v), n
