@@ -56,15 +56,18 @@ __device__ __forceinline__ void adj_load (const AdjArgs<T> &g, int64_t q, const 
 {
   if (!special) return;
   const StepArgs<T> &a = g.a;
-  const int L = a.tab_len;
-  const T *tab = a.pml + (size_t) COMP * 6 * L;
+  const size_t L = (size_t) a.tab_len;
+  const T *tab = a.pml + COMP * 6 * L;
   o.ad = g.ad[COMP][q];
-  o.cac = tab[0 * L + p[SigAxes<COMP>::c]];
-  o.cbc = tab[1 * L + p[SigAxes<COMP>::c]];
-  o.p4 = tab[2 * L + p[SigAxes<COMP>::s4]];
-  o.m4 = tab[3 * L + p[SigAxes<COMP>::s4]];
-  o.ca5 = tab[4 * L + p[SigAxes<COMP>::s5]];
-  o.dd5 = tab[5 * L + p[SigAxes<COMP>::s5]];
+  const Pair<T> c = gld2 (tab + 2 * p[SigAxes<COMP>::c]);
+  const Pair<T> s4 = gld2 (tab + 2 * L + 2 * p[SigAxes<COMP>::s4]);
+  const Pair<T> s5 = gld2 (tab + 4 * L + 2 * p[SigAxes<COMP>::s5]);
+  o.cac = c.a;
+  o.cbc = c.b;
+  o.p4 = s4.a;
+  o.m4 = s4.b;
+  o.ca5 = s5.a;
+  o.dd5 = s5.b;
 }
 
 template <typename T, int COMP>
@@ -82,11 +85,10 @@ __device__ __forceinline__ T adj_cell (const AdjArgs<T> &g, int64_t q, T av, T m
   }
   else
   {
-    const T mod = mat * modc;
-    const T kp = (o.p4 / mod) / o.dd5, km = (o.m4 / mod) / o.dd5;
-    const T mD = o.ad + kp * av;
+    const Pair<T> k = pml_factors (o.p4, o.m4, mat * modc, o.dd5);
+    const T mD = o.ad + k.a * av;
     w = o.cbc * mD;
-    g.ad[COMP][q] = o.cac * mD - km * av;
+    g.ad[COMP][q] = o.cac * mD - k.b * av;
     g.af[COMP][q] = o.ca5 * av;
   }
   return w;

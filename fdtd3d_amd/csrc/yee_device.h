@@ -25,6 +25,41 @@ __device__ __forceinline__ void gst (T *p, T v)
   *(__attribute__ ((address_space (1))) T *) (p) = v;
 }
 
+// A pair of values at p (aligned to the pair) in one load.
+template <typename T>
+struct Pair
+{
+  T a, b;
+};
+
+__device__ __forceinline__ Pair<float> gld2 (const float *p)
+{
+  typedef float v2 __attribute__ ((ext_vector_type (2)));
+  const v2 v = *(const __attribute__ ((address_space (1))) v2 *) (p);
+  return { v.x, v.y };
+}
+
+__device__ __forceinline__ Pair<double> gld2 (const double *p)
+{
+  typedef double v2 __attribute__ ((ext_vector_type (2)));
+  const v2 v = *(const __attribute__ ((address_space (1))) v2 *) (p);
+  return { v.x, v.y };
+}
+
+// The D/B -> field factors (p4 / mod) / dd5 and (m4 / mod) / dd5 of a PML cell (mod = m m0), with the
+// reference's divisions, which round as it does.  Where no sigma acts along the axis of p4 and m4
+// (most cells of a slab, two components of three) the two are equal and so are the factors: a
+// third of a slab's divisions, each some 12 instructions, is left out.  Every kernel that updates
+// or transposes a PML cell uses this one function.
+template <typename T>
+__device__ __forceinline__ Pair<T> pml_factors (T p4, T m4, T mod, T dd5)
+{
+  Pair<T> k;
+  k.a = k.b = (p4 / mod) / dd5;
+  if (m4 != p4) k.b = (m4 / mod) / dd5;
+  return k;
+}
+
 // Row-relative accessors for the fused kernel: `row` is a uniform base pinned to scalar
 // registers (plane_row), `boff` the lane's byte offset and `delta` an element offset folded
 // into the instruction.  The caller passes offsets taken with fresh_offsets (or an equivalent
@@ -101,24 +136,28 @@ __device__ __forceinline__ bool half_cell (const StepArgs<T> &a, int &i, int &j,
   return j < a.run_hi[1] && k >= a.run_lo[2] && k < a.run_hi[2];
 }
 
-// The same for a launch over several boxes: the box whose tile rows hold blockIdx / 8 (a uniform
-// scan of at most 20 records), then its tile in the XCD's band.  A tile may span several planes
-// (a y face is one row high).
-__device__ __forceinline__ bool half_cell_boxes (const HalfBox *box, int nbox, int &i, int &j, int &k)
+// The same for a launch over several boxes: the box whose tile rows hold blockIdx / 8 (counted
+// in the scalar registers, no chain of loads), then its tile in the XCD's band.  A tile may span
+// several planes (a y face is one row high), but a wave stays on one plane, so that i is uniform
+// and what depends on x alone is read with scalar loads.  flags: the box's.
+__device__ __forceinline__ bool half_cell_boxes (const HalfBox *box, const HalfRows &rows, int &i, int &j, int &k,
+                                                 uint32_t &flags)
 {
   const int b = (int) blockIdx.x;
   const int r = b >> 3;
-  int s = nbox - 1;
-  while (s > 0 && r < box[s].first) --s;
+  int s = -1;
+#pragma unroll
+  for (int q = 0; q < kMaxBoxes; ++q) s += r >= rows.first[q] ? 1 : 0;
   const HalfBox x = box[s];
-  const int u = (b & 7) * x.per_xcd + (r - x.first);
-  if (r - x.first >= x.per_xcd || u >= x.ntile) return false;
+  flags = x.flags;
+  const int u = (b & 7) * x.per_xcd + (r - rows.first[s]);
+  if (r - rows.first[s] >= x.per_xcd || u >= x.ntile) return false;
   const int t = u / x.ntx;
   const int ty = t / x.ntz;
   const int tid = (int) threadIdx.x, lbx = 8 - x.lbz - x.lby;
   k = x.tz0 + ((t - ty * x.ntz) << x.lbz) + (tid & ((1 << x.lbz) - 1));
   j = x.lo[1] + (ty << x.lby) + ((tid >> x.lbz) & ((1 << x.lby) - 1));
-  i = x.lo[0] + ((u - t * x.ntx) << lbx) + (tid >> (x.lbz + x.lby));
+  i = x.lo[0] + ((u - t * x.ntx) << lbx) + __builtin_amdgcn_readfirstlane (tid >> (x.lbz + x.lby));
   return i < x.hi[0] && j < x.hi[1] && k >= x.lo[2] && k < x.hi[2];
 }
 

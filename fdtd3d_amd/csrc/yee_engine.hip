@@ -37,8 +37,8 @@ template <typename T> __global__ void point_source (T *, int64_t, double);
 template <typename T> __global__ void tfsf_mask_kernel (StepArgs<T>, int, int, uint8_t *);
 template <typename T, int COMP, int DIM> __global__ void scattered_kernel (StepArgs<T>, const T *, double *, int64_t, int64_t);
 template <typename T, int BY, int MAT, int MAXW> __global__ void step_3d_fused (StepArgs<T>);
-template <typename T, int MODE> __global__ void e_boxes (StepArgs<T>, const HalfBox *, int, int, double *);
-template <typename T, int MODE> __global__ void h_boxes (StepArgs<T>, const HalfBox *, int);
+template <typename T, int MODE> __global__ void e_boxes (StepArgs<T>, HalfRows, const HalfBox *, int, double *);
+template <typename T, int MODE> __global__ void h_boxes (StepArgs<T>, HalfRows, const HalfBox *);
 template <typename T> __global__ void test_fill (StepArgs<T>, T *, int, int, double, int);
 template <typename T> __global__ void ntff_faces (NtffArgs<T>);
 template <typename T>
@@ -486,7 +486,7 @@ int face_boxes (const yee_handle *h, int64_t lo[9][3], int64_t hi[9][3])
 // leaves them out).  Uploaded once, at yee_prepare.
 int build_boxes (yee_handle *h)
 {
-  int64_t lo[20][3], hi[20][3];
+  int64_t lo[kMaxBoxes][3], hi[kMaxBoxes][3];
   int n = slab_boxes (h, lo, hi);
   n += face_boxes (h, lo + n, hi + n);
   if (h->mode == 2)
@@ -520,6 +520,7 @@ int build_boxes (yee_handle *h)
     // group 1: those that meet it, with the ADE code and its registers
     std::vector<HalfBox> v;
     int64_t rows = 0;
+    std::fill (h->box_rows[g].first, h->box_rows[g].first + kMaxBoxes, INT32_MAX);
     for (int s = 0; s < n; ++s)
     {
       bool meets = h->mode == 2;
@@ -535,7 +536,7 @@ int build_boxes (yee_handle *h)
       }
       // 256 threads: 64 z cells (16 or 32 for z slabs), then rows, then planes, so that few idle
       b.lbz = ext[2] <= 16 ? 4 : (ext[2] <= 32 ? 5 : 6);
-      b.lby = 0;
+      b.lby = 6 - b.lbz;
       while (b.lby < 8 - b.lbz && (1 << b.lby) < ext[1]) ++b.lby;
       const int bz = 1 << b.lbz, by = 1 << b.lby, bx = 256 / (bz * by);
       b.tz0 = ext[2] <= bz ? b.lo[2] : (b.lo[2] & ~(bz - 1));
@@ -544,15 +545,26 @@ int build_boxes (yee_handle *h)
       const int64_t nt = (int64_t) b.ntz * ((ext[1] + by - 1) / by) * b.ntx;
       b.per_xcd = (int) ((nt + 7) / 8);
       b.ntile = (int) nt;
-      b.first = (int) rows;
+      bool all = false, none = true, near = h->use_tfsf ();
+      bool src = (h->cfg.point_source & 0x3fu) != 0, cur = (h->cfg.current_source & 0x3fu) != 0;
+      for (int ax = 0; ax < 3; ++ax)
+      {
+        const int64_t P = h->use_pml () ? h->cfg.pml[ax] : -1, Q = h->use_pml () ? h->n[ax] - P - 1 : (int64_t) 1 << 40;
+        all = all || hi[s][ax] <= P || lo[s][ax] >= Q;
+        none = none && lo[s][ax] >= P && hi[s][ax] <= Q;
+        near = near && lo[s][ax] <= h->n[ax] - h->cfg.tfsf_right[ax] && hi[s][ax] > h->cfg.tfsf_left[ax] - 1;
+        src = src && lo[s][ax] <= sp[ax] && sp[ax] < hi[s][ax];
+        cur = cur && lo[s][ax] <= cp[ax] && cp[ax] < hi[s][ax];
+      }
+      b.flags = (all && g == 0 ? kAllPml : 0) | (none && g == 0 ? kNoPml : 0) | (near ? 0 : kNoTfsf) | (src || cur ? 0 : kNoSource);
+      h->box_rows[g].first[v.size ()] = (int) rows;
       rows += b.per_xcd;
       if (8 * rows > (int64_t) 1 << 30) return fail (YEE_EINVAL, "half-step box too large for one launch");
       v.push_back (b);
     }
-    h->nbox[g] = (int) v.size ();
     h->box_blocks[g] = (int) (8 * rows);
     if (v.empty ()) continue;
-    if (!h->boxes[g]) HIP_TRY (hipMalloc ((void **) &h->boxes[g], 20 * sizeof (HalfBox)));
+    if (!h->boxes[g]) HIP_TRY (hipMalloc ((void **) &h->boxes[g], kMaxBoxes * sizeof (HalfBox)));
     HIP_TRY (hipMemcpy (h->boxes[g], v.data (), v.size () * sizeof (HalfBox), hipMemcpyHostToDevice));
   }
   return YEE_OK;
@@ -566,19 +578,20 @@ int launch_boxes (yee_handle *h, bool e_half)
   const int64_t nz = e_half && h->zcorr ? (3 * h->zc_n[0] * h->zc_n[1] + 255) / 256 : 0;
   for (int g = 0; g < 2; ++g)
   {
-    const int nb = h->nbox[g], blk = h->box_blocks[g];
+    const int blk = h->box_blocks[g];
+    const HalfRows &rows = h->box_rows[g];
     const dim3 grid ((unsigned) (blk + (g == 0 ? nz : 0))), block (256);
     if (grid.x == 0) continue;
     const HalfBox *box = h->boxes[g];
     double *zt = (double *) h->zcorr;
     switch ((g == 1 ? 2 : std::min (h->mode, 1)) * 2 + (e_half ? 0 : 1))
     {
-      case 0: hipLaunchKernelGGL ((e_boxes<T, 0>), grid, block, 0, h->stream, a, box, nb, blk, zt); break;
-      case 1: hipLaunchKernelGGL ((h_boxes<T, 0>), grid, block, 0, h->stream, a, box, nb); break;
-      case 2: hipLaunchKernelGGL ((e_boxes<T, 1>), grid, block, 0, h->stream, a, box, nb, blk, zt); break;
-      case 3: hipLaunchKernelGGL ((h_boxes<T, 1>), grid, block, 0, h->stream, a, box, nb); break;
-      case 4: hipLaunchKernelGGL ((e_boxes<T, 2>), grid, block, 0, h->stream, a, box, nb, blk, zt); break;
-      default: hipLaunchKernelGGL ((h_boxes<T, 2>), grid, block, 0, h->stream, a, box, nb); break;
+      case 0: hipLaunchKernelGGL ((e_boxes<T, 0>), grid, block, 0, h->stream, a, rows, box, blk, zt); break;
+      case 1: hipLaunchKernelGGL ((h_boxes<T, 0>), grid, block, 0, h->stream, a, rows, box); break;
+      case 2: hipLaunchKernelGGL ((e_boxes<T, 1>), grid, block, 0, h->stream, a, rows, box, blk, zt); break;
+      case 3: hipLaunchKernelGGL ((h_boxes<T, 1>), grid, block, 0, h->stream, a, rows, box); break;
+      case 4: hipLaunchKernelGGL ((e_boxes<T, 2>), grid, block, 0, h->stream, a, rows, box, blk, zt); break;
+      default: hipLaunchKernelGGL ((h_boxes<T, 2>), grid, block, 0, h->stream, a, rows, box); break;
     }
     HIP_TRY (hipGetLastError ());
   }

@@ -109,13 +109,25 @@ struct IncidentSource
 };
 
 // One box of a half-step launch over several boxes (e_boxes / h_boxes): the cells [lo, hi), tiles
-// of 2^lbz z cells x 2^lby rows x 256 / that planes from (lo[0], lo[1], tz0), their counts, the
-// tiles per XCD band and the first tile row (blockIdx / 8) of the box in the launch.
+// of 2^lbz z cells x 2^lby rows x 256 / that planes from (lo[0], lo[1], tz0) (lbz + lby >= 6: a wave
+// stays on one plane), their counts, the tiles per XCD band, and what no cell of the box needs.
 struct HalfBox
 {
   int lo[3], hi[3];
   int lbz, lby;
-  int tz0, ntz, ntx, ntile, per_xcd, first;
+  int tz0, ntz, ntx, ntile, per_xcd;
+  uint32_t flags;
+};
+
+// What holds for every cell of a half-step launch: each is a PML cell (is_special), none is, none
+// is next to the TF/SF box, none is the point source or the current source.
+constexpr uint32_t kAllPml = 1, kNoPml = 2, kNoTfsf = 4, kNoSource = 8;
+
+// The first tile row (blockIdx / 8) of every box of a launch (INT_MAX past the last box).
+constexpr int kMaxBoxes = 20;
+struct HalfRows
+{
+  int first[kMaxBoxes];
 };
 
 // Near-to-far-field transform (yee_ntff): the complex fields' two parts, the snapshot of H before

@@ -37,16 +37,12 @@ struct PmlCoef
 template <typename T, int COMP>
 __device__ __forceinline__ PmlCoef<T> pml_coef (const StepArgs<T> &a, const int p[3])
 {
-  const int L = a.tab_len;
-  const T *tab = a.pml + (size_t) COMP * 6 * L;
-  PmlCoef<T> c;
-  c.cac = gld (tab + 0 * L + p[SigAxes<COMP>::c]);
-  c.cbc = gld (tab + 1 * L + p[SigAxes<COMP>::c]);
-  c.p4 = gld (tab + 2 * L + p[SigAxes<COMP>::s4]);
-  c.m4 = gld (tab + 3 * L + p[SigAxes<COMP>::s4]);
-  c.ca5 = gld (tab + 4 * L + p[SigAxes<COMP>::s5]);
-  c.dd5 = gld (tab + 5 * L + p[SigAxes<COMP>::s5]);
-  return c;
+  const size_t L = (size_t) a.tab_len;
+  const T *tab = a.pml + COMP * 6 * L;
+  const Pair<T> c = gld2 (tab + 2 * p[SigAxes<COMP>::c]);
+  const Pair<T> s4 = gld2 (tab + 2 * L + 2 * p[SigAxes<COMP>::s4]);
+  const Pair<T> s5 = gld2 (tab + 4 * L + 2 * p[SigAxes<COMP>::s5]);
+  return { c.a, c.b, s4.a, s4.b, s5.a, s5.b };
 }
 
 // New value of one field component at flat index q (reference formulas, see file header),
@@ -123,8 +119,8 @@ __device__ __forceinline__ T cell_value_pc (const StepArgs<T> &a, int64_t q, T f
     const T a2 = ((T) 4 * M * mat - (T) 2 * dt * M * mat * ga + M * wdt2) / A;
     const T m_new = d_new * b0 + d_old * b1 + d_pp * b2 - m_old * a1 - m_pp * a2;
     // D->E from D1 with modifier 1 (calculateFieldStepIterationPML, useMetamaterials)
-    const T one = (T) 1;
-    f_new = f_old * ca5 + m_new * ((p4 / one) / dd5) - m_old * ((m4 / one) / dd5);
+    const Pair<T> k = pml_factors (p4, m4, (T) 1, dd5);
+    f_new = f_old * ca5 + m_new * k.a - m_old * k.b;
     if (store)
     {
       gst (a.dp_n[COMP] + q, d_old);
@@ -134,49 +130,54 @@ __device__ __forceinline__ T cell_value_pc (const StepArgs<T> &a, int64_t q, T f
   }
   else
   {
-    const T mod = mat * modc;
-    f_new = f_old * ca5 + d_new * ((p4 / mod) / dd5) - d_old * ((m4 / mod) / dd5);
+    const Pair<T> k = pml_factors (p4, m4, mat * modc, dd5);
+    f_new = f_old * ca5 + d_new * k.a - d_old * k.b;
   }
   if (store) gst (a.d_n[COMP] + q, d_new);
   return f_new;
 }
 
-// The same, loading the PML coefficients of cell p where they are needed.
+// Update of one component by the half-step kernels (f -> f_n, the same arrays when in place).  The
+// caller loads the old values and the PML coefficients of all of a cell's components before the
+// first store of the cell: the state pointers may alias as far as the compiler knows, so a load
+// after a store would wait for its own round trip to memory (three of them, one a component, were
+// most of a half step's time on small grids).
 template <typename T, int MODE, int COMP>
-__device__ __forceinline__ T cell_value (const StepArgs<T> &a, int64_t q, const int p[3], T f_old, const Old<T> &old,
-                                         T tmp, T mat, bool special, T om, T ga, bool store)
+__device__ __forceinline__ void update_cell (const StepArgs<T> &a, uint32_t fl, int64_t q, const int p[3], T f_old,
+                                             const Old<T> &old, T tmp, T mat, bool special, T om, T ga,
+                                             const PmlCoef<T> &pc)
 {
-  PmlCoef<T> pc {};
-  if (MODE != 0 && special) pc = pml_coef<T, COMP> (a, p);
+  T jdx = (T) 0;
   // current source J / M of this component at this cell (Scheme.inc.h:1171-1260): current * dx
-  const bool cur = ((a.cur_mask >> COMP) & 1u) && p[0] == a.cur_pos[0] && p[1] == a.cur_pos[1] && p[2] == a.cur_pos[2];
-  const T jdx = cur ? (T) a.cur_val * a.dx : (T) 0;
-  return cell_value_pc<T, MODE, COMP> (a, q, f_old, old, tmp, mat, special, om, ga, store, pc, jdx);
-}
-
-// In-place update of one component (half-step kernels).  The old values are loaded by the
-// caller before any store of the cell, so every load of a thread is in flight at once (the
-// state pointers may alias as far as the compiler knows).
-template <typename T, int MODE, int COMP>
-__device__ __forceinline__ void update_cell (const StepArgs<T> &a, int64_t q, const int p[3], T f_old,
-                                             const Old<T> &old, T tmp, T mat, bool special, T om, T ga)
-{
-  T v = cell_value<T, MODE, COMP> (a, q, p, f_old, old, tmp, mat, special, om, ga, true);
+  if (!(fl & kNoSource) && ((a.cur_mask >> COMP) & 1u) && p[0] == a.cur_pos[0] && p[1] == a.cur_pos[1] && p[2] == a.cur_pos[2])
+    jdx = (T) a.cur_val * a.dx;
+  T v = cell_value_pc<T, MODE, COMP> (a, q, f_old, old, tmp, mat, special, om, ga, true, pc, jdx);
   // hard point source (performPointSourceCalc, InternalScheme.inc.h:2818-2895): it replaces the
   // updated value, so storing it here saves a launch per component and half step
-  if (((a.src_mask >> COMP) & 1u) && p[0] == a.src_pos[0] && p[1] == a.src_pos[1] && p[2] == a.src_pos[2])
+  if (!(fl & kNoSource) && ((a.src_mask >> COMP) & 1u) && p[0] == a.src_pos[0] && p[1] == a.src_pos[1] && p[2] == a.src_pos[2])
     v = (T) a.src_val;
   gst (a.f_n[COMP] + q, v);
 }
 
-// Previous value and (special cells) the D/B history of component COMP at q.
+// Whether a cell of a launch with flags fl takes the two-stage D/B update.
+template <typename T, int MODE>
+__device__ __forceinline__ bool special_cell (const StepArgs<T> &a, uint32_t fl, const int p[3], int dim)
+{
+  if (MODE == 0 || (fl & kNoPml)) return false;
+  return (fl & kAllPml) || is_special (a, p, dim, MODE);
+}
+
+// Previous value and (special cells) the D/B history and PML coefficients of component COMP.
 template <typename T, int MODE, int COMP>
-__device__ __forceinline__ void load_old (const StepArgs<T> &a, int64_t q, bool special, T &f_old, Old<T> &old)
+__device__ __forceinline__ void load_old (const StepArgs<T> &a, int64_t q, const int p[3], bool special, T &f_old,
+                                          Old<T> &old, PmlCoef<T> &pc)
 {
   f_old = gld (a.f[COMP] + q);
   old.d = old.dp = old.m = old.mp = (T) 0;
+  pc = PmlCoef<T> {};
   if (MODE != 0 && special)
   {
+    pc = pml_coef<T, COMP> (a, p);
     old.d = gld (a.d[COMP] + q);
     if (MODE == 2)
     {
@@ -196,19 +197,20 @@ __device__ __forceinline__ void load_old (const StepArgs<T> &a, int64_t q, bool 
 // updating in place).
 // ---------------------------------------------------------------------------------------
 template <typename T, int MODE, int LAY = 0>
-__device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, int i, int j, int k)
+__device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, uint32_t fl, int i, int j, int k)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;
   const int sz = a.sz;   // 1, or 0 when the scheme lacks z (a 1D line along x or y)
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy + k;
   const int p[3] = { i, j, k };
-  const bool special = is_special (a, p, 3, MODE);
+  const bool special = special_cell<T, MODE> (a, fl, p, 3);
   T fo0, fo1, fo2;
   Old<T> do0, do1, do2;
-  load_old<T, MODE, 0> (a, q, special, fo0, do0);
-  load_old<T, MODE, 1> (a, q, special, fo1, do1);
-  load_old<T, MODE, 2> (a, q, special, fo2, do2);
+  PmlCoef<T> pc0, pc1, pc2;
+  load_old<T, MODE, 0> (a, q, p, special, fo0, do0, pc0);
+  load_old<T, MODE, 1> (a, q, p, special, fo1, do1, pc1);
+  load_old<T, MODE, 2> (a, q, p, special, fo2, do2, pc2);
   const T *Hx = a.f[3], *Hy = a.f[4], *Hz = a.f[5];
   const T hx = gld (Hx + q), hy = gld (Hy + q), hz = gld (Hz + q);
   // E_CENTERED: H at {-1, 0} along the derivative axis; H_CENTERED: at {0, +1}
@@ -252,7 +254,7 @@ __device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, int i, int j,
       ez_m = avg4 (gld (m + q), gld (m + q + sy), gld (m + q + sx), gld (m + q + sx + sy));
     }
   }
-  if (a.tfsf && tfsf_near<T, 3> (a, i, j, k))
+  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 3> (a, i, j, k))
   {
     tfsf_apply<T, 0, 3, LAY> (a, i, j, k, vx);
     tfsf_apply<T, 1, 3, LAY> (a, i, j, k, vy);
@@ -275,9 +277,9 @@ __device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, int i, int j,
       gzm = avg2 (gld (g + q), gld (g + q + sz));
     }
   }
-  update_cell<T, MODE, 0> (a, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm);
-  update_cell<T, MODE, 1> (a, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym);
-  update_cell<T, MODE, 2> (a, q, p, fo2, do2, curl_rhs<T, 2> (a, vz, p), ez_m, special, ozm, gzm);
+  update_cell<T, MODE, 0> (a, fl, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm, pc0);
+  update_cell<T, MODE, 1> (a, fl, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym, pc1);
+  update_cell<T, MODE, 2> (a, fl, q, p, fo2, do2, curl_rhs<T, 2> (a, vz, p), ez_m, special, ozm, gzm, pc2);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -285,19 +287,20 @@ __device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, int i, int j,
 // which the host points at the new E when the state is double-buffered.
 // ---------------------------------------------------------------------------------------
 template <typename T, int MODE, int LAY = 0>
-__device__ __forceinline__ void h_half_cell (const StepArgs<T> &a, int i, int j, int k)
+__device__ __forceinline__ void h_half_cell (const StepArgs<T> &a, uint32_t fl, int i, int j, int k)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;
   const int sz = a.sz;   // 1, or 0 when the scheme lacks z (a 1D line along x or y)
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy + k;
   const int p[3] = { i, j, k };
-  const bool special = is_special (a, p, 3, MODE);
+  const bool special = special_cell<T, MODE> (a, fl, p, 3);
   T fo3, fo4, fo5;
   Old<T> do3, do4, do5;
-  load_old<T, MODE, 3> (a, q, special, fo3, do3);
-  load_old<T, MODE, 4> (a, q, special, fo4, do4);
-  load_old<T, MODE, 5> (a, q, special, fo5, do5);
+  PmlCoef<T> pc3, pc4, pc5;
+  load_old<T, MODE, 3> (a, q, p, special, fo3, do3, pc3);
+  load_old<T, MODE, 4> (a, q, p, special, fo4, do4, pc4);
+  load_old<T, MODE, 5> (a, q, p, special, fo5, do5, pc5);
   const T *Ex = a.f[0], *Ey = a.f[1], *Ez = a.f[2];
   const T ex = gld (Ex + q), ey = gld (Ey + q), ez = gld (Ez + q);
   // E_CENTERED: E at {0, +1} along the derivative axis; H_CENTERED: at {-1, 0}
@@ -314,7 +317,7 @@ __device__ __forceinline__ void h_half_cell (const StepArgs<T> &a, int i, int j,
     vy[0] = gld (Ez + q - sx); vy[1] = ez; vy[2] = gld (Ex + q - sz); vy[3] = ex;
     vz[0] = gld (Ex + q - sy); vz[1] = ex; vz[2] = gld (Ey + q - sx); vz[3] = ey;
   }
-  if (a.tfsf && tfsf_near<T, 3> (a, i, j, k))
+  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 3> (a, i, j, k))
   {
     tfsf_apply<T, 3, 3, LAY> (a, i, j, k, vx);
     tfsf_apply<T, 4, 3, LAY> (a, i, j, k, vy);
@@ -363,9 +366,9 @@ __device__ __forceinline__ void h_half_cell (const StepArgs<T> &a, int i, int j,
       gzm = sum4 (gld (g + q), gld (g + q + sy), gld (g + q + sx), gld (g + q + sx + sy));
     }
   }
-  update_cell<T, MODE, 3> (a, q, p, fo3, do3, curl_rhs<T, 3> (a, vx, p), hx_m, special, oxm, gxm);
-  update_cell<T, MODE, 4> (a, q, p, fo4, do4, curl_rhs<T, 4> (a, vy, p), hy_m, special, oym, gym);
-  update_cell<T, MODE, 5> (a, q, p, fo5, do5, curl_rhs<T, 5> (a, vz, p), hz_m, special, ozm, gzm);
+  update_cell<T, MODE, 3> (a, fl, q, p, fo3, do3, curl_rhs<T, 3> (a, vx, p), hx_m, special, oxm, gxm, pc3);
+  update_cell<T, MODE, 4> (a, fl, q, p, fo4, do4, curl_rhs<T, 4> (a, vy, p), hy_m, special, oym, gym, pc4);
+  update_cell<T, MODE, 5> (a, fl, q, p, fo5, do5, curl_rhs<T, 5> (a, vz, p), hz_m, special, ozm, gzm, pc5);
 }
 
 // Drude runs (MODE 2): a cell outside the Drude box has omega_p = gamma = 0 in every average,
@@ -380,8 +383,8 @@ __global__ __launch_bounds__ (256) void e_half_3d (StepArgs<T> a)
   int i, j, k;
   if (!half_cell (a, i, j, k)) return;
   const int p[3] = { i, j, k };
-  if (MODE == 2 && !in_drude_box (a, p, 3)) e_half_cell<T, 1> (a, i, j, k);
-  else e_half_cell<T, MODE> (a, i, j, k);
+  if (MODE == 2 && !in_drude_box (a, p, 3)) e_half_cell<T, 1> (a, 0u, i, j, k);
+  else e_half_cell<T, MODE> (a, 0u, i, j, k);
 }
 
 template <typename T, int MODE>
@@ -390,8 +393,8 @@ __global__ __launch_bounds__ (256) void h_half_3d (StepArgs<T> a)
   int i, j, k;
   if (!half_cell (a, i, j, k)) return;
   const int p[3] = { i, j, k };
-  if (MODE == 2 && !in_drude_box (a, p, 3)) h_half_cell<T, 1> (a, i, j, k);
-  else h_half_cell<T, MODE> (a, i, j, k);
+  if (MODE == 2 && !in_drude_box (a, p, 3)) h_half_cell<T, 1> (a, 0u, i, j, k);
+  else h_half_cell<T, MODE> (a, 0u, i, j, k);
 }
 
 // The H_CENTERED layout (--layout-type 1) on the same half-step cells: plain and PML runs
@@ -401,7 +404,7 @@ __global__ __launch_bounds__ (256) void e_half_3d_hc (StepArgs<T> a)
 {
   int i, j, k;
   if (!half_cell (a, i, j, k)) return;
-  e_half_cell<T, MODE, 1> (a, i, j, k);
+  e_half_cell<T, MODE, 1> (a, 0u, i, j, k);
 }
 
 template <typename T, int MODE>
@@ -409,7 +412,7 @@ __global__ __launch_bounds__ (256) void h_half_3d_hc (StepArgs<T> a)
 {
   int i, j, k;
   if (!half_cell (a, i, j, k)) return;
-  h_half_cell<T, MODE, 1> (a, i, j, k);
+  h_half_cell<T, MODE, 1> (a, 0u, i, j, k);
 }
 
 // One z-face correction entry (tfsf_ztable_entry below) and the half steps of several boxes in
@@ -423,7 +426,7 @@ template <typename T>
 __device__ __forceinline__ void tfsf_ztable_entry (const StepArgs<T> &a, double *out, int64_t u);
 
 template <typename T, int MODE>
-__global__ __launch_bounds__ (256) void e_boxes (StepArgs<T> a, const HalfBox *box, int nbox, int nblk, double *zt)
+__global__ __launch_bounds__ (256) void e_boxes (StepArgs<T> a, HalfRows rows, const HalfBox *box, int nblk, double *zt)
 {
   if ((int) blockIdx.x >= nblk)
   {
@@ -432,20 +435,22 @@ __global__ __launch_bounds__ (256) void e_boxes (StepArgs<T> a, const HalfBox *b
     return;
   }
   int i, j, k;
-  if (!half_cell_boxes (box, nbox, i, j, k)) return;
+  uint32_t fl;
+  if (!half_cell_boxes (box, rows, i, j, k, fl)) return;
   const int p[3] = { i, j, k };
-  if (MODE == 2 && !in_drude_box (a, p, 3)) e_half_cell<T, 1> (a, i, j, k);
-  else e_half_cell<T, MODE> (a, i, j, k);
+  if (MODE == 2 && !in_drude_box (a, p, 3)) e_half_cell<T, 1> (a, fl, i, j, k);
+  else e_half_cell<T, MODE> (a, fl, i, j, k);
 }
 
 template <typename T, int MODE>
-__global__ __launch_bounds__ (256) void h_boxes (StepArgs<T> a, const HalfBox *box, int nbox)
+__global__ __launch_bounds__ (256) void h_boxes (StepArgs<T> a, HalfRows rows, const HalfBox *box)
 {
   int i, j, k;
-  if (!half_cell_boxes (box, nbox, i, j, k)) return;
+  uint32_t fl;
+  if (!half_cell_boxes (box, rows, i, j, k, fl)) return;
   const int p[3] = { i, j, k };
-  if (MODE == 2 && !in_drude_box (a, p, 3)) h_half_cell<T, 1> (a, i, j, k);
-  else h_half_cell<T, MODE> (a, i, j, k);
+  if (MODE == 2 && !in_drude_box (a, p, 3)) h_half_cell<T, 1> (a, fl, i, j, k);
+  else h_half_cell<T, MODE> (a, fl, i, j, k);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1043,19 +1048,20 @@ __global__ __launch_bounds__ (64 * MAXW) void step_3d_fused (StepArgs<T> a)
 // TMz half-steps (Ez; Hx, Hy) on [1, N-1)^2; one thread per cell, y lane-contiguous
 // ---------------------------------------------------------------------------------------
 template <typename T, int MODE>
-__device__ __forceinline__ void tmz_e_cell (const StepArgs<T> &a, int i, int j)
+__device__ __forceinline__ void tmz_e_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;   // == 1
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = is_special (a, p, 2, MODE);
+  const bool special = special_cell<T, MODE> (a, fl, p, 2);
   T fo;
   Old<T> dold;
-  load_old<T, MODE, 2> (a, q, special, fo, dold);
+  PmlCoef<T> pc2;
+  load_old<T, MODE, 2> (a, q, p, special, fo, dold, pc2);
   const T *Hx = a.f[3], *Hy = a.f[4];
   T v[4] = { Hy[q - sx], Hy[q], Hx[q - sy], Hx[q] };
-  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 2, 2> (a, i, j, 0, v);
+  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 2, 2> (a, i, j, 0, v);
   // Ez sits on the eps point: the 2-cell average reads the same cell twice
   const T e = a.eps ? a.eps[q] : a.eps_u;
   const T mat = a.matc[2] ? a.matc[2][q] : avg2 (e, e);
@@ -1066,27 +1072,28 @@ __device__ __forceinline__ void tmz_e_cell (const StepArgs<T> &a, int i, int j)
     om = avg2 (o, o);
     ga = avg2 (g, g);
   }
-  update_cell<T, MODE, 2> (a, q, p, fo, dold, curl_rhs<T, 2> (a, v, p), mat, special, om, ga);
+  update_cell<T, MODE, 2> (a, fl, q, p, fo, dold, curl_rhs<T, 2> (a, v, p), mat, special, om, ga, pc2);
 }
 
 template <typename T, int MODE>
-__device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, int i, int j)
+__device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = is_special (a, p, 2, MODE);
+  const bool special = special_cell<T, MODE> (a, fl, p, 2);
   T fo3, fo4;
   Old<T> do3, do4;
-  load_old<T, MODE, 3> (a, q, special, fo3, do3);
-  load_old<T, MODE, 4> (a, q, special, fo4, do4);
+  PmlCoef<T> pc3, pc4;
+  load_old<T, MODE, 3> (a, q, p, special, fo3, do3, pc3);
+  load_old<T, MODE, 4> (a, q, p, special, fo4, do4, pc4);
   const T *Ez = a.f[2];
   const T ez = Ez[q];
   // Hx: Ey operands absent (0), Ez at (i, j) and (i, j+1); Hy: Ez at (i, j) and (i+1, j), Ex absent
   T vx[4] = { (T) 0, (T) 0, ez, Ez[q + sy] };
   T vy[4] = { ez, Ez[q + sx], (T) 0, (T) 0 };
-  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0))
+  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0))
   {
     tfsf_apply<T, 3, 2> (a, i, j, 0, vx);
     tfsf_apply<T, 4, 2> (a, i, j, 0, vy);
@@ -1122,8 +1129,8 @@ __device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, int i, int j)
       gmy = sum4 (g[q], g[q], g[q + sx], g[q + sx]);
     }
   }
-  update_cell<T, MODE, 3> (a, q, p, fo3, do3, curl_rhs<T, 3> (a, vx, p), mx, special, omx, gmx);
-  update_cell<T, MODE, 4> (a, q, p, fo4, do4, curl_rhs<T, 4> (a, vy, p), my, special, omy, gmy);
+  update_cell<T, MODE, 3> (a, fl, q, p, fo3, do3, curl_rhs<T, 3> (a, vx, p), mx, special, omx, gmx, pc3);
+  update_cell<T, MODE, 4> (a, fl, q, p, fo4, do4, curl_rhs<T, 4> (a, vy, p), my, special, omy, gmy, pc4);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1131,23 +1138,24 @@ __device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, int i, int j)
 // (Hy for Ex, Hx for Ey) read as 0, as for TMz; y lane-contiguous, updated in place
 // ---------------------------------------------------------------------------------------
 template <typename T, int MODE>
-__device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, int i, int j)
+__device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;   // == 1
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = is_special (a, p, 2, MODE);
+  const bool special = special_cell<T, MODE> (a, fl, p, 2);
   T fo0, fo1;
   Old<T> do0, do1;
-  load_old<T, MODE, 0> (a, q, special, fo0, do0);
-  load_old<T, MODE, 1> (a, q, special, fo1, do1);
+  PmlCoef<T> pc0, pc1;
+  load_old<T, MODE, 0> (a, q, p, special, fo0, do0, pc0);
+  load_old<T, MODE, 1> (a, q, p, special, fo1, do1, pc1);
   const T *Hz = a.f[5];
   const T hz = Hz[q];
   // Ex: Hz at (i, j-1) and (i, j), Hy absent; Ey: Hx absent, Hz at (i-1, j) and (i, j)
   T vx[4] = { Hz[q - sy], hz, (T) 0, (T) 0 };
   T vy[4] = { (T) 0, (T) 0, Hz[q - sx], hz };
-  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0))
+  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0))
   {
     tfsf_apply<T, 0, 2> (a, i, j, 0, vx);
     tfsf_apply<T, 1, 2> (a, i, j, 0, vy);
@@ -1179,25 +1187,26 @@ __device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, int i, int j)
       gym = avg2 (a.ge[q], a.ge[q + sy]);
     }
   }
-  update_cell<T, MODE, 0> (a, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm);
-  update_cell<T, MODE, 1> (a, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym);
+  update_cell<T, MODE, 0> (a, fl, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm, pc0);
+  update_cell<T, MODE, 1> (a, fl, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym, pc1);
 }
 
 template <typename T, int MODE>
-__device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, int i, int j)
+__device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = is_special (a, p, 2, MODE);
+  const bool special = special_cell<T, MODE> (a, fl, p, 2);
   T fo5;
   Old<T> do5;
-  load_old<T, MODE, 5> (a, q, special, fo5, do5);
+  PmlCoef<T> pc5;
+  load_old<T, MODE, 5> (a, q, p, special, fo5, do5, pc5);
   const T *Ex = a.f[0], *Ey = a.f[1];
   // Hz: Ex at (i, j) and (i, j+1), Ey at (i, j) and (i+1, j)
   T vz[4] = { Ex[q], Ex[q + sy], Ey[q], Ey[q + sx] };
-  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 5, 2> (a, i, j, 0, vz);
+  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 5, 2> (a, i, j, 0, vz);
   // 4-cell transverse average
   T hz_m = a.mu_u;
   if (a.matc[5])
@@ -1216,7 +1225,7 @@ __device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, int i, int j)
     if (o) ozm = sum4 (o[q], o[q + sy], o[q + sx], o[q + sx + sy]);
     if (g) gzm = sum4 (g[q], g[q + sy], g[q + sx], g[q + sx + sy]);
   }
-  update_cell<T, MODE, 5> (a, q, p, fo5, do5, curl_rhs<T, 5> (a, vz, p), hz_m, special, ozm, gzm);
+  update_cell<T, MODE, 5> (a, fl, q, p, fo5, do5, curl_rhs<T, 5> (a, vz, p), hz_m, special, ozm, gzm, pc5);
 }
 
 template <typename T, int MODE>
@@ -1227,8 +1236,8 @@ __global__ __launch_bounds__ (256) void e_half_tez (StepArgs<T> a)
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
   // outside the Drude box: the PML update (see e_half_3d)
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_e_cell<T, 1> (a, i, j);
-  else tez_e_cell<T, MODE> (a, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_e_cell<T, 1> (a, 0u, i, j);
+  else tez_e_cell<T, MODE> (a, 0u, i, j);
 }
 
 template <typename T, int MODE>
@@ -1238,8 +1247,8 @@ __global__ __launch_bounds__ (256) void h_half_tez (StepArgs<T> a)
   const int i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_h_cell<T, 1> (a, i, j);
-  else tez_h_cell<T, MODE> (a, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_h_cell<T, 1> (a, 0u, i, j);
+  else tez_h_cell<T, MODE> (a, 0u, i, j);
 }
 
 template <typename T, int MODE>
@@ -1250,8 +1259,8 @@ __global__ __launch_bounds__ (256) void e_half_tmz (StepArgs<T> a)
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
   // outside the Drude box: the PML update (see e_half_3d)
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_e_cell<T, 1> (a, i, j);
-  else tmz_e_cell<T, MODE> (a, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_e_cell<T, 1> (a, 0u, i, j);
+  else tmz_e_cell<T, MODE> (a, 0u, i, j);
 }
 
 template <typename T, int MODE>
@@ -1261,8 +1270,8 @@ __global__ __launch_bounds__ (256) void h_half_tmz (StepArgs<T> a)
   const int i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_h_cell<T, 1> (a, i, j);
-  else tmz_h_cell<T, MODE> (a, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_h_cell<T, 1> (a, 0u, i, j);
+  else tmz_h_cell<T, MODE> (a, 0u, i, j);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1314,7 +1323,7 @@ struct TmzColCoef
 template <typename T>
 __device__ __forceinline__ T pml_slot (const StepArgs<T> &a, int comp, int slot, int idx)
 {
-  return gld (a.pml + ((size_t) comp * 6 + slot) * a.tab_len + idx);
+  return gld (a.pml + ((size_t) (comp * 3 + slot / 2) * a.tab_len + idx) * 2 + slot % 2);
 }
 
 // The same as a vector load even for a uniform index (vector loads complete in order, so a
@@ -1325,7 +1334,7 @@ __device__ __forceinline__ T pml_slot_v (const StepArgs<T> &a, int comp, int slo
 {
   int z = 0;
   asm volatile ("" : "+v"(z));
-  return gld (a.pml + ((size_t) comp * 6 + slot) * a.tab_len + idx + z);
+  return gld (a.pml + ((size_t) (comp * 3 + slot / 2) * a.tab_len + idx + z) * 2 + slot % 2);
 }
 
 template <typename T, int MODE>
@@ -1463,8 +1472,8 @@ __device__ __forceinline__ T tmz_update (const StepArgs<T> &a, T f_old, T d_old,
     return f_old * (T) 1.0 + tmp * cb;
   }
   d_new = d_old * pc.cac + tmp * pc.cbc;
-  const T mod = mat * modc;
-  return f_old * pc.ca5 + d_new * ((pc.p4 / mod) / pc.dd5) - d_old * ((pc.m4 / mod) / pc.dd5);
+  const Pair<T> k = pml_factors (pc.p4, pc.m4, mat * modc, pc.dd5);
+  return f_old * pc.ca5 + d_new * k.a - d_old * k.b;
 }
 
 // Row-dependent H coefficients and PML flag of a row, kept for the second step's H update.
@@ -2158,12 +2167,12 @@ __global__ void tfsf_mask_kernel (StepArgs<T> a, int comp, int dim, uint8_t *out
   template __global__ void step_3d_fused<T, FUSED_BY (T), 1, 12> (StepArgs<T>);            \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 2, 12> (StepArgs<T>);            \
   template __global__ void step_3d_fused<T, FUSED_BY (T), 3, 12> (StepArgs<T>);            \
-  template __global__ void e_boxes<T, 0> (StepArgs<T>, const HalfBox *, int, int, double *); \
-  template __global__ void e_boxes<T, 1> (StepArgs<T>, const HalfBox *, int, int, double *); \
-  template __global__ void e_boxes<T, 2> (StepArgs<T>, const HalfBox *, int, int, double *); \
-  template __global__ void h_boxes<T, 0> (StepArgs<T>, const HalfBox *, int);              \
-  template __global__ void h_boxes<T, 1> (StepArgs<T>, const HalfBox *, int);              \
-  template __global__ void h_boxes<T, 2> (StepArgs<T>, const HalfBox *, int);              \
+  template __global__ void e_boxes<T, 0> (StepArgs<T>, HalfRows, const HalfBox *, int, double *); \
+  template __global__ void e_boxes<T, 1> (StepArgs<T>, HalfRows, const HalfBox *, int, double *); \
+  template __global__ void e_boxes<T, 2> (StepArgs<T>, HalfRows, const HalfBox *, int, double *); \
+  template __global__ void h_boxes<T, 0> (StepArgs<T>, HalfRows, const HalfBox *);              \
+  template __global__ void h_boxes<T, 1> (StepArgs<T>, HalfRows, const HalfBox *);              \
+  template __global__ void h_boxes<T, 2> (StepArgs<T>, HalfRows, const HalfBox *);              \
   template __global__ void point_source<T> (T *, int64_t, double);                         \
   template __global__ void tfsf_mask_kernel<T> (StepArgs<T>, int, int, uint8_t *); \
   template __global__ void test_fill<T> (StepArgs<T>, T *, int, int, double, int); \

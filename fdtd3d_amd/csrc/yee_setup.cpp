@@ -304,28 +304,28 @@ std::vector<double> pml_tables (const yee_config &cfg, int64_t tab_len)
   for (int comp = 0; comp < 6; ++comp)
   {
     const CompDesc &c = kComp[comp];
-    double *T = &tab[(size_t) comp * kNumRoles * tab_len];
+    auto T = [&] (int role, int64_t p) -> double & { return tab[pml_index (comp, role, p, tab_len)]; };
     for (int64_t p = 0; p < tab_len; ++p)
     {
       if (axis_active (cfg, c.sig_curl) ? p < cfg.size[c.sig_curl] : p == 0)
       {
         const double m = at (comp, c.sig_curl, p);
         const double dd = (2 * e0 * 1.0 + m * dt);
-        T[kCAC * tab_len + p] = (2 * e0 * 1.0 - m * dt) / dd;
-        T[kCBC * tab_len + p] = (2 * e0 * dt / dx) / dd;
+        T (kCAC, p) = (2 * e0 * 1.0 - m * dt) / dd;
+        T (kCBC, p) = (2 * e0 * dt / dx) / dd;
       }
       if (axis_active (cfg, c.sig4) ? p < cfg.size[c.sig4] : p == 0)
       {
         const double m = at (comp, c.sig4, p);
-        T[kP4 * tab_len + p] = 2 * e0 * 1.0 + m * dt;
-        T[kM4 * tab_len + p] = 2 * e0 * 1.0 - m * dt;
+        T (kP4, p) = 2 * e0 * 1.0 + m * dt;
+        T (kM4, p) = 2 * e0 * 1.0 - m * dt;
       }
       if (axis_active (cfg, c.sig5) ? p < cfg.size[c.sig5] : p == 0)
       {
         const double m = at (comp, c.sig5, p);
         const double dd = (2 * e0 * 1.0 + m * dt);
-        T[kCA5 * tab_len + p] = (2 * e0 * 1.0 - m * dt) / dd;
-        T[kDD5 * tab_len + p] = dd;
+        T (kCA5, p) = (2 * e0 * 1.0 - m * dt) / dd;
+        T (kDD5, p) = dd;
       }
     }
   }

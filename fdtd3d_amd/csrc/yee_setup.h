@@ -76,7 +76,12 @@ std::vector<double> sigma_profile (const yee_config &cfg, int axis);
 //   P4, M4   : 2 eps0 +- sigma4 dt, along sig4  (calculateFieldStepIterationPML, :2620-2627)
 //   CA5, DD5 : Ca and denominator, along sig5
 enum PmlRole { kCAC = 0, kCBC = 1, kP4 = 2, kM4 = 3, kCA5 = 4, kDD5 = 5, kNumRoles = 6 };
-// Returns [comp][role][tab_len] (tab_len = max size), zero-filled where unused.
+// Returns [comp][axis pair][tab_len][2] (tab_len = max size), zero-filled where unused: the two
+// roles of an axis side by side, so that a kernel reads them with one load.
+inline size_t pml_index (int comp, int role, int64_t p, int64_t tab_len)
+{
+  return ((size_t) (comp * 3 + role / 2) * tab_len + p) * 2 + role % 2;
+}
 std::vector<double> pml_tables (const yee_config &cfg, int64_t tab_len);
 
 // Averaged sigma of `comp` along `axis` at index p (InternalScheme::getMaterial on a sigma grid).
