@@ -27,6 +27,7 @@
 
 #include "../../include/yee.h"
 #include "yee_kernels.h"
+#include "yee_readback.h"
 #include "yee_setup.h"
 
 namespace yee {
@@ -68,6 +69,7 @@ struct yee_batch
   std::vector<void *> f[2], d[2];       // [parity][sim][3] Ez, Hx, Hy and Dz, Bx, By
   std::vector<void *> pml;              // [sim] PML tables
   std::vector<int> tab_len;
+  int device = 0;                       // the device current at yee_batch_create
   hipStream_t stream = nullptr;
   hipEvent_t ev[2] = { nullptr, nullptr };
   void *sims = nullptr;                 // StepArgs<T>[nsim][2] (by step parity)
@@ -564,6 +566,7 @@ int yee_batch_create (const yee_config *cfgs, int32_t nsim, yee_batch **out)
       return batch_fail (YEE_EINVAL, "batched point sources must lie in the interior");
   }
   yee_batch *b = new yee_batch ();
+  readback_ref ();
   b->nsim = nsim;
   b->wsize = prec == 4 ? 4 : 8;
   b->cfg.assign (cfgs, cfgs + nsim);
@@ -585,8 +588,8 @@ int yee_batch_create (const yee_config *cfgs, int32_t nsim, yee_batch **out)
   if (hipStreamCreateWithFlags (&b->stream, hipStreamNonBlocking) != hipSuccess) return bail (batch_fail (YEE_EDEVICE, "hipStreamCreate failed"));
   if (hipEventCreate (&b->ev[0]) != hipSuccess || hipEventCreate (&b->ev[1]) != hipSuccess)
     return bail (batch_fail (YEE_EDEVICE, "hipEventCreate failed"));
-  int dev = 0;
-  if (hipGetDevice (&dev) == hipSuccess) (void) hipDeviceGetAttribute (&b->ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  if (hipGetDevice (&b->device) == hipSuccess)
+    (void) hipDeviceGetAttribute (&b->ncu, hipDeviceAttributeMultiprocessorCount, b->device);
   for (int32_t s = 0; s < nsim; ++s)
   {
     const size_t bytes = (size_t) (cfgs[s].size[0] * cfgs[s].size[1]) * b->wsize;
@@ -614,6 +617,7 @@ void yee_batch_destroy (yee_batch *b)
   for (hipEvent_t e : b->ev)
     if (e) (void) hipEventDestroy (e);
   if (b->stream) (void) hipStreamDestroy (b->stream);
+  readback_unref ();
   delete b;
 }
 
@@ -732,16 +736,7 @@ int yee_batch_get_field (yee_batch *b, int32_t sim, int32_t comp, double *out)
     std::fill (out, out + n, 0.0);
     return YEE_OK;
   }
-  if (b->wsize == 4)
-  {
-    std::vector<float> v (n);
-    BHIP (hipMemcpy (v.data (), src, n * 4, hipMemcpyDeviceToHost));
-    for (size_t q = 0; q < n; ++q) out[q] = v[q];
-  }
-  else
-  {
-    BHIP (hipMemcpy (out, src, n * 8, hipMemcpyDeviceToHost));
-  }
+  BHIP (read_back (b->device, b->stream, src, (int64_t) n, b->wsize, out, b->wsize == 4));
   return YEE_OK;
 }
 

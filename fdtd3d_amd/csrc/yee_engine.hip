@@ -19,6 +19,7 @@
 #include "../../include/yee.h"
 #include "yee_internal.h"
 #include "yee_kernels.h"
+#include "yee_readback.h"
 #include "yee_setup.h"
 
 namespace yee {
@@ -483,8 +484,8 @@ int face_boxes (const yee_handle *h, int64_t lo[9][3], int64_t hi[9][3])
 
 // The boxes of the half-step launches around the fused kernel: the PML slabs, the TF/SF x / y
 // faces, the Drude box, the cells of the point source and of the current source (the fused kernel
-// leaves them out).  Uploaded once, at yee_prepare.
-int build_boxes (yee_handle *h)
+// leaves them out).  Built once, at yee_prepare: group 0, then group 1, into `all`.
+int build_boxes (yee_handle *h, std::vector<HalfBox> &all)
 {
   int64_t lo[kMaxBoxes][3], hi[kMaxBoxes][3];
   int n = slab_boxes (h, lo, hi);
@@ -545,27 +546,26 @@ int build_boxes (yee_handle *h)
       const int64_t nt = (int64_t) b.ntz * ((ext[1] + by - 1) / by) * b.ntx;
       b.per_xcd = (int) ((nt + 7) / 8);
       b.ntile = (int) nt;
-      bool all = false, none = true, near = h->use_tfsf ();
+      bool pml = false, none = true, near = h->use_tfsf ();
       bool src = (h->cfg.point_source & 0x3fu) != 0, cur = (h->cfg.current_source & 0x3fu) != 0;
       for (int ax = 0; ax < 3; ++ax)
       {
         const int64_t P = h->use_pml () ? h->cfg.pml[ax] : -1, Q = h->use_pml () ? h->n[ax] - P - 1 : (int64_t) 1 << 40;
-        all = all || hi[s][ax] <= P || lo[s][ax] >= Q;
+        pml = pml || hi[s][ax] <= P || lo[s][ax] >= Q;
         none = none && lo[s][ax] >= P && hi[s][ax] <= Q;
         near = near && lo[s][ax] <= h->n[ax] - h->cfg.tfsf_right[ax] && hi[s][ax] > h->cfg.tfsf_left[ax] - 1;
         src = src && lo[s][ax] <= sp[ax] && sp[ax] < hi[s][ax];
         cur = cur && lo[s][ax] <= cp[ax] && cp[ax] < hi[s][ax];
       }
-      b.flags = (all && g == 0 ? kAllPml : 0) | (none && g == 0 ? kNoPml : 0) | (near ? 0 : kNoTfsf) | (src || cur ? 0 : kNoSource);
+      b.flags = (pml && g == 0 ? kAllPml : 0) | (none && g == 0 ? kNoPml : 0) | (near ? 0 : kNoTfsf) | (src || cur ? 0 : kNoSource);
       h->box_rows[g].first[v.size ()] = (int) rows;
       rows += b.per_xcd;
       if (8 * rows > (int64_t) 1 << 30) return fail (YEE_EINVAL, "half-step box too large for one launch");
       v.push_back (b);
     }
     h->box_blocks[g] = (int) (8 * rows);
-    if (v.empty ()) continue;
-    if (!h->boxes[g]) HIP_TRY (hipMalloc ((void **) &h->boxes[g], kMaxBoxes * sizeof (HalfBox)));
-    HIP_TRY (hipMemcpy (h->boxes[g], v.data (), v.size () * sizeof (HalfBox), hipMemcpyHostToDevice));
+    if (g == 0) h->box_count0 = (int) v.size ();
+    all.insert (all.end (), v.begin (), v.end ());
   }
   return YEE_OK;
 }
@@ -971,7 +971,7 @@ int fine_averages (yee_handle *h)
 }
 
 template <typename T>
-int upload_tfsf_geom (yee_handle *h)
+int upload_geom (yee_handle *h, const std::vector<HalfBox> &boxes)
 {
   TfsfGeom<T> g {};
   for (int ax = 0; ax < 3; ++ax) g.zinc[ax] = h->sc.zero_inc[ax];
@@ -980,8 +980,15 @@ int upload_tfsf_geom (yee_handle *h)
   g.S2 = h->sc.S2;
   g.C2 = h->sc.C2;
   for (int c = 0; c < 6; ++c) g.proj[c] = h->sc.proj[c];
-  if (!h->tg) HIP_TRY (hipMalloc (&h->tg, sizeof g));
-  HIP_TRY (hipMemcpy (h->tg, &g, sizeof g, hipMemcpyHostToDevice));
+  // one buffer: the geometry, then the boxes of the fused step
+  const size_t at = (sizeof g + 63) & ~(size_t) 63;
+  const size_t bytes = at + boxes.size () * sizeof (HalfBox);
+  std::vector<char> buf (bytes);
+  std::memcpy (buf.data (), &g, sizeof g);
+  if (!boxes.empty ()) std::memcpy (buf.data () + at, boxes.data (), boxes.size () * sizeof (HalfBox));
+  if (!h->tg) HIP_TRY (hipMalloc (&h->tg, bytes));
+  HIP_TRY (hipMemcpy (h->tg, buf.data (), bytes, hipMemcpyHostToDevice));
+  for (int k = 0; k < 2; ++k) h->boxes[k] = (HalfBox *) ((char *) h->tg + at) + (k ? h->box_count0 : 0);
   return YEE_OK;
 }
 
@@ -1089,6 +1096,19 @@ int set_exact_exp_part (yee_handle *h, int32_t kind, int32_t pair, double border
   return YEE_OK;
 }
 
+// yee_get_field_raw / yee_get_field: a component in the field precision, or widened to FP64.
+int get_field (yee_handle *h, int32_t comp, void *out, bool widen)
+{
+  if (!h || !out) return fail (YEE_EINVAL, "null argument");
+  if (comp < 0 || comp > 17) return fail (YEE_EINVAL, "unknown component");
+  const int base = comp % 6;
+  if (!h->exposed[base]) return fail (YEE_EINVAL, "component not present in this scheme");
+  const void *src = comp < 6 ? h->f[h->cur][base] : (comp < 12 ? h->d[h->cur][base] : h->d1[h->cur][base]);
+  if (!src) return fail (YEE_EINVAL, "component not allocated (enable PML / metamaterials)");
+  HIP_TRY (read_back (h->device, h->stream, src, h->ncell, h->wsize, out, widen));
+  return YEE_OK;
+}
+
 }  // namespace
 
 namespace yee {
@@ -1157,6 +1177,7 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   int rc = validate (cfg);
   if (rc) return rc;
   yee_handle *h = new yee_handle ();
+  readback_ref ();
   h->cfg = *cfg;
   // 2D schemes on the (y, z) and (x, z) planes run on the 3D kernels with the missing axis of
   // extent 1 (neighbours along it are the cell itself, the offsets the reference drops); TEz
@@ -1363,11 +1384,10 @@ void yee_destroy (yee_handle *h)
   if (h->inc_mem) (void) hipFree (h->inc_mem);
   for (hipEvent_t e : h->ev)
     if (e) (void) hipEventDestroy (e);
-  for (yee::HalfBox *b : h->boxes)
-    if (b) (void) hipFree (b);
   if (h->norm_part) (void) hipFree (h->norm_part);
   if (h->ntff_buf) (void) hipFree (h->ntff_buf);
   if (h->stream) (void) hipStreamDestroy (h->stream);
+  readback_unref ();
   delete h;
 }
 
@@ -1460,8 +1480,12 @@ int yee_prepare (yee_handle *h)
     }
   }
   {
-    // incident-wave geometry of the TF/SF correction, read by the corrected cells only
-    int rc = h->fp32 () ? upload_tfsf_geom<float> (h) : upload_tfsf_geom<double> (h);
+    // incident-wave geometry of the TF/SF correction, read by the corrected cells only, and the
+    // boxes of the fused step
+    std::vector<HalfBox> boxes;
+    int rc = h->fused ? build_boxes (h, boxes) : YEE_OK;
+    if (rc) return rc;
+    rc = h->fp32 () ? upload_geom<float> (h, boxes) : upload_geom<double> (h, boxes);
     if (rc) return rc;
   }
   if (h->fine ())
@@ -1474,11 +1498,6 @@ int yee_prepare (yee_handle *h)
     h->tab_len = (int) std::max (h->n[0], std::max (h->n[1], h->n[2]));
     std::vector<double> tab = pml_tables (h->cfg, h->tab_len);
     int rc = upload (h, &h->pml, tab.data (), tab.size ());
-    if (rc) return rc;
-  }
-  if (h->fused)
-  {
-    int rc = build_boxes (h);
     if (rc) return rc;
   }
   if (h->fn_start)
@@ -1597,26 +1616,12 @@ int yee_last_step_ms (yee_handle *h, double *ms)
 
 int yee_get_field_raw (yee_handle *h, int32_t comp, void *out)
 {
-  if (!h || !out) return fail (YEE_EINVAL, "null argument");
-  if (comp < 0 || comp > 17) return fail (YEE_EINVAL, "unknown component");
-  const int base = comp % 6;
-  if (!h->exposed[base]) return fail (YEE_EINVAL, "component not present in this scheme");
-  void *src = comp < 6 ? h->f[h->cur][base] : (comp < 12 ? h->d[h->cur][base] : h->d1[h->cur][base]);
-  if (!src) return fail (YEE_EINVAL, "component not allocated (enable PML / metamaterials)");
-  HIP_TRY (hipStreamSynchronize (h->stream));
-  HIP_TRY (hipMemcpy (out, src, (size_t) h->ncell * h->wsize, hipMemcpyDeviceToHost));
-  return YEE_OK;
+  return get_field (h, comp, out, false);
 }
 
 int yee_get_field (yee_handle *h, int32_t comp, double *out)
 {
-  if (!h || !out) return fail (YEE_EINVAL, "null argument");
-  if (!h->fp32 ()) return yee_get_field_raw (h, comp, out);
-  std::vector<float> tmp ((size_t) h->ncell);
-  int rc = yee_get_field_raw (h, comp, tmp.data ());
-  if (rc) return rc;
-  for (size_t q = 0; q < tmp.size (); ++q) out[q] = tmp[q];
-  return YEE_OK;
+  return get_field (h, comp, out, h && h->fp32 ());
 }
 
 int yee_material_size (yee_handle *h, int64_t out[3])

@@ -50,8 +50,10 @@ struct yee_handle
   int64_t fbox_lo[3] = { 1, 1, 1 }, fbox_hi[3] = { 1, 1, 1 };   // PML-free box of the fused kernel
   int fused_lx = 0, fused_nstrips = 0, fused_nchunks = 0, fused_threads = 0;
   // boxes of the fused step's half-step launches (device memory): [0] those that miss the Drude
-  // box, [1] those that meet it; their first tile rows and the count of workgroups
-  yee::HalfBox *boxes[2] = { nullptr, nullptr };
+  // box, [1] those that meet it (in the buffer of tg); their first tile rows and the count of
+  // workgroups
+  const yee::HalfBox *boxes[2] = { nullptr, nullptr };
+  int box_count0 = 0;
   yee::HalfRows box_rows[2] = {};
   int box_blocks[2] = { 0, 0 };
   // padded grid allocations (every grid-sized array; the views above point inside them)

@@ -69,3 +69,24 @@ def test_incident_steps_in_groups(args, precision, engine_lib):
         eng.close()
     for n, v in out[0].items():
         assert np.array_equal(out[1][n], v), n
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("size", [(90, 91, 92), (100, 128, 131), (181, 257, 199)])
+def test_large_fields_read_back_in_chunks(size, precision, engine_lib):
+    """Fields on both sides of the least size of the chunked read, with a ragged last chunk: every
+    value of yee_get_field_raw and of yee_get_field (widened from FP32) is the device's."""
+    cfg = parse_args(f"--3d --size x:{size[0]},y:{size[1]},z:{size[2]} --point-source x:40,y:41,z:42 --point-source-ez "
+                     "--time-steps 60".split(), precision=precision)
+    eng = Engine(cfg)
+    eng.prepare()
+    eng.step(60)
+    raw, wide = eng.field_raw("Ez"), eng.field("Ez")
+    assert raw.shape == size and wide.dtype == np.float64
+    assert np.array_equal(raw.astype(np.float64), wide)
+    # the vacuum pattern is mirror symmetric about the source in x: every plane is in its place
+    assert np.count_nonzero(raw) > 1000
+    assert np.allclose(raw[40 + 5, 30:50, 30:50], raw[40 - 5, 30:50, 30:50], rtol=1e-4, atol=1e-9)
+    small = np.array([eng.field_raw("Ez").sum() for _ in range(3)])
+    assert np.all(small == small[0])
+    eng.close()
