@@ -31,7 +31,7 @@ HIP_FLAGS = [
     "-Wall", "-Wno-unused-function", "-Wno-unknown-pragmas",
 ]
 
-SOURCES = ["yee_setup.cpp", "yee_readback.cpp", "yee_kernels.hip", "yee_engine.hip", "yee_batch.hip", "yee_adjoint.hip"]
+SOURCES = ["yee_setup.cpp", "yee_readback.cpp", "yee_kernels.hip", "yee_plane.hip", "yee_engine.hip", "yee_batch.hip", "yee_adjoint.hip"]
 
 
 def hipcc() -> str:

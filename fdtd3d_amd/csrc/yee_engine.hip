@@ -19,6 +19,7 @@
 #include "../../include/yee.h"
 #include "yee_internal.h"
 #include "yee_kernels.h"
+#include "yee_plane.h"
 #include "yee_readback.h"
 #include "yee_setup.h"
 
@@ -1109,9 +1110,62 @@ int get_field (yee_handle *h, int32_t comp, void *out, bool widen)
   return YEE_OK;
 }
 
+// The next steps of a 2D run in one launch (yee_plane.hip), at most `ahead`.  t = 0 (which only
+// fires the sources), Drude media, test functions, current sources and a hard source outside the
+// updated cells take the half-step kernels.
+bool plane_runs (const yee_handle *h)
+{
+  return h->plane && h->t > 0 && !h->fn_any () && !(h->cfg.current_source & 0x3fu)
+         && (!(h->cfg.point_source & 0x3fu) || source_in_update (h));
+}
+
+template <typename T>
+int plane_advance (yee_handle *h, int32_t ahead, int32_t &done)
+{
+  int rc = incident_ahead<T> (h, ahead);
+  if (rc) return rc;
+  int n = (int) std::min<int32_t> (ahead, kPlaneSteps);
+  if (h->use_tfsf ()) n = std::min (n, h->inc_t - h->t);   // the incident rows at hand
+  StepArgs<T> a = make_args<T> (h);
+  for (int c = 0; c < 6; ++c)
+  {
+    a.f_n[c] = (T *) h->f[1 - h->cur][c];
+    a.d_n[c] = (T *) h->d[1 - h->cur][c];
+  }
+  PlaneSource src {};
+  for (int s = 0; s < n && a.src_mask; ++s)
+    for (int half = 0; half < 2; ++half) src.v[s][half] = source_value (h, half == 0, h->t + s);
+  const int ma = missing_axis (h->cfg), ra = ma == 0 ? 1 : 0, ca = ma == 2 ? 1 : 2;
+  PlaneGrid g {};
+  g.n = n;
+  g.margin = n;
+  const int rows = PLANE_RW (T) * kPlaneWaves - 2 * g.margin, cols = 64 - 2 * g.margin;
+  g.ncol = (int) ((h->n[ca] - 2 + cols - 1) / cols);
+  const int64_t nt = (h->n[ra] - 2 + rows - 1) / rows * (int64_t) g.ncol;
+  if (nt > (int64_t) 1 << 28) return fail (YEE_EINVAL, "grid too large for one launch");
+  g.ntile = (int) nt;
+  g.per_xcd = (int) ((nt + 7) / 8);
+  {
+    ProfScope ps (h, 3);
+    launch_plane<T> (h->cfg.scheme, a, g, src, h->stream);
+  }
+  HIP_TRY (hipGetLastError ());
+  h->cur = 1 - h->cur;
+  h->t += n;
+  done = n;
+  return YEE_OK;
+}
+
 }  // namespace
 
 namespace yee {
+
+int engine_steps (yee_handle *h, int32_t ahead, int32_t &done)
+{
+  if (plane_runs (h)) return h->fp32 () ? plane_advance<float> (h, ahead, done) : plane_advance<double> (h, ahead, done);
+  done = 1;
+  return engine_step_once (h, ahead);
+}
 
 int engine_step_once (yee_handle *h, int32_t ahead)
 {
@@ -1296,13 +1350,20 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   // are disjoint, face boxes are clipped to the fused box), so they update in place: the second
   // buffer's views alias the first's.  The Drude box overlaps slab and face boxes, so Drude
   // runs keep two buffers.
-  const int nbuf = h->fused ? 2 : 1;
+  // 2D runs keep two buffers of every array too when they fit (a tile's margin reads old values)
+  {
+    int active = 0;
+    for (int ax = 0; ax < 3; ++ax) active += axis_active (*cfg, ax) ? 1 : 0;
+    h->plane = active == 2 && h->mode <= 1 && cfg->layout == 0 && want_fused
+               && 24.0 * (double) h->ncell * (double) h->wsize < 200e9;
+  }
+  const int nbuf = h->fused || h->plane ? 2 : 1;
   for (int bsel = 0; bsel < nbuf; ++bsel)
     for (int c = 0; c < 6; ++c)
     {
       if (!h->present[c]) continue;
       if ((rc = alloc_grid (h, &h->f[bsel][c]))) return bail (rc);
-      if (bsel == 1 && h->mode == 1)
+      if (bsel == 1 && h->mode == 1 && !h->plane)
       {
         h->d[1][c] = h->d[0][c];
         h->dp[1][c] = h->dp[0][c];
@@ -1517,12 +1578,13 @@ int yee_step (yee_handle *h, int32_t n)
   if (n < 0) return fail (YEE_EINVAL, "negative step count");
   HIP_TRY (hipEventRecord (h->ev[0], h->stream));
   if (h->imag) HIP_TRY (hipStreamWaitEvent (h->imag->stream, h->ev[0], 0));
-  for (int32_t s = 0; s < n; ++s)
+  for (int32_t s = 0, k = 0; s < n; s += k)
   {
-    int rc = engine_step_once (h, n - s);
+    int rc = engine_steps (h, n - s, k);
     if (rc) return rc;
     // complex fields: the imaginary part on its own stream, alongside
-    if (h->imag && (rc = engine_step_once (h->imag, n - s))) return rc;
+    for (int32_t i = 0, ki = 0; h->imag && i < k; i += ki)
+      if ((rc = engine_steps (h->imag, n - s - i, ki))) return rc;
   }
   if (h->imag)
   {

@@ -56,6 +56,8 @@ struct yee_handle
   int box_count0 = 0;
   yee::HalfRows box_rows[2] = {};
   int box_blocks[2] = { 0, 0 };
+  // 2D runs advanced several steps a launch (yee_plane.hip): two buffers of every state array
+  bool plane = false;
   // padded grid allocations (every grid-sized array; the views above point inside them)
   std::vector<void *> grids;
   void *tg = nullptr;   // TfsfGeom<T> in device memory
@@ -133,8 +135,10 @@ struct yee_handle
 
 namespace yee {
 
-// One time step of the handle (the body of yee_step), enqueued on its stream; the caller takes
-// `ahead` >= 1 steps in a row before it reads or saves the state.
+// The next time step of the handle, enqueued on its stream, or several of the `ahead` >= 1 steps that
+// the caller takes in a row before it reads or saves the state; `done`: how many.
+int engine_steps (yee_handle *h, int32_t ahead, int32_t &done);
+// One time step, with `ahead` as above.
 int engine_step_once (yee_handle *h, int32_t ahead);
 // Padded, zero-filled grid allocation owned by the handle.
 int engine_alloc_grid (yee_handle *h, void **view);

@@ -90,3 +90,54 @@ def test_large_fields_read_back_in_chunks(size, precision, engine_lib):
     small = np.array([eng.field_raw("Ez").sum() for _ in range(3)])
     assert np.all(small == small[0])
     eng.close()
+
+
+# 2D schemes by the option, their two axes; sizes around the owned part of a tile (48 x 48 cells in
+# FP32, 32 x 48 in FP64 with the full margin of 8) and the smallest grids
+PLANES = {"tmz": "xy", "tez": "xy", "tex": "yz", "tmx": "yz", "tey": "xz", "tmy": "xz"}
+
+
+def _plane_args(scheme, na, nb, pml, tfsf, source):
+    a, b = PLANES[scheme]
+    s = f"--2d-{scheme} --size {a}:{na},{b}:{nb} --angle-teta {90 if scheme in ('tmz', 'tez') else 40} "
+    s += {"tmz": "--angle-phi 30 ", "tez": "--angle-phi 30 ", "tex": "--angle-phi 90 ", "tmx": "--angle-phi 90 ",
+          "tey": "--angle-phi 0 ", "tmy": "--angle-phi 0 "}[scheme]
+    s += "--angle-psi 0 " if scheme in ("tez", "tex", "tmy") else "--angle-psi 90 "
+    if pml:
+        s += f"--use-pml --pml-size {a}:{pml},{b}:{pml + 1} "
+    if tfsf:
+        s += f"--use-tfsf --tfsf-size-left {a}:{tfsf},{b}:{tfsf + 2} --tfsf-size-right {a}:{tfsf + 1},{b}:{tfsf} "
+    if source:
+        s += f"--point-source {a}:{na // 2},{b}:{nb // 3} --point-source-{source} "
+    return s + "--time-steps 60"
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("scheme,na,nb,pml,tfsf,source", [
+    ("tmz", 98, 99, 6, 12, ""), ("tmz", 50, 50, 0, 0, "ez"), ("tmz", 34, 147, 5, 0, "hx"), ("tmz", 3, 60, 0, 0, "ez"),
+    ("tez", 67, 98, 4, 9, "hz"), ("tez", 131, 49, 0, 11, "ex"), ("tex", 51, 97, 5, 13, "ey"), ("tmx", 66, 51, 6, 0, "hy"),
+    ("tey", 35, 100, 3, 10, "ez"), ("tmy", 99, 66, 7, 13, "hz"), ("tmy", 52, 3, 0, 0, "ey"),
+])
+def test_plane_steps_in_one_launch(scheme, na, nb, pml, tfsf, source, precision, engine_lib, monkeypatch):
+    """Up to 8 steps a launch on register tiles: the fields and D / B of the half-step kernels, bit
+    for bit, however the steps are split into calls, with eps and mu grids."""
+    cfg = parse_args(_plane_args(scheme, na, nb, pml, tfsf, source).split(), precision=precision)
+    rng = np.random.default_rng(11)
+    eps, mu = rng.uniform(1.0, 5.0, size=cfg.shape), rng.uniform(1.0, 2.0, size=cfg.shape)
+    print(f"[gpu] plane {scheme} {na}x{nb} pml {pml} tfsf {tfsf} source {source or '-'} precision {precision}", flush=True)
+    out = []
+    for kernel, calls in (("split", [60]), ("plane", [60]), ("plane", [1, 1, 2, 7, 9, 17, 23])):
+        monkeypatch.setenv("YEE_KERNEL", kernel)
+        eng = Engine(cfg)
+        eng.set_material("eps", eps)
+        eng.set_material("mu", mu)
+        eng.prepare()
+        for n in calls:
+            eng.step(n)
+        names = list(cfg.components) + ([("D" if c[0] == "E" else "B") + c[1] for c in cfg.components] if pml else [])
+        out.append({n: eng.field_raw(n) for n in names})
+        eng.close()
+    for n, v in out[0].items():
+        assert np.array_equal(out[1][n], v), n
+        assert np.array_equal(out[2][n], v), n
+    assert any(np.abs(v).max() > 0 for v in out[0].values())
