@@ -306,24 +306,28 @@ __device__ __forceinline__ bool tfsf_near (const StepArgs<T> &a, int i, int j, i
   return face;
 }
 
+// Distance of component OPP at integer position (i, j, k) along the incident wave
+// (approximateIncidentWave, InternalScheme.cpp:375-407).
+template <typename T, int OPP, int DIM, int LAY = 0>
+__device__ __forceinline__ double incident_distance (const StepArgs<T> &a, int i, int j, int k, double ddiff)
+{
+  const TfsfGeom<T> &tg = *a.tg;
+  const double x = 0.5 * (double) twice_coord<OPP, 0, LAY> (i) - tg.zinc[0];
+  const double y = 0.5 * (double) twice_coord<OPP, 1, LAY> (j) - tg.zinc[1];
+  if (DIM == 3)
+  {
+    const double z = 0.5 * (double) twice_coord<OPP, 2, LAY> (k) - tg.zinc[2];
+    return x * tg.S1 * tg.C2 + y * tg.S1 * tg.S2 + z * tg.C1 - ddiff;
+  }
+  return x * tg.C2 + y * tg.S2 - ddiff;
+}
+
 // Incident value of component OPP at integer position (i, j, k): approximateIncidentWave +
 // get<opp>FromIncident (InternalScheme.cpp:375-407, InternalScheme.inc.h:500-515).
 template <typename T, int OPP, int DIM, int LAY = 0>
 __device__ double incident_at (const StepArgs<T> &a, int i, int j, int k, const T *inc, double ddiff)
 {
-  const TfsfGeom<T> &tg = *a.tg;
-  const double x = 0.5 * (double) twice_coord<OPP, 0, LAY> (i) - tg.zinc[0];
-  const double y = 0.5 * (double) twice_coord<OPP, 1, LAY> (j) - tg.zinc[1];
-  double d;
-  if (DIM == 3)
-  {
-    const double z = 0.5 * (double) twice_coord<OPP, 2, LAY> (k) - tg.zinc[2];
-    d = x * tg.S1 * tg.C2 + y * tg.S1 * tg.S2 + z * tg.C1 - ddiff;
-  }
-  else
-  {
-    d = x * tg.C2 + y * tg.S2 - ddiff;
-  }
+  const double d = incident_distance<T, OPP, DIM, LAY> (a, i, j, k, ddiff);
   const double c1 = (double) (long long) d;
   long long i1 = (long long) c1;
   // the reference asserts d > 0; clamp so a degenerate box can never read out of bounds
@@ -332,7 +336,7 @@ __device__ double incident_at (const StepArgs<T> &a, int i, int j, int k, const 
   const double p2 = d - c1;
   const double p1 = 1 - p2;
   const double v = (double) gld (inc + i1) * p1 + (double) gld (inc + i1 + 1) * p2;
-  return v * tg.proj[OPP];
+  return v * a.tg->proj[OPP];
 }
 
 // One operand pair of calculateTFSF.  E components (E_CENTERED) correct the operand opposite

@@ -222,6 +222,7 @@ StepArgs<T> make_args (const yee_handle *h, ArgRole role = kRoleE)
   a.mu0 = (T) mu0 ();
   a.pml = (const T *) h->pml;
   a.tab_len = h->tab_len;
+  for (int c = 0; c < 6; ++c) a.pfac[c] = (const T *) h->pfac[c];
   a.tfsf = h->use_tfsf () ? 1 : 0;
   a.tg = (const TfsfGeom<T> *) h->tg;
   a.zcorr = (const double *) h->zcorr;
@@ -719,7 +720,7 @@ int incident_ahead (yee_handle *h, int32_t ahead)
   const int64_t cells = std::max (std::min (h->inc_len, (int64_t) h->t + n + 2), h->hist_len);
   const int b = h->inc_cur;
   ProfScope ps (h, 0);
-  hipLaunchKernelGGL ((incident_steps<T>), dim3 ((unsigned) ((cells + kIncTile - 1) / kIncTile)), dim3 (256), 0, h->stream,
+  hipLaunchKernelGGL ((incident_steps<T>), dim3 ((unsigned) ((cells + kIncTile - 1) / kIncTile)), dim3 (64), 0, h->stream,
                      (const T *) h->einc[b], (const T *) h->hinc[b], (T *) h->einc[1 - b], (T *) h->hinc[1 - b],
                      h->inc_len, n, modE, modH, src, (T *) h->hist_e, (T *) h->hist_h, h->hist_len);
   HIP_TRY (hipGetLastError ());
@@ -1136,15 +1137,8 @@ int plane_advance (yee_handle *h, int32_t ahead, int32_t &done)
   for (int s = 0; s < n && a.src_mask; ++s)
     for (int half = 0; half < 2; ++half) src.v[s][half] = source_value (h, half == 0, h->t + s);
   const int ma = missing_axis (h->cfg), ra = ma == 0 ? 1 : 0, ca = ma == 2 ? 1 : 2;
-  PlaneGrid g {};
-  g.n = n;
-  g.margin = n;
-  const int rows = PLANE_RW (T) * kPlaneWaves - 2 * g.margin, cols = 64 - 2 * g.margin;
-  g.ncol = (int) ((h->n[ca] - 2 + cols - 1) / cols);
-  const int64_t nt = (h->n[ra] - 2 + rows - 1) / rows * (int64_t) g.ncol;
-  if (nt > (int64_t) 1 << 28) return fail (YEE_EINVAL, "grid too large for one launch");
-  g.ntile = (int) nt;
-  g.per_xcd = (int) ((nt + 7) / 8);
+  const PlaneGrid g = plane_grid<T> (h->n[ra], h->n[ca], n, h->ncu);
+  if (g.ntile < 0) return fail (YEE_EINVAL, "grid too large for one launch");
   {
     ProfScope ps (h, 3);
     launch_plane<T> (h->cfg.scheme, a, g, src, h->stream);
@@ -1281,6 +1275,7 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     return code;
   };
   if (hipGetDevice (&h->device) != hipSuccess) return bail (fail (YEE_EDEVICE, "hipGetDevice failed"));
+  (void) hipDeviceGetAttribute (&h->ncu, hipDeviceAttributeMultiprocessorCount, h->device);
   hipError_t e = hipStreamCreateWithFlags (&h->stream, hipStreamNonBlocking);
   if (e != hipSuccess) return bail (fail (YEE_EDEVICE, std::string ("hipStreamCreate: ") + hipGetErrorString (e)));
   if (hipEventCreate (&h->ev[0]) != hipSuccess || hipEventCreate (&h->ev[1]) != hipSuccess)
@@ -1313,8 +1308,6 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   if (h->fused)
   {
     const int by = h->fp32 () ? FUSED_BY (float) : FUSED_BY (double);
-    int dev = 0, ncu = 256;
-    if (hipGetDevice (&dev) == hipSuccess) (void) hipDeviceGetAttribute (&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     const int64_t rows = h->fbox_hi[1] - h->fbox_lo[1], planes = h->fbox_hi[0] - h->fbox_lo[0];
     h->fused_nstrips = (int) ((rows + by - 1) / by);
     // x chunks: a CU holds 16 waves of this kernel (<= 128 VGPRs each), i.e. 16 / (waves per
@@ -1322,7 +1315,7 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     // chunk (+1 for the chunk's first plane, read twice): enough workgroups to fill every CU,
     // and no last round left mostly empty.
     const int64_t waves = (h->n[2] + 63) / 64;
-    const int64_t slots = (int64_t) ncu * std::max<int64_t> (1, 16 / waves);
+    const int64_t slots = (int64_t) h->ncu * std::max<int64_t> (1, 16 / waves);
     auto chunk_cost = [&] (int64_t c) {
       const int64_t rounds = (h->fused_nstrips * c + slots - 1) / slots;
       return (double) rounds * (double) ((planes + c - 1) / c + 1);
@@ -1355,7 +1348,7 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     int active = 0;
     for (int ax = 0; ax < 3; ++ax) active += axis_active (*cfg, ax) ? 1 : 0;
     h->plane = active == 2 && h->mode <= 1 && cfg->layout == 0 && want_fused
-               && 24.0 * (double) h->ncell * (double) h->wsize < 200e9;
+               && 36.0 * (double) h->ncell * (double) h->wsize < 200e9;
   }
   const int nbuf = h->fused || h->plane ? 2 : 1;
   for (int bsel = 0; bsel < nbuf; ++bsel)
@@ -1560,6 +1553,18 @@ int yee_prepare (yee_handle *h)
     std::vector<double> tab = pml_tables (h->cfg, h->tab_len);
     int rc = upload (h, &h->pml, tab.data (), tab.size ());
     if (rc) return rc;
+  }
+  if (h->plane && h->use_pml ())
+  {
+    // (one allocation: pairs for each of the scheme's three components)
+    void *p = nullptr;
+    HIP_TRY (hipMalloc (&p, 6 * (size_t) h->ncell * h->wsize));
+    h->grids.push_back (p);
+    for (int c = 0, k = 0; c < 6; ++c)
+      if (h->exposed[c]) h->pfac[c] = (char *) p + 2 * k++ * (size_t) h->ncell * h->wsize;
+    if (h->fp32 ()) launch_plane_factors<float> (h->cfg.scheme, make_args<float> (h), h->stream);
+    else launch_plane_factors<double> (h->cfg.scheme, make_args<double> (h), h->stream);
+    HIP_TRY (hipGetLastError ());
   }
   if (h->fn_start)
   {

@@ -58,6 +58,8 @@ struct yee_handle
   int box_blocks[2] = { 0, 0 };
   // 2D runs advanced several steps a launch (yee_plane.hip): two buffers of every state array
   bool plane = false;
+  void *pfac[6] = {};   // D/B -> field factors of the PML cells (pairs)
+  int ncu = 256;        // compute units of the device
   // padded grid allocations (every grid-sized array; the views above point inside them)
   std::vector<void *> grids;
   void *tg = nullptr;   // TfsfGeom<T> in device memory

@@ -59,6 +59,8 @@ struct StepArgs
   // per-component 1D PML coefficient tables, [comp][role][tab_len]
   const T *pml;
   int tab_len;
+  // 2D runs: the D/B -> field factors of each PML cell, pairs (pml_factors), per component
+  const T *pfac[6];
 
   // TF/SF: the box bounds are tested for every cell; the incident-wave geometry is only read
   // by the O(N^2) corrected cells and lives in device memory (keeps scalar registers free)
@@ -102,7 +104,7 @@ struct StepArgs
 
 // Incident steps of one launch (incident_steps) and the source values sin (dt t 2 pi f) at cell 0.
 constexpr int kIncSteps = 32;
-constexpr int kIncTile = 448;   // cells of a workgroup; with 2 kIncSteps of margin 512, two a thread
+constexpr int kIncTile = 192;   // cells of a wave: 64 lanes of 4, less kIncSteps of margin on both sides
 struct IncidentSource
 {
   double v[kIncSteps];

@@ -1692,65 +1692,77 @@ __global__ void batch_advance (int *state, const int *sims, int n, int k)
 // Incident 1D grid: performPlaneWaveESteps then performPlaneWaveHSteps of n <= kIncSteps steps
 // from step t0 (InternalScheme.inc.h:3276-3357) in one launch.
 //
-// A workgroup owns kIncTile cells and keeps them and n more on either side in LDS: a step reaches
-// one cell to each side, so the owned cells are exact after n steps while the margin spoils from
-// its ends inward.  The state goes from e0 / h0 to e1 / h1 (other workgroups still read the old
-// values), and the first hist_len cells of every step, all that the TF/SF box of the grid reads,
-// to row s of hist_h (HInc before step t0 + s, read by its E update) and hist_e (EInc after it, read
-// by its H update).  Cells the wave has not reached are zero and stay so.  The values at cell 0
-// come from the host's C library.
+// A wave owns kIncTile cells and keeps them and a margin on either side in registers, four to a lane:
+// a step reaches one cell to each side, so the owned cells are exact after n <= kIncSteps steps
+// while the margin spoils from its ends inward.  Neighbours come from the next lane (DPP): no LDS
+// and no barrier.  The state goes from e0 / h0 to e1 / h1 (other waves still read the old values),
+// and the first hist_len cells of every step, all that the TF/SF box of the grid reads, to row s of
+// hist_h (HInc before step t0 + s, read by its E update) and hist_e (EInc after it, read by its H
+// update).  Cells the wave has not reached are zero and stay so.  The values at cell 0 come from
+// the host's C library.
 //
-// One step a launch cost 2.3 - 4.5 us each (and more as the wave grew: one workgroup walked all
-// of it); it is pure latency, two barriers and four LDS accesses a step, about 0.3 us of it.
+// One step a launch cost 2.3 - 4.5 us each, more as the wave grew (one workgroup walked all of
+// it); 32 steps a launch through LDS with two barriers a step 25 us.  It is pure latency: four
+// dependent operations a half step.
 // ---------------------------------------------------------------------------------------
 template <typename T>
-__global__ __launch_bounds__ (256) void incident_steps (const T *e0, const T *h0, T *e1, T *h1, int64_t len, int n,
-                                                        double modE, double modH, IncidentSource src, T *hist_e,
-                                                        T *hist_h, int64_t hist_len)
+__global__ __launch_bounds__ (64) void incident_steps (const T *e0, const T *h0, T *e1, T *h1, int64_t len, int n,
+                                                       double modE, double modH, IncidentSource src, T *hist_e,
+                                                       T *hist_h, int64_t hist_len)
 {
-  __shared__ T e[kIncTile + 2 * kIncSteps], h[kIncTile + 2 * kIncSteps];
-  const int tid = (int) threadIdx.x;
-  const int L = kIncTile + 2 * n;
-  const int64_t base = (int64_t) blockIdx.x * kIncTile - n;   // cell of LDS index 0
-  for (int l = tid; l < L; l += 256)
+  constexpr int C = 4;
+  const int lane = (int) threadIdx.x;
+  const int64_t first = (int64_t) blockIdx.x * kIncTile - kIncSteps + lane * C;   // the lane's first cell
+  T e[C], h[C];
+  bool ein[C], hin[C];   // cells the E and H updates change
+#pragma unroll
+  for (int c = 0; c < C; ++c)
   {
-    const int64_t i = base + l;
+    const int64_t i = first + c;
     const bool in = i >= 0 && i < len;
-    e[l] = in ? gld (e0 + i) : (T) 0;
-    h[l] = in ? gld (h0 + i) : (T) 0;
+    e[c] = in ? gld (e0 + i) : (T) 0;
+    h[c] = in ? gld (h0 + i) : (T) 0;
+    ein[c] = i >= 1 && i < len;
+    hin[c] = i >= 0 && i < len - 1;
   }
-  __syncthreads ();
-  for (int s = 0; s < n; ++s)
+  // lanes 8 .. 55 own their cells (kIncSteps = 8 lanes of margin on either side)
+  const bool own = lane >= kIncSteps / C && lane < 64 - kIncSteps / C;
+  const T mE = (T) modE, mH = (T) modH;
+  T *rh = hist_h + first, *re = hist_e + first;
+  for (int s = 0; s < n; ++s, rh += hist_len, re += hist_len)
   {
-    for (int l = tid; l < L; l += 256)
+    const T hm = lane_prev (h[C - 1], h[C - 1]);
+    const T v0 = (T) src.v[s];
+    T en[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
     {
-      const int64_t i = base + l;
-      const bool own = l >= n && l < n + kIncTile && i < hist_len;
-      const T hv = h[l];
-      T ev = e[l];
-      if (own) gst (hist_h + s * hist_len + i, hv);
-      if (i == 0) ev = (T) src.v[s];
-      else if (l >= 1 && i >= 1 && i < len) ev = ev + (h[l - 1] - hv) * (T) modE;
-      e[l] = ev;
-      if (own) gst (hist_e + s * hist_len + i, ev);
+      const T d = (c ? h[c - 1] : hm) - h[c];
+      en[c] = ein[c] ? e[c] + d * mE : e[c];
+      if (first + c == 0) en[c] = v0;
     }
-    __syncthreads ();
-    for (int l = tid; l + 1 < L; l += 256)
+    const T ep = lane_next (en[0], en[0]);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
     {
-      const int64_t i = base + l;
-      if (i >= 0 && i < len - 1) h[l] = h[l] + (e[l] - e[l + 1]) * (T) modH;
-    }
-    __syncthreads ();
-  }
-  for (int l = n + tid; l < n + kIncTile; l += 256)
-  {
-    const int64_t i = base + l;
-    if (i < len)
-    {
-      gst (e1 + i, e[l]);
-      gst (h1 + i, h[l]);
+      if (own && first + c < hist_len)
+      {
+        gst (rh + c, h[c]);
+        gst (re + c, en[c]);
+      }
+      const T d = en[c] - (c + 1 < C ? en[c + 1] : ep);
+      h[c] = hin[c] ? h[c] + d * mH : h[c];
+      e[c] = en[c];
     }
   }
+  if (!own) return;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    if (first + c < len)
+    {
+      gst (e1 + first + c, e[c]);
+      gst (h1 + first + c, h[c]);
+    }
 }
 
 // Hard point source (performPointSourceCalc, InternalScheme.inc.h:2818-2895).  The sine is

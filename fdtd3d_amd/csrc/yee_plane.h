@@ -7,11 +7,11 @@
 
 namespace yee {
 
-// The most steps of a launch, the waves of a tile and the rows of a wave (FP64 holds half as many
-// values per register).
+// The most steps of a launch, the rows of a wave (FP64 holds half as many values per register) and
+// the waves of a tile.
 constexpr int kPlaneSteps = 8;
-constexpr int kPlaneWaves = 16;
 #define PLANE_RW(T) (sizeof (T) == 4 ? 4 : 3)
+constexpr int kPlaneWaves = 16, kPlaneWavesSmall = 8;
 
 // Tiles of a launch: columns of tiles, their count, tiles per XCD band, the margin of a tile and
 // the steps to take (n <= margin).
@@ -19,13 +19,43 @@ struct PlaneGrid
 {
   int ncol, ntile, per_xcd;
   int margin, n;
+  int waves;
 };
+
+// The tiles of n steps on a plane of nr x nc cells: kPlaneWavesSmall waves while the device's ncu
+// compute units take all such tiles at once (a step of a tile then takes half as long: 100^2 FP64
+// 2.5 us a step with 16 waves, 1.8 with 8), kPlaneWaves where tiles run in turns (less of a larger
+// tile is margin).
+template <typename T>
+PlaneGrid plane_grid (int64_t nr, int64_t nc, int n, int ncu)
+{
+  PlaneGrid g {};
+  g.n = n;
+  g.margin = n;
+  const int64_t cols = 64 - 2 * n;
+  g.ncol = (int) ((nc - 2 + cols - 1) / cols);
+  int64_t nt = 0;
+  for (int w : { kPlaneWavesSmall, kPlaneWaves })
+  {
+    g.waves = w;
+    const int64_t rows = PLANE_RW (T) * w - 2 * n;
+    nt = (nr - 2 + rows - 1) / rows * (int64_t) g.ncol;
+    if (nt <= ncu) break;
+  }
+  g.ntile = nt > (int64_t) 1 << 28 ? -1 : (int) nt;   // -1: too large for one launch
+  g.per_xcd = (int) ((nt + 7) / 8);
+  return g;
+}
 
 // Value of the hard source in every half step of a launch.
 struct PlaneSource
 {
   double v[kPlaneSteps][2];
 };
+
+// Fills a.pfac (arrays of pairs) for the components the scheme has.
+template <typename T>
+void launch_plane_factors (int scheme, const StepArgs<T> &a, hipStream_t stream);
 
 template <typename T>
 void launch_plane (int scheme, const StepArgs<T> &a, const PlaneGrid &g, const PlaneSource &src, hipStream_t stream);

@@ -11,7 +11,8 @@
 // A tile is 64 columns (the lanes, along the contiguous axis) by NW waves of RW rows: column
 // neighbours come from the next lane (DPP), row neighbours from the thread's own registers, and
 // only the rows between two waves go through LDS (one write, one barrier and one read a half step).
-// The coefficients of a cell are divided out once a launch.  Every cell is computed with the
+// The D -> field factors of PML cells (IEEE divisions that took 8 of the 21 us of a launch at 100^2
+// FP64) come from arrays made once, by plane_factors.  Every cell is computed with the
 // expressions of e_half_cell / tmz_e_cell in their order, so the results are the half-step
 // kernels' bits.
 #include <hip/hip_runtime.h>
@@ -87,67 +88,83 @@ struct TileComp
   TileCoef<T, RW> cac, cbc, ca5;
 };
 
-// Averaged material of component COMP at cell q (e_half_cell / h_half_cell with stride 0 along the
-// missing axis): rs, cs the strides of a row and a column.
+// Averaged material of component COMP at byte offset o of the row that starts at cell r0
+// (e_half_cell / h_half_cell with stride 0 along the missing axis); rs: cells of a row.
 template <typename T, class S, int COMP>
-__device__ __forceinline__ T tile_mat (const StepArgs<T> &a, int64_t q, int64_t rs)
+__device__ __forceinline__ T tile_mat (const StepArgs<T> &a, int64_t r0, uint32_t o, int64_t rs)
 {
-  if (a.matc[COMP]) return gld (a.matc[COMP] + q);
+  if (a.matc[COMP]) return rld (a.matc[COMP] + r0, o);
   const T *m = COMP < 3 ? a.eps : a.mu;
   if (!m) return COMP < 3 ? a.eps_u : a.mu_u;
+  const T *m0 = m + r0, *m1 = m0 + rs;
   if constexpr (COMP < 3)
   {
     // 2-cell average along the component's axis (the cell itself along the missing one)
-    const T e = gld (m + q);
-    return avg2 (e, COMP == S::ma ? e : gld (m + q + (COMP == S::ra ? rs : 1)));
+    const T e = rld (m0, o);
+    return avg2 (e, COMP == S::ma ? e : (COMP == S::ra ? rld (m1, o) : rld (m0, o, 1)));
   }
   else
   {
     // 4-cell average across it
     constexpr int ax = COMP - 3;
-    if constexpr (ax == S::ma) return avg4 (gld (m + q), gld (m + q + 1), gld (m + q + rs), gld (m + q + rs + 1));
+    if constexpr (ax == S::ma) return avg4 (rld (m0, o), rld (m0, o, 1), rld (m1, o), rld (m1, o, 1));
     else
     {
-      const T u = gld (m + q), v = gld (m + q + (ax == S::ra ? 1 : rs));
+      const T u = rld (m0, o), v = ax == S::ra ? rld (m0, o, 1) : rld (m1, o);
       return avg4 (u, u, v, v);
     }
   }
 }
 
+// The loads of one component (every address is clamped into the grid, so that none waits for a
+// branch), then, for all three components loaded, tile_factors.
+template <typename T, int RW>
+struct TileRaw
+{
+  T mat[RW];
+  Pair<T> k[RW];
+};
+
 template <typename T, class S, int RW, int COMP, bool PML>
-__device__ __forceinline__ void tile_load (const StepArgs<T> &a, int i0, int j, int64_t q0, int64_t rs, uint32_t in,
-                                           uint32_t upd, uint32_t sp, TileComp<T, RW> &x)
+__device__ __forceinline__ void tile_load (const StepArgs<T> &a, int i0, int j, const int64_t (&r0)[RW], uint32_t o, int64_t rs,
+                                           TileComp<T, RW> &x, TileRaw<T, RW> &w)
+{
+#pragma unroll
+  for (int q = 0; q < RW; ++q)
+  {
+    x.f[q] = rld ((const T *) a.f[COMP] + r0[q], o);
+    w.mat[q] = tile_mat<T, S, COMP> (a, r0[q], o, rs);
+    if (PML)
+    {
+      x.d[q] = rld ((const T *) a.d[COMP] + r0[q], o);
+      // (equal for the component of the missing axis)
+      w.k[q].a = rld (a.pfac[COMP] + 2 * r0[q], 2 * o);
+      if (COMP != S::cc) w.k[q].b = rld (a.pfac[COMP] + 2 * r0[q], 2 * o, 1);
+    }
+  }
+  if (PML)
+  {
+    TileCoef<T, RW> dd5;
+    tile_coef<T, S, RW, COMP, 0> (a, i0, j, x.cac, x.cbc);
+    tile_coef<T, S, RW, COMP, 2> (a, i0, j, x.ca5, dd5);
+  }
+}
+
+template <typename T, class S, int RW, int COMP, bool PML>
+__device__ __forceinline__ void tile_factors (const StepArgs<T> &a, uint32_t in, uint32_t sp, TileComp<T, RW> &x,
+                                              const TileRaw<T, RW> &w)
 {
   const T modc = COMP >= 3 ? a.mu0 : a.eps0;
 #pragma unroll
   for (int q = 0; q < RW; ++q)
   {
-    x.f[q] = (in >> q) & 1u ? gld (a.f[COMP] + q0 + q * rs) : (T) 0;
-    x.d[q] = x.ka[q] = x.kb[q] = (T) 0;
-    if (PML && ((sp >> q) & 1u)) x.d[q] = gld (a.d[COMP] + q0 + q * rs);
-  }
-  TileCoef<T, RW> p4, m4, dd5;
-  if (PML)
-  {
-    tile_coef<T, S, RW, COMP, 0> (a, i0, j, x.cac, x.cbc);
-    tile_coef<T, S, RW, COMP, 1> (a, i0, j, p4, m4);
-    tile_coef<T, S, RW, COMP, 2> (a, i0, j, x.ca5, dd5);
-  }
-#pragma unroll
-  for (int q = 0; q < RW; ++q)
-  {
-    if (!((upd >> q) & 1u)) continue;
-    const T mat = tile_mat<T, S, COMP> (a, q0 + q * rs, rs);
-    if (PML && ((sp >> q) & 1u))
+    const bool s = PML && ((sp >> q) & 1u);
+    if (!((in >> q) & 1u)) x.f[q] = (T) 0;
+    x.ka[q] = direct_cb (a.dt, w.mat[q], modc, a.dx);
+    if (s)
     {
-      const Pair<T> k = pml_factors (coef_at<T, S, RW, COMP, 1> (p4, q), coef_at<T, S, RW, COMP, 1> (m4, q), mat * modc,
-                                     coef_at<T, S, RW, COMP, 2> (dd5, q));
-      x.ka[q] = k.a;
-      x.kb[q] = k.b;
-    }
-    else
-    {
-      x.ka[q] = direct_cb (a.dt, mat, modc, a.dx);
+      x.ka[q] = w.k[q].a;
+      if (COMP != S::cc) x.kb[q] = w.k[q].b;
     }
   }
 }
@@ -160,7 +177,9 @@ __device__ __forceinline__ void tile_update (TileComp<T, RW> &x, int q, T tmp, u
   if (PML && ((sp >> q) & 1u))
   {
     const T d = x.d[q] * coef_at<T, S, RW, COMP, 0> (x.cac, q) + tmp * coef_at<T, S, RW, COMP, 0> (x.cbc, q);
-    x.f[q] = x.f[q] * coef_at<T, S, RW, COMP, 2> (x.ca5, q) + d * x.ka[q] - x.d[q] * x.kb[q];
+    // (the missing axis has no sigma, so the two factors of its component are equal)
+    const T kb = COMP == S::cc ? x.ka[q] : x.kb[q];
+    x.f[q] = x.f[q] * coef_at<T, S, RW, COMP, 2> (x.ca5, q) + d * x.ka[q] - x.d[q] * kb;
     x.d[q] = d;
   }
   else
@@ -193,31 +212,55 @@ struct TileFaces
   double col[kPlaneSteps][2][2][ROWS];
 };
 
-// The correction of the difference along the row (ROWDIR) or column axis of half step `half` (0: E,
-// 1: H) at cell (i, j) on the lo (side 0) or hi (side 1) face.
+// Where a correction reads the incident wave, the same in every step: cells i1 and i1 + 1 with the
+// weights p1 and p2, times the component's projection (incident_at), negated for H.
+struct FacePoint
+{
+  int i1;
+  double p1, p2, proj;
+};
+
+// The correction of operand pair PAIR of component COMP at cell p on the lo (side 0) or hi (side 1)
+// face plane (tfsf_pair_diff); false where there is none.
+template <typename T, int COMP, int PAIR, int DIM>
+__device__ __forceinline__ bool face_point (const StepArgs<T> &a, int side, const int p[3], FacePoint &f)
+{
+  constexpr bool h = COMP >= 3;
+  constexpr int OPP = Tab::opp[COMP][PAIR];
+  const bool on = side == 0 ? tfsf_pred<T, COMP, Tab::dir[COMP][2 * PAIR], DIM> (a, p[0], p[1], p[2])
+                            : tfsf_pred<T, COMP, Tab::dir[COMP][2 * PAIR + 1], DIM> (a, p[0], p[1], p[2]);
+  if (!on) return false;
+  // E corrects the operand across the face (lo face: the hi slot), H the one on its side
+  const bool hi_slot = h ? side == 1 : side == 0;
+  constexpr int lo = 2 * PAIR, hi = 2 * PAIR + 1;
+  const int i = p[0] + (hi_slot ? Tab::off[COMP][hi][0] : Tab::off[COMP][lo][0]);
+  const int j = p[1] + (hi_slot ? Tab::off[COMP][hi][1] : Tab::off[COMP][lo][1]);
+  const int k = DIM == 3 ? p[2] + (hi_slot ? Tab::off[COMP][hi][2] : Tab::off[COMP][lo][2]) : 0;
+  const double d = incident_distance<T, OPP, DIM> (a, i, j, k, h ? 0.0 : 0.5);
+  const double c1 = (double) (long long) d;
+  long long i1 = (long long) c1;
+  if (i1 < 0) i1 = 0;
+  if (i1 > a.inc_len - 2) i1 = a.inc_len - 2;
+  f.i1 = (int) i1;
+  f.p2 = d - c1;
+  f.p1 = 1 - f.p2;
+  f.proj = h ? -a.tg->proj[OPP] : a.tg->proj[OPP];
+  return true;
+}
+
+// The same for the difference along the row (ROWDIR) or column axis of half step `half` (0: E, 1: H).
 template <typename T, class S, bool ROWDIR>
-__device__ double tile_face (const StepArgs<T> &a, int half, int side, int i, int j)
+__device__ __forceinline__ bool tile_face (const StepArgs<T> &a, int half, int side, int i, int j, FacePoint &f)
 {
   int p[3] = { 0, 0, 0 };
   p[S::ra] = i;
   p[S::ca] = j;
-  double lo = 0, hi = 0;
-  if (S::te == (half == 0))
-  {
-    // the two components of the plane: each is differenced along one axis only
-    constexpr int comp = ROWDIR ? S::ck : S::cr;
-    constexpr int b = ROWDIR ? S::ra : S::ca;
-    constexpr int pair = (Tab::dir[comp][0] >> 1) == b ? 0 : 1;
-    tfsf_pair_diff<T, comp, pair, S::dim> (a, p[0], p[1], p[2], lo, hi);
-  }
-  else
-  {
-    constexpr int b = ROWDIR ? S::ra : S::ca;
-    constexpr int pair = (Tab::dir[S::cc][0] >> 1) == b ? 0 : 1;
-    tfsf_pair_diff<T, S::cc, pair, S::dim> (a, p[0], p[1], p[2], lo, hi);
-  }
-  // E corrects the operand across the face (lo face: hi slot), H the one on its side
-  return (half == 0) == (side == 0) ? hi : lo;
+  constexpr int b = ROWDIR ? S::ra : S::ca;
+  // the component of the missing axis is differenced along both axes, the other two along one each
+  constexpr int one = ROWDIR ? S::ck : S::cr;
+  constexpr int pair1 = (Tab::dir[one][0] >> 1) == b ? 0 : 1, pair2 = (Tab::dir[S::cc][0] >> 1) == b ? 0 : 1;
+  if (S::te == (half == 0)) return face_point<T, one, pair1, S::dim> (a, side, p, f);
+  return face_point<T, S::cc, pair2, S::dim> (a, side, p, f);
 }
 
 // What a tile's steps need beside the record: its place and the values of the hard source.
@@ -248,7 +291,8 @@ __device__ __forceinline__ void tile_steps (const StepArgs<T> &a, const TileJob<
   for (int q = 0; q < RW; ++q)
   {
     const int i = i0 + q;
-    const bool g = i >= 0 && i < nr && j >= 0 && j < nc;
+    // (the last row and column are always zero: no step and no source writes them)
+    const bool g = i >= 0 && i < nr - 1 && j >= 0 && j < nc - 1;
     const bool u = i >= 1 && i < nr - 1 && j >= 1 && j < nc - 1;
     const bool s = u && (i < a.slab_lo[S::ra] || i >= a.slab_hi[S::ra] || j < a.slab_lo[S::ca] || j >= a.slab_hi[S::ca]);
     const int li = i - job.x0, lj = j - job.y0;
@@ -257,10 +301,6 @@ __device__ __forceinline__ void tile_steps (const StepArgs<T> &a, const TileJob<
     sp |= s ? 1u << q : 0u;
     own |= u && li >= 0 && li < job.rows && lj >= 0 && lj < job.cols ? 1u << q : 0u;
   }
-  TileComp<T, RW> C, R, K2;
-  tile_load<T, S, RW, S::cc, PML> (a, i0, j, q0, rs, in, upd, sp, C);
-  tile_load<T, S, RW, S::cr, PML> (a, i0, j, q0, rs, in, upd, sp, R);
-  tile_load<T, S, RW, S::ck, PML> (a, i0, j, q0, rs, in, upd, sp, K2);
   // face planes of the TF/SF box as tile rows / lanes: E on L-1 and R, H on L-1 and R-1
   const int tx = job.x0 - K, ty = job.y0 - K;
   const int lo_r = a.tl[S::ra] - 1 - tx, hi_r = a.tr[S::ra] - tx, lo_c = a.tl[S::ca] - 1 - ty, hi_c = a.tr[S::ca] - ty;
@@ -271,30 +311,55 @@ __device__ __forceinline__ void tile_steps (const StepArgs<T> &a, const TileJob<
     fcol = (lo_c >= 0 && lo_c < 64) || (hi_c >= 0 && hi_c <= 64);
     if (frow || fcol)
     {
-      // a task is a face cell of one half step: all its reads of the incident rows are in flight
-      // at once, before the first step needs one
+      // a thread takes a face cell of one half step: where it reads the incident wave is the same
+      // in every step, and the reads of all steps are in flight at once, before the first step
       const int per = 2 * 64 + 2 * ROWS;
-      for (int u = tid; u < job.n * 2 * per; u += 64 * NW)
+      for (int u = tid; u < 2 * per; u += 64 * NW)
       {
-        const int s = u / (2 * per), half = (u / per) & 1, v = u % per;
-        StepArgs<T> b = a;
-        b.einc = a.einc + s * a.inc_len;
-        b.hinc = a.hinc + s * a.inc_len;
-        if (v < 128)
+        const int half = u >= per ? 1 : 0, v = u - half * per;
+        const bool rowdir = v < 128;
+        const int side = rowdir ? v >> 6 : (v - 128) / ROWS;
+        const int at = rowdir ? v & 63 : v - 128 - side * ROWS;   // lane, or row of the tile
+        const int plane = rowdir ? (side ? hi_r - half : lo_r) : (side ? hi_c - half : lo_c);
+        if (plane < 0 || plane >= (rowdir ? ROWS : 64)) continue;   // no such face in the tile
+        const int i = tx + (rowdir ? plane : at), jj = ty + (rowdir ? at : plane);
+        const bool ok = i >= 1 && i < nr - 1 && jj >= 1 && jj < nc - 1;
+        FacePoint f {};
+        const bool on = ok && (rowdir ? tile_face<T, S, true> (a, half, side, i, jj, f) : tile_face<T, S, false> (a, half, side, i, jj, f));
+        const T *inc = half ? a.einc : a.hinc;
+        T g0[kPlaneSteps], g1[kPlaneSteps];
+#pragma unroll
+        for (int s = 0; s < kPlaneSteps; ++s)
         {
-          const int side = v >> 6, i = (side ? hi_r - half : lo_r) + tx, jj = ty + (v & 63);
-          const bool ok = i >= 1 && i < nr - 1 && jj >= 1 && jj < nc - 1;
-          faces->row[s][half][side][v & 63] = ok ? tile_face<T, S, true> (b, half, side, i, jj) : 0.0;
+          const T *r = inc + (s < job.n ? s : 0) * a.inc_len + f.i1;
+          g0[s] = gld (r);
+          g1[s] = gld (r + 1);
         }
-        else
+#pragma unroll
+        for (int s = 0; s < kPlaneSteps; ++s)
         {
-          const int side = (v - 128) / ROWS, r = (v - 128) % ROWS;
-          const int i = tx + r, jj = (side ? hi_c - half : lo_c) + ty;
-          const bool ok = i >= 1 && i < nr - 1 && jj >= 1 && jj < nc - 1;
-          faces->col[s][half][side][r] = ok ? tile_face<T, S, false> (b, half, side, i, jj) : 0.0;
+          const double val = on ? ((double) g0[s] * f.p1 + (double) g1[s] * f.p2) * f.proj : 0.0;
+          if (rowdir) faces->row[s][half][side][at] = val;
+          else faces->col[s][half][side][at] = val;
         }
       }
     }
+  }
+  TileComp<T, RW> C, R, K2;
+  {
+    // clamped below the last row and column, whose cells no step updates (and tile_mat reads one
+    // further)
+    int64_t r0[RW];   // uniform: scalar registers
+#pragma unroll
+    for (int q = 0; q < RW; ++q) r0[q] = (int64_t) max (0, min (i0 + q, nr - 2)) * rs;
+    const uint32_t o = (uint32_t) max (0, min (j, nc - 2)) * (uint32_t) sizeof (T);
+    TileRaw<T, RW> wc, wr, wk;
+    tile_load<T, S, RW, S::cc, PML> (a, i0, j, r0, o, rs, C, wc);
+    tile_load<T, S, RW, S::cr, PML> (a, i0, j, r0, o, rs, R, wr);
+    tile_factors<T, S, RW, S::cc, PML> (a, in, sp, C, wc);
+    tile_load<T, S, RW, S::ck, PML> (a, i0, j, r0, o, rs, K2, wk);
+    tile_factors<T, S, RW, S::cr, PML> (a, in, sp, R, wr);
+    tile_factors<T, S, RW, S::ck, PML> (a, in, sp, K2, wk);
   }
   // the hard source as a row of the thread, and its lane
   const int src_q = a.src_mask ? a.src_pos[S::ra] - i0 : -1;
@@ -430,12 +495,14 @@ __device__ __forceinline__ bool tile_pml (const StepArgs<T> &a, int x0, int y0, 
 }
 
 // n steps of a single run.  Tiles are numbered along the columns and handed to the XCDs in bands.
-template <typename T, int SCHEME, bool TFSF>
-__global__ __launch_bounds__ (64 * kPlaneWaves) void plane_steps (StepArgs<T> a, PlaneGrid g, PlaneSource src)
+// (FP32 without TF/SF: 64 VGPRs, so that a compute unit holds two tiles of 16 waves.)
+template <typename T, int SCHEME, bool TFSF, int NW>
+__global__ __launch_bounds__ (64 * NW, sizeof (T) == 4 && !TFSF && NW == kPlaneWaves ? 8 : 4)
+void plane_steps (StepArgs<T> a, PlaneGrid g, PlaneSource src)
 {
   using S = Plane<SCHEME>;
-  constexpr int RW = PLANE_RW (T), ROWS = RW * kPlaneWaves;
-  __shared__ T xlo[kPlaneWaves + 1][64], xhi[kPlaneWaves + 1][64];
+  constexpr int RW = PLANE_RW (T), ROWS = RW * NW;
+  __shared__ T xlo[NW + 1][64], xhi[NW + 1][64];
   extern __shared__ char dyn[];
   TileFaces<ROWS> *faces = (TileFaces<ROWS> *) dyn;
   const int b = (int) blockIdx.x, u = (b & 7) * g.per_xcd + (b >> 3);
@@ -450,34 +517,91 @@ __global__ __launch_bounds__ (64 * kPlaneWaves) void plane_steps (StepArgs<T> a,
   job.n = g.n;
   auto value = [&] (int s, int half) { return (T) src.v[s][half]; };
   if (tile_pml<T, S> (a, job.x0 - g.margin, job.y0 - g.margin, ROWS, 64))
-    tile_steps<T, S, RW, kPlaneWaves, true, TFSF> (a, job, xlo, xhi, faces, value);
+    tile_steps<T, S, RW, NW, true, TFSF> (a, job, xlo, xhi, faces, value);
   else
-    tile_steps<T, S, RW, kPlaneWaves, false, TFSF> (a, job, xlo, xhi, faces, value);
+    tile_steps<T, S, RW, NW, false, TFSF> (a, job, xlo, xhi, faces, value);
 }
+
+// The D/B -> field factors of the updated PML cells of one component.
+template <typename T, class S, int COMP>
+__device__ __forceinline__ void plane_factor (const StepArgs<T> &a, const int p[3], int64_t r0, int j, int64_t rs)
+{
+  const size_t L = (size_t) a.tab_len;
+  const T *tab = a.pml + COMP * 6 * L;
+  const Pair<T> s4 = gld2 (tab + 2 * L + 2 * p[SigAxes<COMP>::s4]);
+  const Pair<T> s5 = gld2 (tab + 4 * L + 2 * p[SigAxes<COMP>::s5]);
+  const Pair<T> k = pml_factors (s4.a, s4.b, tile_mat<T, S, COMP> (a, r0, (uint32_t) j * (uint32_t) sizeof (T), rs) * (COMP >= 3 ? a.mu0 : a.eps0), s5.b);
+  gst ((T *) a.pfac[COMP] + 2 * (r0 + j), k.a);
+  gst ((T *) a.pfac[COMP] + 2 * (r0 + j) + 1, k.b);
+}
+
+template <typename T, int SCHEME>
+__global__ __launch_bounds__ (256) void plane_factors (StepArgs<T> a)
+{
+  using S = Plane<SCHEME>;
+  const int nr = S::ra == 0 ? a.nx : a.ny, nc = S::ca == 1 ? a.ny : a.nz;
+  const int64_t rs = S::ra == 0 ? a.sx : (int64_t) a.sy;
+  const int64_t n = (int64_t) nr * nc;
+  for (int64_t u = blockIdx.x * (int64_t) 256 + threadIdx.x; u < n; u += (int64_t) gridDim.x * 256)
+  {
+    const int i = (int) (u / nc), j = (int) (u - (int64_t) i * nc);
+    if (i < 1 || i >= nr - 1 || j < 1 || j >= nc - 1) continue;
+    if (i >= a.slab_lo[S::ra] && i < a.slab_hi[S::ra] && j >= a.slab_lo[S::ca] && j < a.slab_hi[S::ca]) continue;
+    int p[3] = { 0, 0, 0 };
+    p[S::ra] = i;
+    p[S::ca] = j;
+    plane_factor<T, S, S::cc> (a, p, i * rs, j, rs);
+    plane_factor<T, S, S::cr> (a, p, i * rs, j, rs);
+    plane_factor<T, S, S::ck> (a, p, i * rs, j, rs);
+  }
+}
+
+template <typename T, int SCHEME>
+void launch_plane_scheme (const StepArgs<T> &a, const PlaneGrid &g, const PlaneSource &src, hipStream_t stream)
+{
+  const dim3 grid ((unsigned) (8 * g.per_xcd)), block (64 * g.waves);
+  constexpr int RW = PLANE_RW (T), NS = kPlaneWavesSmall, NL = kPlaneWaves;
+  if (g.waves == NS && a.tfsf)
+    hipLaunchKernelGGL ((plane_steps<T, SCHEME, true, NS>), grid, block, sizeof (TileFaces<RW * NS>), stream, a, g, src);
+  else if (g.waves == NS)
+    hipLaunchKernelGGL ((plane_steps<T, SCHEME, false, NS>), grid, block, 0, stream, a, g, src);
+  else if (a.tfsf)
+    hipLaunchKernelGGL ((plane_steps<T, SCHEME, true, NL>), grid, block, sizeof (TileFaces<RW * NL>), stream, a, g, src);
+  else
+    hipLaunchKernelGGL ((plane_steps<T, SCHEME, false, NL>), grid, block, 0, stream, a, g, src);
+}
+
+#define YEE_PLANES(X) X (YEE_SCHEME_TEX) X (YEE_SCHEME_TEY) X (YEE_SCHEME_TEZ) X (YEE_SCHEME_TMX) X (YEE_SCHEME_TMY) X (YEE_SCHEME_TMZ)
 
 template <typename T>
 void launch_plane (int scheme, const StepArgs<T> &a, const PlaneGrid &g, const PlaneSource &src, hipStream_t stream)
 {
-  const dim3 grid ((unsigned) (8 * g.per_xcd)), block (64 * kPlaneWaves);
-  const size_t lds = a.tfsf ? sizeof (TileFaces<PLANE_RW (T) * kPlaneWaves>) : 0;
-#define YEE_PLANE(S)                                                                                              \
-  case S:                                                                                                         \
-    if (a.tfsf) hipLaunchKernelGGL ((plane_steps<T, S, true>), grid, block, lds, stream, a, g, src);               \
-    else hipLaunchKernelGGL ((plane_steps<T, S, false>), grid, block, lds, stream, a, g, src);                     \
-    break;
+#define YEE_PLANE(S) case S: launch_plane_scheme<T, S> (a, g, src, stream); break;
   switch (scheme)
   {
-    YEE_PLANE (YEE_SCHEME_TEX)
-    YEE_PLANE (YEE_SCHEME_TEY)
-    YEE_PLANE (YEE_SCHEME_TEZ)
-    YEE_PLANE (YEE_SCHEME_TMX)
-    YEE_PLANE (YEE_SCHEME_TMY)
-    YEE_PLANE (YEE_SCHEME_TMZ)
+    YEE_PLANES (YEE_PLANE)
     default: break;
   }
 #undef YEE_PLANE
 }
+
+template <typename T>
+void launch_plane_factors (int scheme, const StepArgs<T> &a, hipStream_t stream)
+{
+  const int64_t n = (int64_t) a.nx * a.ny * a.nz;
+  const dim3 grid ((unsigned) (n / 256 + 1 < 4096 ? n / 256 + 1 : 4096)), block (256);
+#define YEE_PLANE(S) case S: hipLaunchKernelGGL ((plane_factors<T, S>), grid, block, 0, stream, a); break;
+  switch (scheme)
+  {
+    YEE_PLANES (YEE_PLANE)
+    default: break;
+  }
+#undef YEE_PLANE
+}
+
 template void launch_plane<float> (int, const StepArgs<float> &, const PlaneGrid &, const PlaneSource &, hipStream_t);
 template void launch_plane<double> (int, const StepArgs<double> &, const PlaneGrid &, const PlaneSource &, hipStream_t);
+template void launch_plane_factors<float> (int, const StepArgs<float> &, hipStream_t);
+template void launch_plane_factors<double> (int, const StepArgs<double> &, hipStream_t);
 
 }  // namespace yee
