@@ -1111,7 +1111,7 @@ int get_field (yee_handle *h, int32_t comp, void *out, bool widen)
   return YEE_OK;
 }
 
-// The next steps of a 2D run in one launch (yee_plane.hip), at most `ahead`.  t = 0 (which only
+// The next steps of a 1D or 2D run in one launch (yee_plane.hip), at most `ahead`.  t = 0 (which only
 // fires the sources), Drude media, test functions, current sources and a hard source outside the
 // updated cells take the half-step kernels.
 bool plane_runs (const yee_handle *h)
@@ -1125,7 +1125,8 @@ int plane_advance (yee_handle *h, int32_t ahead, int32_t &done)
 {
   int rc = incident_ahead<T> (h, ahead);
   if (rc) return rc;
-  int n = (int) std::min<int32_t> (ahead, kPlaneSteps);
+  const bool line = line_axis (h->cfg) >= 0;
+  int n = (int) std::min<int32_t> (ahead, line ? kIncSteps : kPlaneSteps);
   if (h->use_tfsf ()) n = std::min (n, h->inc_t - h->t);   // the incident rows at hand
   StepArgs<T> a = make_args<T> (h);
   for (int c = 0; c < 6; ++c)
@@ -1133,13 +1134,24 @@ int plane_advance (yee_handle *h, int32_t ahead, int32_t &done)
     a.f_n[c] = (T *) h->f[1 - h->cur][c];
     a.d_n[c] = (T *) h->d[1 - h->cur][c];
   }
-  PlaneSource src {};
-  for (int s = 0; s < n && a.src_mask; ++s)
-    for (int half = 0; half < 2; ++half) src.v[s][half] = source_value (h, half == 0, h->t + s);
-  const int ma = missing_axis (h->cfg), ra = ma == 0 ? 1 : 0, ca = ma == 2 ? 1 : 2;
-  const PlaneGrid g = plane_grid<T> (h->n[ra], h->n[ca], n, h->ncu);
-  if (g.ntile < 0) return fail (YEE_EINVAL, "grid too large for one launch");
+  auto sources = [&] (double (*v)[2]) {
+    for (int s = 0; s < n && a.src_mask; ++s)
+      for (int half = 0; half < 2; ++half) v[s][half] = source_value (h, half == 0, h->t + s);
+  };
+  if (line)
   {
+    LineSource src {};
+    sources (src.v);
+    ProfScope ps (h, 3);
+    launch_line<T> (h->cfg.scheme, a, n, src, h->stream);
+  }
+  else
+  {
+    PlaneSource src {};
+    sources (src.v);
+    const int ma = missing_axis (h->cfg), ra = ma == 0 ? 1 : 0, ca = ma == 2 ? 1 : 2;
+    const PlaneGrid g = plane_grid<T> (h->n[ra], h->n[ca], n, h->ncu);
+    if (g.ntile < 0) return fail (YEE_EINVAL, "grid too large for one launch");
     ProfScope ps (h, 3);
     launch_plane<T> (h->cfg.scheme, a, g, src, h->stream);
   }
@@ -1343,11 +1355,11 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   // are disjoint, face boxes are clipped to the fused box), so they update in place: the second
   // buffer's views alias the first's.  The Drude box overlaps slab and face boxes, so Drude
   // runs keep two buffers.
-  // 2D runs keep two buffers of every array too when they fit (a tile's margin reads old values)
+  // 1D and 2D runs keep two buffers of every array too when they fit (a tile's margin reads old values)
   {
     int active = 0;
     for (int ax = 0; ax < 3; ++ax) active += axis_active (*cfg, ax) ? 1 : 0;
-    h->plane = active == 2 && h->mode <= 1 && cfg->layout == 0 && want_fused
+    h->plane = active <= 2 && h->mode <= 1 && cfg->layout == 0 && want_fused
                && 36.0 * (double) h->ncell * (double) h->wsize < 200e9;
   }
   const int nbuf = h->fused || h->plane ? 2 : 1;
@@ -1554,7 +1566,7 @@ int yee_prepare (yee_handle *h)
     int rc = upload (h, &h->pml, tab.data (), tab.size ());
     if (rc) return rc;
   }
-  if (h->plane && h->use_pml ())
+  if (h->plane && h->use_pml () && line_axis (h->cfg) < 0)
   {
     // (one allocation: pairs for each of the scheme's three components)
     void *p = nullptr;

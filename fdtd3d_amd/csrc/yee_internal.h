@@ -56,7 +56,7 @@ struct yee_handle
   int box_count0 = 0;
   yee::HalfRows box_rows[2] = {};
   int box_blocks[2] = { 0, 0 };
-  // 2D runs advanced several steps a launch (yee_plane.hip): two buffers of every state array
+  // 1D and 2D runs advanced several steps a launch (yee_plane.hip): two buffers of every state array
   bool plane = false;
   void *pfac[6] = {};   // D/B -> field factors of the PML cells (pairs)
   int ncu = 256;        // compute units of the device

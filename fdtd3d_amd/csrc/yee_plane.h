@@ -1,4 +1,4 @@
-// Several steps of a 2D run in one launch (yee_plane.hip).
+// Several steps of a 2D or 1D run in one launch (yee_plane.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -56,6 +56,16 @@ struct PlaneSource
 // Fills a.pfac (arrays of pairs) for the components the scheme has.
 template <typename T>
 void launch_plane_factors (int scheme, const StepArgs<T> &a, hipStream_t stream);
+
+// Value of the hard source in every half step of a launch of a 1D run.
+struct LineSource
+{
+  double v[kIncSteps][2];
+};
+
+// n <= kIncSteps steps of a 1D run (scheme YEE_SCHEME_EXHY .. EZHY).
+template <typename T>
+void launch_line (int scheme, const StepArgs<T> &a, int n, const LineSource &src, hipStream_t stream);
 
 template <typename T>
 void launch_plane (int scheme, const StepArgs<T> &a, const PlaneGrid &g, const PlaneSource &src, hipStream_t stream);

@@ -599,6 +599,196 @@ void launch_plane_factors (int scheme, const StepArgs<T> &a, hipStream_t stream)
 #undef YEE_PLANE
 }
 
+// ---------------------------------------------------------------------------------------
+// Up to kIncSteps steps of a 1D run in one launch.
+//
+// A line has a few thousand cells at most in practice, so a step is pure latency: three launches
+// took 25 us of it.  As in incident_steps, a wave owns 192 cells and keeps them with a margin of
+// kIncSteps cells on either side in registers, four to a lane; neighbours come from the next lane
+// (DPP), with no LDS, no barrier and no memory access between the first and the last step.  The
+// coefficients of a cell are divided out once a launch, and lane s holds the TF/SF corrections of
+// step s.  Operands and order are those of e_half_cell / h_half_cell.
+// ---------------------------------------------------------------------------------------
+template <int SCHEME>
+struct Line
+{
+  static constexpr int ea = (SCHEME - YEE_SCHEME_EXHY) / 2;                            // Ex Ex Ey Ey Ez Ez
+  static constexpr int ha = SCHEME == YEE_SCHEME_EXHY || SCHEME == YEE_SCHEME_EZHY ? 1
+                            : (SCHEME == YEE_SCHEME_EXHZ || SCHEME == YEE_SCHEME_EYHZ ? 2 : 0);
+  static constexpr int axis = 3 - ea - ha;
+  static constexpr int ce = ea, ch = 3 + ha;
+  static constexpr bool pos = axis == (ea + 1) % 3;   // curl: + d H and + d E, else both negated
+};
+
+// One component of a lane's cells.
+template <typename T>
+struct LineComp
+{
+  T f[4], d[4], k[4], cac[4], cbc[4], ca5[4];
+};
+
+template <typename T, class S, int COMP>
+__device__ __forceinline__ void line_load (const StepArgs<T> &a, int first, int n, uint32_t sp, LineComp<T> &x)
+{
+  const T modc = COMP >= 3 ? a.mu0 : a.eps0;
+  const T *m = COMP < 3 ? a.eps : a.mu;
+  const size_t L = (size_t) a.tab_len;
+  const T *tab = a.pml + COMP * 6 * L;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+  {
+    const int i = max (0, min (first + c, n - 2));   // (the last cell is always zero)
+    const bool in = first + c >= 0 && first + c < n - 1;
+    const T f = gld (a.f[COMP] + i);
+    x.f[c] = in ? f : (T) 0;
+    T mat = COMP < 3 ? a.eps_u : a.mu_u;
+    if (a.matc[COMP]) mat = gld (a.matc[COMP] + i);
+    else if (m && COMP < 3) mat = gld (m + i);                       // 2-cell average of one cell
+    else if (m) mat = avg2 (gld (m + i), gld (m + i + 1));           // 4-cell average of two
+    x.k[c] = direct_cb (a.dt, mat, modc, a.dx);
+    x.d[c] = x.cac[c] = x.cbc[c] = x.ca5[c] = (T) 0;
+    if ((sp >> c) & 1u)
+    {
+      // the component's own axis is not the line's: p4 == m4 and the two factors are one
+      const Pair<T> cu = gld2 (tab + 2 * (SigAxes<COMP>::c == S::axis ? i : 0));
+      const Pair<T> s4 = gld2 (tab + 2 * L), s5 = gld2 (tab + 4 * L + 2 * (SigAxes<COMP>::s5 == S::axis ? i : 0));
+      x.d[c] = gld (a.d[COMP] + i);
+      x.cac[c] = cu.a;
+      x.cbc[c] = cu.b;
+      x.ca5[c] = s5.a;
+      x.k[c] = pml_factors (s4.a, s4.b, mat * modc, s5.b).a;
+    }
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void line_update (LineComp<T> &x, int c, T tmp, uint32_t upd, uint32_t sp)
+{
+  const T direct = x.f[c] * (T) 1.0 + tmp * x.k[c];
+  const T d = x.d[c] * x.cac[c] + tmp * x.cbc[c];
+  const T pml = x.f[c] * x.ca5[c] + d * x.k[c] - x.d[c] * x.k[c];
+  const bool s = (sp >> c) & 1u, u = (upd >> c) & 1u;
+  x.f[c] = s ? pml : (u ? direct : x.f[c]);
+  x.d[c] = s ? d : x.d[c];
+}
+
+// The value of lane s (uniform).
+__device__ __forceinline__ double lane_value (double v, int s)
+{
+  int2 w = __builtin_bit_cast (int2, v);
+  w.x = __builtin_amdgcn_readlane (w.x, s);
+  w.y = __builtin_amdgcn_readlane (w.y, s);
+  return __builtin_bit_cast (double, w);
+}
+
+template <typename T, int SCHEME>
+__global__ __launch_bounds__ (64) void line_steps (StepArgs<T> a, int steps, LineSource src)
+{
+  using S = Line<SCHEME>;
+  const int lane = (int) threadIdx.x;
+  const int n = S::axis == 0 ? a.nx : (S::axis == 1 ? a.ny : a.nz);
+  const int base = 1 + (int) blockIdx.x * kIncTile - kIncSteps, first = base + 4 * lane;
+  const bool mine = lane >= kIncSteps / 4 && lane < 64 - kIncSteps / 4;
+  uint32_t upd = 0, sp = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+  {
+    const int i = first + c;
+    const bool u = i >= 1 && i < n - 1;
+    upd |= u ? 1u << c : 0u;
+    sp |= a.pml && u && (i < a.slab_lo[S::axis] || i >= a.slab_hi[S::axis]) ? 1u << c : 0u;
+  }
+  LineComp<T> E, H;
+  line_load<T, S, S::ce> (a, first, n, sp, E);
+  line_load<T, S, S::ch> (a, first, n, sp, H);
+  // TF/SF: E on cells L-1 (operand H at L-1) and R (H at R-1), H on L-1 (E at L-1) and R-1 (E at R)
+  const int lo = a.tl[S::axis] - 1, hi = a.tr[S::axis];
+  const bool face = a.tfsf && ((lo >= base && lo < base + 256) || (hi >= base && hi <= base + 256));
+  double e_lo = 0, e_hi = 0, h_lo = 0, h_hi = 0;
+  if (face && lane < steps)
+  {
+    constexpr int pe = (Tab::dir[S::ce][0] >> 1) == S::axis ? 0 : 1, ph = (Tab::dir[S::ch][0] >> 1) == S::axis ? 0 : 1;
+    StepArgs<T> b = a;
+    b.einc = a.einc + lane * a.inc_len;
+    b.hinc = a.hinc + lane * a.inc_len;
+    double skip;
+    int p[3] = { 0, 0, 0 };
+    p[S::axis] = lo;
+    tfsf_pair_diff<T, S::ce, pe, 3> (b, p[0], p[1], p[2], skip, e_lo);
+    tfsf_pair_diff<T, S::ch, ph, 3> (b, p[0], p[1], p[2], h_lo, skip);
+    p[S::axis] = hi;
+    tfsf_pair_diff<T, S::ce, pe, 3> (b, p[0], p[1], p[2], e_hi, skip);
+    p[S::axis] = hi - 1;
+    tfsf_pair_diff<T, S::ch, ph, 3> (b, p[0], p[1], p[2], skip, h_hi);
+  }
+  const int at = a.src_mask ? a.src_pos[S::axis] - first : -1;   // the hard source among the lane's cells
+  const bool se = (a.src_mask >> S::ce) & 1u, sh = (a.src_mask >> S::ch) & 1u;
+  for (int s = 0; s < steps; ++s)
+  {
+    {
+      T before = lane_prev (H.f[3], H.f[3]);
+      const double dl = face ? lane_value (e_lo, s) : 0.0, dh = face ? lane_value (e_hi, s) : 0.0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+      {
+        T m = before, z = H.f[c];
+        before = z;
+        if (face && first + c == lo) z = (T) ((double) z - dl);
+        if (face && first + c == hi) m = (T) ((double) m - dh);
+        line_update (E, c, S::pos ? z - m : m - z, upd, sp);
+        if (se && c == at) E.f[c] = (T) src.v[s][0];
+      }
+    }
+    {
+      T after = lane_next (E.f[0], E.f[0]);
+      const double dl = face ? lane_value (h_lo, s) : 0.0, dh = face ? lane_value (h_hi, s) : 0.0;
+#pragma unroll
+      for (int c = 3; c >= 0; --c)
+      {
+        T p = after, z = E.f[c];
+        after = z;
+        if (face && first + c == lo) z = (T) ((double) z - dl);
+        if (face && first + c == hi - 1) p = (T) ((double) p - dh);
+        line_update (H, c, S::pos ? p - z : z - p, upd, sp);
+        if (sh && c == at) H.f[c] = (T) src.v[s][1];
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+  {
+    if (!mine || !((upd >> c) & 1u)) continue;
+    gst (a.f_n[S::ce] + first + c, E.f[c]);
+    gst (a.f_n[S::ch] + first + c, H.f[c]);
+    if ((sp >> c) & 1u)
+    {
+      gst (a.d_n[S::ce] + first + c, E.d[c]);
+      gst (a.d_n[S::ch] + first + c, H.d[c]);
+    }
+  }
+}
+
+template <typename T>
+void launch_line (int scheme, const StepArgs<T> &a, int n, const LineSource &src, hipStream_t stream)
+{
+  const int64_t cells = (int64_t) a.nx * a.ny * a.nz;
+  const dim3 grid ((unsigned) ((cells - 2 + kIncTile - 1) / kIncTile)), block (64);
+#define YEE_LINE(S) case S: hipLaunchKernelGGL ((line_steps<T, S>), grid, block, 0, stream, a, n, src); break;
+  switch (scheme)
+  {
+    YEE_LINE (YEE_SCHEME_EXHY)
+    YEE_LINE (YEE_SCHEME_EXHZ)
+    YEE_LINE (YEE_SCHEME_EYHX)
+    YEE_LINE (YEE_SCHEME_EYHZ)
+    YEE_LINE (YEE_SCHEME_EZHX)
+    YEE_LINE (YEE_SCHEME_EZHY)
+    default: break;
+  }
+#undef YEE_LINE
+}
+
+template void launch_line<float> (int, const StepArgs<float> &, int, const LineSource &, hipStream_t);
+template void launch_line<double> (int, const StepArgs<double> &, int, const LineSource &, hipStream_t);
 template void launch_plane<float> (int, const StepArgs<float> &, const PlaneGrid &, const PlaneSource &, hipStream_t);
 template void launch_plane<double> (int, const StepArgs<double> &, const PlaneGrid &, const PlaneSource &, hipStream_t);
 template void launch_plane_factors<float> (int, const StepArgs<float> &, hipStream_t);

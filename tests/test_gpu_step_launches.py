@@ -141,3 +141,44 @@ def test_plane_steps_in_one_launch(scheme, na, nb, pml, tfsf, source, precision,
         assert np.array_equal(out[1][n], v), n
         assert np.array_equal(out[2][n], v), n
     assert any(np.abs(v).max() > 0 for v in out[0].values())
+
+
+LINES = {"exhy": ("z", 0, 0), "exhz": ("y", 90, 90), "eyhx": ("z", 0, 90), "eyhz": ("x", 90, 0), "ezhx": ("y", 90, 90),
+         "ezhy": ("x", 90, 0)}
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("scheme,n,pml,tfsf,right,source", [
+    ("exhy", 600, 50, 150, 0, ""), ("exhz", 193, 7, 20, 15, ""), ("eyhx", 194, 0, 0, 0, "ey"), ("eyhz", 195, 6, 0, 0, "hz"),
+    ("ezhx", 386, 9, 190, 3, "ez"), ("ezhy", 3, 0, 0, 0, "ez"), ("ezhy", 421, 5, 30, 200, ""),
+])
+def test_line_steps_in_one_launch(scheme, n, pml, tfsf, right, source, precision, engine_lib, monkeypatch):
+    """Up to 32 steps a launch of a 1D line, a wave to 192 cells: the half-step kernels' fields and
+    D / B bit for bit, however the steps are split into calls."""
+    ax, teta, phi = LINES[scheme]
+    s = f"--1d-{scheme} --size {ax}:{n} --angle-teta {teta} --angle-phi {phi} --angle-psi 90 "
+    if pml:
+        s += f"--use-pml --pml-size {ax}:{pml} "
+    if tfsf:
+        s += f"--use-tfsf --tfsf-size-left {ax}:{tfsf} --tfsf-size-right {ax}:{right} "
+    if source:
+        s += f"--point-source {ax}:{max(1, n // 2 - 1)} --point-source-{source} "
+    cfg = parse_args((s + "--time-steps 300").split(), precision=precision)
+    rng = np.random.default_rng(13)
+    eps, mu = rng.uniform(1.0, 5.0, size=cfg.shape), rng.uniform(1.0, 2.0, size=cfg.shape)
+    out = []
+    for kernel, calls in (("split", [300]), ("line", [300]), ("line", [1, 1, 30, 31, 32, 33, 64, 108])):
+        monkeypatch.setenv("YEE_KERNEL", kernel)
+        eng = Engine(cfg)
+        eng.set_material("eps", eps)
+        eng.set_material("mu", mu)
+        eng.prepare()
+        for k in calls:
+            eng.step(k)
+        names = list(cfg.components) + ([("D" if c[0] == "E" else "B") + c[1] for c in cfg.components] if pml else [])
+        out.append({c: eng.field_raw(c) for c in names})
+        eng.close()
+    for c, v in out[0].items():
+        assert np.array_equal(out[1][c], v), c
+        assert np.array_equal(out[2][c], v), c
+    assert any(np.abs(v).max() > 0 for v in out[0].values())
