@@ -27,6 +27,7 @@
 
 #include "../../include/yee.h"
 #include "yee_kernels.h"
+#include "yee_plane.h"
 #include "yee_readback.h"
 #include "yee_setup.h"
 
@@ -38,7 +39,7 @@ template <typename T>
 __global__ void batch_tmz_step2 (const StepArgs<T> *, const int4 *, int, const int *, const T *, int);
 template <typename T>
 __global__ void batch_tmz_sources (const StepArgs<T> *, int, const int *, const T *, int);
-__global__ void batch_advance (int *, const int *, int, int);
+__global__ void batch_advance (int *, const int *, int, int, int);
 
 int batch_fail (int code, const std::string &msg);
 
@@ -53,6 +54,8 @@ struct BatchGroup
   int *list = nullptr;                  // the same indices in device memory (batch_advance)
   int4 *tiles[2][4] = {};               // [two-step][length] tile tables (kLx[0..3] x rows)
   int ntiles[2][4] = {};
+  int4 *plane = nullptr;                // tiles of batch_plane_steps
+  int nplane = 0;
   hipGraphExec_t graph = nullptr;
 };
 
@@ -67,7 +70,7 @@ struct yee_batch
   std::vector<void *> mat;              // [sim][2] eps, mu grids (nullptr: uniform)
   std::vector<void *> grids;            // every device allocation of the batch
   std::vector<void *> f[2], d[2];       // [parity][sim][3] Ez, Hx, Hy and Dz, Bx, By
-  std::vector<void *> pml;              // [sim] PML tables
+  std::vector<void *> pml, pfac;        // [sim] PML tables, D/B -> field factors
   std::vector<int> tab_len;
   int device = 0;                       // the device current at yee_batch_create
   hipStream_t stream = nullptr;
@@ -188,6 +191,7 @@ StepArgs<T> sim_args (const yee_batch *b, int s, int parity)
   a.mu0 = (T) mu0 ();
   a.pml = (const T *) b->pml[s];
   a.tab_len = b->tab_len[s];
+  for (int k = 0; k < 3 && b->pfac[s]; ++k) a.pfac[YEE_EZ + k] = (const T *) b->pfac[s] + 2 * k * c.size[0] * c.size[1];
   a.tfsf = 0;
   const int64_t *p = c.point_source_pos;
   a.src_mask = c.point_source & ((1u << YEE_EZ) | (1u << YEE_HX) | (1u << YEE_HY));
@@ -255,12 +259,13 @@ void launch_step (yee_batch *b, const BatchGroup &g, int two, int sel)
                        b->state, (const T *) b->src_tab, b->src_len);
 }
 
-void launch_advance (yee_batch *b, const int *list, int n, int k)
+void launch_advance (yee_batch *b, const int *list, int n, int k, int flip)
 {
-  hipLaunchKernelGGL (batch_advance, dim3 ((unsigned) ((n + 63) / 64)), dim3 (64), 0, b->stream, b->state, list, n, k);
+  hipLaunchKernelGGL (batch_advance, dim3 ((unsigned) ((n + 63) / 64)), dim3 (64), 0, b->stream, b->state, list, n, k, flip);
 }
 
-// Candidates of the tuner: (grouping, steps per launch, tile length index).
+// Candidates of the tuner: grouping, kind of launch (0: one step, 1: two, 2: BATCH_STEPS on register
+// tiles), tile length index.
 struct Cand
 {
   int grouping, two, sel;
@@ -269,26 +274,49 @@ struct Cand
 constexpr double kBudgetMiB[] = { 0, 160, 64 };
 constexpr int kNumGroupings = (int) (sizeof kBudgetMiB / sizeof kBudgetMiB[0]);
 const Cand kCands[] = { { 0, 0, 0 }, { 0, 0, 1 }, { 0, 0, 2 }, { 0, 1, 0 }, { 0, 1, 1 }, { 0, 1, 2 },
-                        { 0, 1, 3 }, { 1, 1, 1 }, { 1, 1, 2 }, { 2, 1, 0 }, { 2, 1, 1 }, { 2, 1, 2 } };
+                        { 0, 1, 3 }, { 1, 1, 1 }, { 1, 1, 2 }, { 2, 1, 0 }, { 2, 1, 1 }, { 2, 1, 2 }, { 0, 2, 2 } };
 constexpr int kNumCands = (int) (sizeof kCands / sizeof kCands[0]);
+constexpr int kPlaneCand = kNumCands - 1;
 constexpr int kTuneSteps = 4;
+constexpr int kTuneTotal = (kNumCands - 1) * kTuneSteps + 8;   // the register tiles take 8
 constexpr int kGraphSteps = 16;
+constexpr int kPlaneRun = 64;   // steps of the register tiles between two batch_advance
+static_assert (kBatchRows == kLx[2], "the rows reported for the register tiles");
 
-// `k` steps (1, or 2 with a two-step candidate) of group g with candidate c's tiles.
+// Steps per launch of a candidate.
+int cand_stride (const yee_batch *b, const Cand &c)
+{
+  return c.two == 2 ? (b->wsize == 4 ? BATCH_STEPS (float) : BATCH_STEPS (double)) : (c.two ? 2 : 1);
+}
+
+// A mu grid rules out the two-step kernel.
+bool cand_ok (const yee_batch *b, const Cand &c)
+{
+  return c.two != 1 || b->two_ok;
+}
+
+// `k` steps of group g with candidate c's tiles: one launch where k is at most the candidate's
+// stride (a two-step candidate takes 1 or 2), with the step counters moved on after it; or, for the
+// register tiles, several launches that count from the group's counters, moved on once at the end.
 template <typename T>
 int enqueue_steps (yee_batch *b, const BatchGroup &g, const Cand &c, int k)
 {
-  const int two = (c.two && k == 2) ? 1 : 0;
-  launch_step<T> (b, g, two, c.sel);
-  launch_advance (b, g.list, (int) g.sims.size (), two ? 2 : 1);
+  if (c.two == 2)
+  {
+    int launches = 0;
+    for (int s = 0; s < k; s += BATCH_STEPS (T), ++launches)
+      launch_batch_plane<T> ((const StepArgs<T> *) b->sims, g.plane, g.nplane, b->state, (const T *) b->src_tab, b->src_len, s,
+                             launches & 1, std::min (BATCH_STEPS (T), k - s), b->stream);
+    launch_advance (b, g.list, (int) g.sims.size (), k, launches & 1);
+  }
+  else
+  {
+    const int two = (c.two && k == 2) ? 1 : 0;
+    launch_step<T> (b, g, two, c.sel);
+    launch_advance (b, g.list, (int) g.sims.size (), two ? 2 : 1, 1);
+  }
   BHIP (hipGetLastError ());
   return YEE_OK;
-}
-
-// Steps per launch of a candidate.
-int cand_stride (const Cand &c)
-{
-  return c.two ? 2 : 1;
 }
 
 template <typename T>
@@ -302,7 +330,7 @@ int build_graph (yee_batch *b, BatchGroup &grp, const Cand &c)
   hipGraph_t g = nullptr;
   BHIP (hipStreamBeginCapture (b->stream, hipStreamCaptureModeThreadLocal));
   int rc = YEE_OK;
-  for (int s = 0; s < kGraphSteps && rc == YEE_OK; s += cand_stride (c)) rc = enqueue_steps<T> (b, grp, c, cand_stride (c));
+  for (int s = 0; s < kGraphSteps && rc == YEE_OK; s += cand_stride (b, c)) rc = enqueue_steps<T> (b, grp, c, cand_stride (b, c));
   hipError_t e = hipStreamEndCapture (b->stream, &g);
   if (rc) return rc;
   if (e != hipSuccess) return batch_fail (YEE_EDEVICE, std::string ("hipStreamEndCapture: ") + hipGetErrorString (e));
@@ -326,7 +354,7 @@ int step_impl (yee_batch *b, int32_t n)
   {
     hipLaunchKernelGGL ((batch_tmz_sources<T>), dim3 ((unsigned) ((b->nsim + 63) / 64)), dim3 (64), 0, b->stream,
                        (const StepArgs<T> *) b->sims, b->nsim, b->state, (const T *) b->src_tab, b->src_len);
-    launch_advance (b, b->all, b->nsim, 1);
+    launch_advance (b, b->all, b->nsim, 1, 1);
     BHIP (hipGetLastError ());
     ++done;
     ++b->t;
@@ -335,14 +363,14 @@ int step_impl (yee_batch *b, int32_t n)
   if (const char *fc = std::getenv ("YEE_BATCH_CAND"))
   {
     const int ci = std::atoi (fc);
-    if (ci < 0 || ci >= kNumCands || (kCands[ci].two && !b->two_ok)) return batch_fail (YEE_EINVAL, "YEE_BATCH_CAND out of range");
+    if (ci < 0 || ci >= kNumCands || !cand_ok (b, kCands[ci])) return batch_fail (YEE_EINVAL, "YEE_BATCH_CAND out of range");
     if (b->cand != ci) rc = drop_graphs (b);
     if (rc) return rc;
     b->cand = ci;
   }
   // tuner: kTuneSteps ordinary steps of every simulation per candidate, timed, on the first
   // call that has room
-  if (b->cand < 0 && n - done >= kNumCands * kTuneSteps)
+  if (b->cand < 0 && n - done >= kTuneTotal)
   {
     b->tune_ms.assign (kNumCands, 0.0);
     hipEvent_t e0, e1;
@@ -351,36 +379,38 @@ int step_impl (yee_batch *b, int32_t n)
     double best = 1e30;
     for (int c = 0; c < kNumCands; ++c)
     {
-      if (kCands[c].two && !b->two_ok)
+      if (!cand_ok (b, kCands[c]))
       {
         b->tune_ms[c] = 0;
         continue;
       }
       BHIP (hipEventRecord (e0, b->stream));
-      const int stride = cand_stride (kCands[c]);
+      const int steps = c == kPlaneCand ? kTuneTotal - c * kTuneSteps : kTuneSteps;
+      const int stride = c == kPlaneCand ? steps : cand_stride (b, kCands[c]);
       for (const BatchGroup &g : b->groupings[kCands[c].grouping])
-        for (int s = 0; s < kTuneSteps; s += stride)
+        for (int s = 0; s < steps; s += stride)
           if ((rc = enqueue_steps<T> (b, g, kCands[c], stride))) return rc;
       BHIP (hipEventRecord (e1, b->stream));
       BHIP (hipEventSynchronize (e1));
       float ms = 0;
       BHIP (hipEventElapsedTime (&ms, e0, e1));
-      b->tune_ms[c] = ms / kTuneSteps;
-      if (ms < best)
+      b->tune_ms[c] = ms / steps;
+      if (b->tune_ms[c] < best)
       {
-        best = ms;
+        best = b->tune_ms[c];
         b->cand = c;
       }
-      done += kTuneSteps;
-      b->t += kTuneSteps;
+      done += steps;
+      b->t += steps;
     }
     (void) hipEventDestroy (e0);
     (void) hipEventDestroy (e1);
   }
-  if (b->cand < 0) b->cand = 2;   // too few steps to tune: one group, 64-row tiles
+  if (b->cand < 0) b->cand = kPlaneCand;   // too few steps to tune
   const Cand &c = kCands[b->cand];
   const char *use_graph = std::getenv ("YEE_BATCH_GRAPH");
-  const bool graphs = !(use_graph && std::strcmp (use_graph, "0") == 0);
+  // (a launch of the register tiles covers enough steps by itself)
+  const bool graphs = !(use_graph && std::strcmp (use_graph, "0") == 0) && c.two != 2;
   // each group runs all the remaining steps before the next one starts
   const int32_t left = n - done;
   for (BatchGroup &g : b->groupings[c.grouping])
@@ -396,7 +426,8 @@ int step_impl (yee_batch *b, int32_t n)
       }
       else
       {
-        const int kk = std::min (cand_stride (c), left - k);
+        // (the register tiles' launches share one advance)
+        const int kk = std::min (c.two == 2 ? kPlaneRun : cand_stride (b, c), left - k);
         if ((rc = enqueue_steps<T> (b, g, c, kk))) return rc;
         k += kk;
       }
@@ -445,6 +476,12 @@ int prepare_impl (yee_batch *b)
       BHIP (hipMemcpyAsync (p, tv.data (), tv.size () * sizeof (T), hipMemcpyHostToDevice, b->stream));
       BHIP (hipStreamSynchronize (b->stream));
       b->pml[s] = p;
+      // the D/B -> field factors of the register tiles' PML cells (pairs for Ez, Hx, Hy)
+      BHIP (hipMalloc (&p, 6 * (size_t) (c.size[0] * c.size[1]) * sizeof (T)));
+      b->grids.push_back (p);
+      b->pfac[s] = p;
+      launch_plane_factors<T> (YEE_SCHEME_TMZ, sim_args<T> (b, s, 0), b->stream);
+      BHIP (hipGetLastError ());
     }
     args[2 * s] = sim_args<T> (b, s, 0);
     args[2 * s + 1] = sim_args<T> (b, s, 1);
@@ -501,6 +538,18 @@ int prepare_impl (yee_batch *b)
           BHIP (hipMemcpyAsync (p, tv.data (), tv.size () * sizeof (int4), hipMemcpyHostToDevice, b->stream));
           g.tiles[two][sel] = (int4 *) p;
         }
+      std::vector<int4> tv;
+      for (int s : g.sims)
+      {
+        const yee_config &c = b->cfg[s];
+        for (int64_t x0 = 1; x0 < c.size[0] - 1; x0 += kBatchRows)
+          for (int64_t y0 = 1; y0 < c.size[1] - 1; y0 += 64 - 2 * BATCH_STEPS (T))
+            tv.push_back (make_int4 (s, (int) x0, (int) y0, 0));
+      }
+      g.nplane = (int) tv.size ();
+      if ((rc = alloc_zero (b, &p, std::max<size_t> (1, tv.size ()) * sizeof (int4)))) return rc;
+      BHIP (hipMemcpyAsync (p, tv.data (), tv.size () * sizeof (int4), hipMemcpyHostToDevice, b->stream));
+      g.plane = (int4 *) p;
     }
   }
   {
@@ -580,6 +629,7 @@ int yee_batch_create (const yee_config *cfgs, int32_t nsim, yee_batch **out)
     b->d[par].assign (3 * (size_t) nsim, nullptr);
   }
   b->pml.assign (nsim, nullptr);
+  b->pfac.assign (nsim, nullptr);
   b->tab_len.assign (nsim, 0);
   auto bail = [&] (int code) {
     yee_batch_destroy (b);
@@ -698,7 +748,7 @@ int yee_batch_tuning (yee_batch *b, int32_t out[3], double *cand_ms, int32_t nca
     const Cand &c = kCands[b->cand];
     const std::vector<BatchGroup> &gs = b->groupings[c.grouping];
     out[0] = kLx[c.sel];
-    out[1] = gs.empty () ? 0 : (gs[0].ntiles[c.two][c.sel] + 3) / 4;
+    out[1] = gs.empty () ? 0 : (c.two == 2 ? gs[0].nplane : (gs[0].ntiles[c.two][c.sel] + 3) / 4);
     out[2] = (int32_t) gs.size ();
   }
   else

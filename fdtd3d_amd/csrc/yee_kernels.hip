@@ -1676,15 +1676,14 @@ __global__ void batch_tmz_sources (const StepArgs<T> *sims, int nsim, const int 
 }
 
 // After a launch that advanced simulations sims[0..n) by k steps (the last node of every
-// captured step): their step counters move on by k and their newest fields are now in the
-// other buffer.
-__global__ void batch_advance (int *state, const int *sims, int n, int k)
+// captured step): their step counters move on by k and their newest fields are `flip` buffers on.
+__global__ void batch_advance (int *state, const int *sims, int n, int k, int flip)
 {
   const int u = (int) (blockIdx.x * blockDim.x + threadIdx.x);
   if (u < n)
   {
     state[2 * sims[u]] += k;
-    state[2 * sims[u] + 1] ^= 1;
+    state[2 * sims[u] + 1] ^= flip;
   }
 }
 

@@ -57,6 +57,22 @@ struct PlaneSource
 template <typename T>
 void launch_plane_factors (int scheme, const StepArgs<T> &a, hipStream_t stream);
 
+// Tiles of a batched TMz sweep: 40 owned rows; the steps of a launch (the margin), the waves of a tile
+// and the rows of a wave.  FP32: 8 waves of 7 rows (118 registers, two tiles a compute unit): 64
+// simulations of 5.7e7 cells take 196 us a step, 242 with 14 waves of 4 rows (one tile a unit), 214
+// with 12 of 4 and a margin of 4, 268 with 8 of 6 and a margin of 4.  FP64: 16 of 3 with a margin of
+// 4, half the steps for less margin, which its lower tiles make dearer.
+constexpr int kBatchRows = 40;
+#define BATCH_STEPS(T) (sizeof (T) == 4 ? 8 : 4)
+#define BATCH_WAVES(T) (sizeof (T) == 4 ? 8 : 16)
+#define BATCH_RW(T) (sizeof (T) == 4 ? 7 : 3)
+
+// n <= BATCH_STEPS steps of the simulations of a tile table (sim, x0, y0, -): from the step and buffer
+// in state[sim], `off` steps and `flip` buffers on.
+template <typename T>
+void launch_batch_plane (const StepArgs<T> *sims, const int4 *tiles, int ntiles, const int *state, const T *src_tab,
+                         int src_len, int off, int flip, int n, hipStream_t stream);
+
 // Value of the hard source in every half step of a launch of a 1D run.
 struct LineSource
 {

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from fdtd3d_amd.config import parse_args
-from fdtd3d_amd.engine import Engine
+from fdtd3d_amd.engine import Batch, Engine
 
 pytestmark = pytest.mark.gpu
 
@@ -182,3 +182,41 @@ def test_line_steps_in_one_launch(scheme, n, pml, tfsf, right, source, precision
         assert np.array_equal(out[1][c], v), c
         assert np.array_equal(out[2][c], v), c
     assert any(np.abs(v).max() > 0 for v in out[0].values())
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("shapes,mu", [(((42, 50), (43, 98), (3, 64), (121, 57)), False), (((81, 49), (30, 33)), True)])
+def test_batch_register_tiles(shapes, mu, precision, engine_lib, monkeypatch):
+    """The batch's register tiles (40 x 48 owned cells in FP32, 40 x 56 in FP64) against single runs,
+    bit for bit: edges of tiles, a mu grid, calls that are no multiple of a launch's steps."""
+    sims = [f"--2d-tmz --size x:{a},y:{b} --point-source x:{a // 2},y:{b // 2} --point-source-ez --point-source-hy "
+            + ("--use-pml --pml-size x:4,y:5 " if min(a, b) > 20 and k != 1 else "--pml-size x:0,y:0 ")
+            + "--time-steps 80"
+            for k, (a, b) in enumerate(shapes)]
+    cfgs = [parse_args(s.split(), precision=precision) for s in sims]
+    rng = np.random.default_rng(17)
+    eps = [rng.uniform(1.0, 5.0, size=c.shape) for c in cfgs]
+    mus = [rng.uniform(1.0, 2.0, size=c.shape) for c in cfgs]
+    monkeypatch.setenv("YEE_BATCH_CAND", "12")
+    b = Batch(cfgs)
+    for s, c in enumerate(cfgs):
+        b.set_material(s, "eps", eps[s])
+        if mu:
+            b.set_material(s, "mu", mus[s])
+        b.set_point_source_gaussian(s, 30.0, 10.0)
+    b.prepare()
+    for n in (1, 3, 64, 5, 7):
+        b.step(n)
+    monkeypatch.setenv("YEE_KERNEL", "split")
+    for s, c in enumerate(cfgs):
+        e = Engine(c)
+        e.set_material("eps", eps[s])
+        if mu:
+            e.set_material("mu", mus[s])
+        e.set_point_source_gaussian(30.0, 10.0)
+        e.prepare()
+        e.step(80)
+        for f in ("Ez", "Hx", "Hy") + (("Dz", "Bx", "By") if c.use_pml else ()):
+            assert np.array_equal(b.field(s, f), e.field(f)), f"sim {s} {f}"
+        e.close()
+    b.close()
