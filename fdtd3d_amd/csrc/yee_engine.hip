@@ -1325,12 +1325,17 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     // x chunks: a CU holds 16 waves of this kernel (<= 128 VGPRs each), i.e. 16 / (waves per
     // row) workgroups.  The chunk count minimises rounds of resident workgroups x planes per
     // chunk (+1 for the chunk's first plane, read twice): enough workgroups to fill every CU,
-    // and no last round left mostly empty.
+    // and no last round left mostly empty.  Rows of five waves put two on one SIMD, and a third
+    // workgroup (15 of the 16 waves) measures as not resident: counted as two a CU, with a fifth
+    // added for more than one round, 251x187x301 FP32 takes 157 us of 192 (6 chunks of 9),
+    // 320^3 392 of 450 (3 of 5), 220x260x300 193 of 230 (4 of 13) and FP64 458 of 512 (2 of 13).
+    // (Other row lengths gain nothing from either: 256^3 FP64 400 us, 412 with one round.)
     const int64_t waves = (h->n[2] + 63) / 64;
-    const int64_t slots = (int64_t) h->ncu * std::max<int64_t> (1, 16 / waves);
+    const bool five = waves == 5;
+    const int64_t slots = (int64_t) h->ncu * (five ? 2 : std::max<int64_t> (1, 16 / waves));
     auto chunk_cost = [&] (int64_t c) {
       const int64_t rounds = (h->fused_nstrips * c + slots - 1) / slots;
-      return (double) rounds * (double) ((planes + c - 1) / c + 1);
+      return (five && rounds > 1 ? 1.2 : 1.0) * (double) rounds * (double) ((planes + c - 1) / c + 1);
     };
     double best = 1e300;
     for (int64_t c = 1; c <= planes; ++c) best = std::min (best, chunk_cost (c));

@@ -803,13 +803,16 @@ template <typename T, int BY, int MAT>
 __device__ __forceinline__ void fused_plane (const StepArgs<T> &a, const FusedPos &g, const uint32_t (&ro)[BY + 2],
                                              int x, int xend, int PAR, int lane, int wave, int nw, FusedLds<T, BY> &s,
                                              const Carry<T, BY> &c, const PlaneLoads<T, BY> &L, Carry<T, BY> &o,
-                                             PlaneLoads<T, BY> &nxt)
+                                             PlaneLoads<T, BY> &nxt, double &zc)
 {
   constexpr int kZStage = 2 * 3 * (BY + 1) * 4;   // z-face table entries per parity
   const int i = x - 1;                            // H plane
   e_load<T, BY, MAT> (a, min (x + 1, xend), g, ro, nxt);   // prefetch the next plane
-  // z-face corrections of the next plane (written to LDS before the barrier)
-  const double zpre = zstage_load<T, BY> (a, g.k, min (x + 1, xend), g.j0);
+  // z-face corrections of the plane after the next; those of the next (zc) were loaded an iteration
+  // ago and go to LDS before the barrier.  (Loaded here and stored there in one iteration, they made
+  // every plane wait for all the loads prefetched before them: the sweep of 512^3 FP32 took 1431 us so and
+  // takes 1250-1320 us, 256^3 199 and 182 us.)
+  const double zpre = zstage_load<T, BY> (a, g.k, min (x + 2, xend), g.j0);
   // z+1 neighbours from the next lane (DPP shift); lane 63 takes lane 0 of the next wave,
   // which that wave left in LDS before the last barrier
   const bool edge = lane == 63 && wave + 1 < nw;
@@ -904,7 +907,8 @@ __device__ __forceinline__ void fused_plane (const StepArgs<T> &a, const FusedPo
   }
   if (a.tfsf)
   {
-    if (g.k < kZStage) (&s.zl[PAR ^ 1][0][0][0][0])[g.k] = zpre;
+    if (g.k < kZStage) (&s.zl[PAR ^ 1][0][0][0][0])[g.k] = zc;
+    zc = zpre;
     // a 64-thread block (short z rows) loads the entries past its width here
     for (int t = g.k + (int) blockDim.x; t < kZStage; t += (int) blockDim.x)
       (&s.zl[PAR ^ 1][0][0][0][0])[t] = zstage_load<T, BY> (a, t, min (x + 1, xend), g.j0);
@@ -1020,14 +1024,15 @@ __global__ __launch_bounds__ (64 * MAXW) void step_3d_fused (StepArgs<T> a)
     __syncthreads ();
   }
 
+  double zc = zstage_load<T, BY> (a, g.k, min (xa + 2, xend), g.j0);   // of plane xa + 2
   if (sizeof (T) == 4 || MAXW <= 12)
   {
     // unrolled by two planes: the two copies of the state swap roles without register copies
     for (int x = xa + 1; x <= xend; x += 2)
     {
-      fused_plane<T, BY, MAT> (a, g, ro, x, xend, 1, lane, wave, nw, s, c0, p0, c1, p1);
+      fused_plane<T, BY, MAT> (a, g, ro, x, xend, 1, lane, wave, nw, s, c0, p0, c1, p1, zc);
       if (x + 1 > xend) break;
-      fused_plane<T, BY, MAT> (a, g, ro, x + 1, xend, 0, lane, wave, nw, s, c1, p1, c0, p0);
+      fused_plane<T, BY, MAT> (a, g, ro, x + 1, xend, 0, lane, wave, nw, s, c1, p1, c0, p0, zc);
     }
   }
   else
@@ -1037,7 +1042,7 @@ __global__ __launch_bounds__ (64 * MAXW) void step_3d_fused (StepArgs<T> a)
     int par = 1;
     for (int x = xa + 1; x <= xend; ++x, par ^= 1)
     {
-      fused_plane<T, BY, MAT> (a, g, ro, x, xend, par, lane, wave, nw, s, c0, p0, c1, p1);
+      fused_plane<T, BY, MAT> (a, g, ro, x, xend, par, lane, wave, nw, s, c0, p0, c1, p1, zc);
       c0 = c1;
       p0 = p1;
     }
