@@ -1293,11 +1293,19 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   if (hipEventCreate (&h->ev[0]) != hipSuccess || hipEventCreate (&h->ev[1]) != hipSuccess)
     return bail (fail (YEE_EDEVICE, "hipEventCreate failed"));
   // 3D runs use the fused step kernel on the PML-free box outside the Drude box (double-
-  // buffered state) when the doubled state fits in HBM; TMz runs update in place with the
-  // half-step kernels.  YEE_KERNEL=split in the environment selects the half-step kernels for 3D
-  // as well (A/B checks).
+  // buffered state) when the doubled state fits in HBM and E and H are too large for the 256 MB
+  // last-level cache.  Smaller grids take one half-step launch over the whole grid for E and one for
+  // H, in place: their second pass over E and H is served by that cache, and every cell has a thread
+  // of its own, while the sweep has few workgroups that march along x one plane after the other.
+  // us a step, sweep and half steps, with PML and TF/SF: FP32 48^3 36 and 13, 96^3 67 and 37, 160^3
+  // 152 and 105, 192^3 223 and 181, 208^3 255 and 255, 320^3 730 and 742; FP64 96^3 64 and 55, 160^3
+  // 233 and 225, 176^3 289 and 293, 256^3 705 and 816.  Without them: FP32 192^3 150 and 85, 256^3
+  // 241 and 266; FP64 128^3 71 and 55, 192^3 215 and 220.  Drude box: FP32 192^3 367 and 325, FP64
+  // 128^3 218 and 214, 192^3 576 and 687.  The line lies at 200 MB of E and H (202^3 FP32, 160^3 FP64).
+  // YEE_KERNEL=split or fused in the environment selects one of the two (A/B checks).
   const char *kern = std::getenv ("YEE_KERNEL");
   const bool want_fused = !(kern && std::strcmp (kern, "split") == 0);
+  const bool force_fused = kern && std::strcmp (kern, "fused") == 0;
   h->fused = false;
   // (double material precision keeps the half-step kernels: they read per-component averages)
   // (the fused kernel is E_CENTERED: H_CENTERED runs take the half-step kernels)
@@ -1315,7 +1323,8 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     // metamaterials (24)
     const int arrays = 12 + (h->mode == 1 ? 6 : 0) + (h->mode == 2 ? 48 : 0);
     const double bytes = (double) arrays * (double) h->ncell * (double) h->wsize;
-    h->fused = ok && bytes < 200e9;
+    const bool cached = 6.0 * (double) h->ncell * (double) h->wsize <= 200e6;
+    h->fused = ok && bytes < 200e9 && (force_fused || !cached);
   }
   if (h->fused)
   {

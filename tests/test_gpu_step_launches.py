@@ -220,3 +220,19 @@ def test_batch_register_tiles(shapes, mu, precision, engine_lib, monkeypatch):
             assert np.array_equal(b.field(s, f), e.field(f)), f"sim {s} {f}"
         e.close()
     b.close()
+
+
+@pytest.mark.parametrize("precision,y", [(4, 128), (8, 64)])
+@pytest.mark.parametrize("z", [1017, 1018])
+def test_sweep_and_half_steps_meet(z, y, precision, engine_lib, monkeypatch):
+    """Grids whose E and H fill at most 200 MB run by whole-grid half steps, larger ones by the
+    fused sweep: the fields on both sides of that line are those of the sweep."""
+    args = f"--3d --size x:64,y:{y},z:{z} --use-pml --pml-size x:5,y:5,z:5 --use-tfsf --tfsf-size-left x:9,y:9,z:9 " \
+           "--tfsf-size-right x:9,y:9,z:9 --angle-teta 30 --angle-phi 45 --angle-psi 90 --time-steps 8"
+    print(f"[gpu] line between sweep and half steps, z {z}, precision {precision}", flush=True)
+    eps = np.kron(np.random.default_rng(4).uniform(1.0, 4.0, size=(8, y // 8, 128)), np.ones((8, 8, 8)))[:, :, :z]
+    ref = _run(args, precision, monkeypatch, "fused", eps, 8)
+    got = _run(args, precision, monkeypatch, "", eps, 8)
+    for n, v in ref.items():
+        assert np.array_equal(got[n], v), n
+    assert np.abs(ref["Ez"]).max() > 0
