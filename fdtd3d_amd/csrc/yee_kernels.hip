@@ -188,6 +188,32 @@ __device__ __forceinline__ void load_old (const StepArgs<T> &a, int64_t q, const
   }
 }
 
+// The cells of a material grid that the three components of a cell average, and the averages: over
+// two cells along each axis, or over the four around each axis (OP: avg4 or sum4).
+template <typename T>
+__device__ __forceinline__ void axis_load (const T *m, int64_t sx, int sy, int sz, T (&v)[7])
+{
+  v[0] = gld (m); v[1] = gld (m + sx); v[2] = gld (m + sy); v[3] = gld (m + sz);
+}
+
+template <typename T>
+__device__ __forceinline__ void cross_load (const T *m, int64_t sx, int sy, int sz, T (&v)[7])
+{
+  axis_load (m, sx, sy, sz, v);
+  v[4] = gld (m + sy + sz); v[5] = gld (m + sx + sz); v[6] = gld (m + sx + sy);
+}
+
+template <typename T>
+__device__ __forceinline__ void axis_avgs (const T (&v)[7], T &x, T &y, T &z)
+{
+  x = avg2 (v[0], v[1]); y = avg2 (v[0], v[2]); z = avg2 (v[0], v[3]);
+}
+
+template <auto OP, typename T>
+__device__ __forceinline__ void cross_avgs (const T (&v)[7], T &x, T &y, T &z)
+{
+  x = OP (v[0], v[3], v[2], v[4]); y = OP (v[0], v[3], v[1], v[5]); z = OP (v[0], v[2], v[1], v[6]);
+}
 
 // ---------------------------------------------------------------------------------------
 // 3D E half-step: Ex, Ey, Ez on the run box (all of [1, N-1)^3, or one PML slab when the
@@ -211,6 +237,28 @@ __device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, uint32_t fl, 
   load_old<T, MODE, 0> (a, q, p, special, fo0, do0, pc0);
   load_old<T, MODE, 1> (a, q, p, special, fo1, do1, pc1);
   load_old<T, MODE, 2> (a, q, p, special, fo2, do2, pc2);
+  // Every load of the cell before the first use of one: a material loaded after the curl, then each
+  // Drude parameter, waited for memory once more each (E boxes and half steps: drude 256^3 FP32 283 us
+  // so, 265 now; 512^3 569 and 554; 192^3 with PML 99 and 95, without 48 and 46).  H keeps its order:
+  // the 7 values of mu are more registers than 8 waves a SIMD leave, and it became 1 to 3 % slower.
+  T em[7], om[7], gm[7];
+  if (a.matc[0])
+  {
+    // double material precision: the 8-cell averages, precomputed per component
+    em[0] = gld (a.matc[0] + q);
+    em[1] = gld (a.matc[1] + q);
+    em[2] = gld (a.matc[2] + q);
+  }
+  else if (a.eps)
+  {
+    if constexpr (LAY == 0) axis_load (a.eps + q, sx, sy, sz, em);
+    else cross_load (a.eps + q, sx, sy, sz, em);
+  }
+  if (MODE == 2 && special)
+  {
+    if (a.ope) axis_load (a.ope + q, sx, sy, sz, om);
+    if (a.ge) axis_load (a.ge + q, sx, sy, sz, gm);
+  }
   const T *Hx = a.f[3], *Hy = a.f[4], *Hz = a.f[5];
   const T hx = gld (Hx + q), hy = gld (Hy + q), hz = gld (Hz + q);
   // E_CENTERED: H at {-1, 0} along the derivative axis; H_CENTERED: at {0, +1}
@@ -227,55 +275,31 @@ __device__ __forceinline__ void e_half_cell (const StepArgs<T> &a, uint32_t fl, 
     vy[0] = hx; vy[1] = gld (Hx + q + sz); vy[2] = hz; vy[3] = gld (Hz + q + sx);
     vz[0] = hy; vz[1] = gld (Hy + q + sx); vz[2] = hx; vz[3] = gld (Hx + q + sy);
   }
-  T ex_m = a.eps_u, ey_m = a.eps_u, ez_m = a.eps_u;
-  if (a.matc[0])
-  {
-    // double material precision: the 8-cell averages, precomputed per component
-    ex_m = gld (a.matc[0] + q);
-    ey_m = gld (a.matc[1] + q);
-    ez_m = gld (a.matc[2] + q);
-  }
-  else if (a.eps)
-  {
-    const T *m = a.eps;
-    if constexpr (LAY == 0)
-    {
-      // 2-cell averages along each component's axis (getMaterial, E_CENTERED)
-      const T e = gld (m + q);
-      ex_m = avg2 (e, gld (m + q + sx));
-      ey_m = avg2 (e, gld (m + q + sy));
-      ez_m = avg2 (e, gld (m + q + sz));
-    }
-    else
-    {
-      // 4-cell transverse averages (getMaterial, H_CENTERED, E components)
-      ex_m = avg4 (gld (m + q), gld (m + q + sz), gld (m + q + sy), gld (m + q + sy + sz));
-      ey_m = avg4 (gld (m + q), gld (m + q + sz), gld (m + q + sx), gld (m + q + sx + sz));
-      ez_m = avg4 (gld (m + q), gld (m + q + sy), gld (m + q + sx), gld (m + q + sx + sy));
-    }
-  }
   if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 3> (a, i, j, k))
   {
     tfsf_apply<T, 0, 3, LAY> (a, i, j, k, vx);
     tfsf_apply<T, 1, 3, LAY> (a, i, j, k, vy);
     tfsf_apply<T, 2, 3, LAY> (a, i, j, k, vz);
   }
+  T ex_m = a.eps_u, ey_m = a.eps_u, ez_m = a.eps_u;
+  if (a.matc[0])
+  {
+    ex_m = em[0];
+    ey_m = em[1];
+    ez_m = em[2];
+  }
+  else if (a.eps)
+  {
+    // 2-cell averages along each component's axis (getMaterial, E_CENTERED) or 4-cell transverse ones
+    if constexpr (LAY == 0) axis_avgs (em, ex_m, ey_m, ez_m);
+    else cross_avgs<avg4<T>> (em, ex_m, ey_m, ez_m);
+  }
   T oxm = 0, oym = 0, ozm = 0, gxm = 0, gym = 0, gzm = 0;
   if (MODE == 2 && special)
   {
     // Drude 2-cell averages (getMetaMaterial / approximateDrudeModel)
-    if (a.ope)
-    {
-      const T *o = a.ope;
-      oxm = avg2 (gld (o + q), gld (o + q + sx)); oym = avg2 (gld (o + q), gld (o + q + sy));
-      ozm = avg2 (gld (o + q), gld (o + q + sz));
-    }
-    if (a.ge)
-    {
-      const T *g = a.ge;
-      gxm = avg2 (gld (g + q), gld (g + q + sx)); gym = avg2 (gld (g + q), gld (g + q + sy));
-      gzm = avg2 (gld (g + q), gld (g + q + sz));
-    }
+    if (a.ope) axis_avgs (om, oxm, oym, ozm);
+    if (a.ge) axis_avgs (gm, gxm, gym, gzm);
   }
   update_cell<T, MODE, 0> (a, fl, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm, pc0);
   update_cell<T, MODE, 1> (a, fl, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym, pc1);
@@ -387,8 +411,10 @@ __global__ __launch_bounds__ (256) void e_half_3d (StepArgs<T> a)
   else e_half_cell<T, MODE> (a, 0u, i, j, k);
 }
 
+// FP32 H kernels are held to the registers of 8 (Drude: 7) waves a SIMD, which cost them no spills (192^3
+// 90 us without, 88 with; the H boxes of drude 256^3 240 and 231).  E needs 66 and more: it spills at 8.
 template <typename T, int MODE>
-__global__ __launch_bounds__ (256) void h_half_3d (StepArgs<T> a)
+__global__ __launch_bounds__ (256, sizeof (T) == 4 ? (MODE < 2 ? 8 : 7) : 1) void h_half_3d (StepArgs<T> a)
 {
   int i, j, k;
   if (!half_cell (a, i, j, k)) return;
@@ -443,7 +469,7 @@ __global__ __launch_bounds__ (256) void e_boxes (StepArgs<T> a, HalfRows rows, c
 }
 
 template <typename T, int MODE>
-__global__ __launch_bounds__ (256) void h_boxes (StepArgs<T> a, HalfRows rows, const HalfBox *box)
+__global__ __launch_bounds__ (256, sizeof (T) == 4 ? (MODE < 2 ? 8 : 7) : 1) void h_boxes (StepArgs<T> a, HalfRows rows, const HalfBox *box)
 {
   int i, j, k;
   uint32_t fl;
