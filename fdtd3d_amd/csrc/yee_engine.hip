@@ -1350,6 +1350,14 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     for (int64_t c = 1; c <= planes; ++c) best = std::min (best, chunk_cost (c));
     int64_t nch = 1;   // the fewest chunks within 1 % of the best
     while (nch < planes && chunk_cost (nch) > 1.01 * best) ++nch;
+    // FP32 rows of six to eight waves (two workgroups a CU, HBM-bound): short chunks, so that the
+    // workgroups that run together stay on the same planes, unless one round fills the chip.  Sweep of
+    // 384^3 630 us of 657 (11 chunks before), 448^3 970 of 1006 (7), 512^3 1410 of 1457 (2; the same
+    // order on a faster card, 1196 of 1270), 512x300x420 735 of 768; 360^3 545 of 536 (3, which fill it).
+    // Longer rows lose (200x500x640 725 of 660), as do short sweeps (100x400x400 147 of 142).
+    if (h->fp32 () && waves >= 6 && waves <= 8 && planes >= 200
+        && !(h->fused_nstrips * nch <= slots && h->fused_nstrips * nch > slots * 95 / 100))
+      nch = std::max (nch, std::min<int64_t> (32, planes / 10));
     if (const char *e = std::getenv ("YEE_FUSED_CHUNKS")) nch = std::max (1, std::atoi (e));
     nch = std::min (nch, planes);
     h->fused_lx = (int) ((planes + nch - 1) / nch);
