@@ -463,6 +463,21 @@ int prepare_impl (yee_batch *b)
 {
   int rc;
   std::vector<StepArgs<T>> args (2 * (size_t) b->nsim);
+  // the D/B -> field factors of the register tiles' PML cells (pairs for Ez, Hx, Hy), in one allocation
+  std::vector<size_t> pf_at ((size_t) b->nsim);
+  size_t pf_bytes = 0;
+  for (int s = 0; s < b->nsim; ++s)
+  {
+    const yee_config &c = b->cfg[s];
+    pf_at[s] = pf_bytes;
+    if (c.flags & YEE_USE_PML) pf_bytes += (6 * (size_t) (c.size[0] * c.size[1]) * sizeof (T) + 255) / 256 * 256;
+  }
+  void *pf = nullptr;
+  if (pf_bytes)
+  {
+    BHIP (hipMalloc (&pf, pf_bytes));
+    b->grids.push_back (pf);
+  }
   for (int s = 0; s < b->nsim; ++s)
   {
     const yee_config &c = b->cfg[s];
@@ -476,10 +491,7 @@ int prepare_impl (yee_batch *b)
       BHIP (hipMemcpyAsync (p, tv.data (), tv.size () * sizeof (T), hipMemcpyHostToDevice, b->stream));
       BHIP (hipStreamSynchronize (b->stream));
       b->pml[s] = p;
-      // the D/B -> field factors of the register tiles' PML cells (pairs for Ez, Hx, Hy)
-      BHIP (hipMalloc (&p, 6 * (size_t) (c.size[0] * c.size[1]) * sizeof (T)));
-      b->grids.push_back (p);
-      b->pfac[s] = p;
+      b->pfac[s] = (char *) pf + pf_at[s];
       launch_plane_factors<T> (YEE_SCHEME_TMZ, sim_args<T> (b, s, 0), b->stream);
       BHIP (hipGetLastError ());
     }

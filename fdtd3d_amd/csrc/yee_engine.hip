@@ -1385,11 +1385,29 @@ int yee_create (const yee_config *cfg, yee_handle **out)
                && 36.0 * (double) h->ncell * (double) h->wsize < 200e9;
   }
   const int nbuf = h->fused || h->plane ? 2 : 1;
+  // the arrays of a 1D or 2D run in one allocation (each costs about 10 us, and its clearing a launch)
+  char *pool = nullptr;
+  const size_t each = ((size_t) (kPadFront + h->ncell + pad_back (h)) * h->wsize + 255) / 256 * 256;
+  if (h->plane && each <= (size_t) 1 << 26)
+  {
+    const int present = (int) std::count (h->present, h->present + 6, true);
+    void *all = nullptr;
+    rc = alloc_zero (h, &all, (size_t) (present * nbuf * (h->mode >= 1 ? 2 : 1)) * each);
+    if (all) h->grids.push_back (all);
+    if (rc) return bail (rc);
+    pool = (char *) all;
+  }
+  auto state_grid = [&] (void **view) {
+    if (!pool) return alloc_grid (h, view);
+    *view = pool + kPadFront * h->wsize;
+    pool += each;
+    return YEE_OK;
+  };
   for (int bsel = 0; bsel < nbuf; ++bsel)
     for (int c = 0; c < 6; ++c)
     {
       if (!h->present[c]) continue;
-      if ((rc = alloc_grid (h, &h->f[bsel][c]))) return bail (rc);
+      if ((rc = state_grid (&h->f[bsel][c]))) return bail (rc);
       if (bsel == 1 && h->mode == 1 && !h->plane)
       {
         h->d[1][c] = h->d[0][c];
@@ -1398,7 +1416,7 @@ int yee_create (const yee_config *cfg, yee_handle **out)
         h->d1p[1][c] = h->d1p[0][c];
         continue;
       }
-      if (h->mode >= 1 && (rc = alloc_grid (h, &h->d[bsel][c]))) return bail (rc);
+      if (h->mode >= 1 && (rc = state_grid (&h->d[bsel][c]))) return bail (rc);
       if (h->mode == 2)
       {
         if ((rc = alloc_grid (h, &h->dp[bsel][c]))) return bail (rc);
