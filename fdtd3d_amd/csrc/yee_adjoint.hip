@@ -40,7 +40,46 @@ struct AdjArgs
   T *w[6];                    // curl weights of the current reverse step
   uint32_t src_mask;          // hard sources (adjoint dropped at src_q)
   int64_t src_q;
+  const T *mon;               // recorded Ez of the monitor rectangle at this step, [x][y] (null: none)
+  int mx0, my0, mnx, mny, mz;
 };
+
+// Trace box geometry: E cells [lo, lo + n) of the three components, [comp][x][y][z].
+struct TraceBox
+{
+  int lo[3], n[3];
+  __host__ __device__ int64_t cells () const { return (int64_t) n[0] * n[1] * n[2]; }
+  __host__ __device__ int64_t at (int c, int x, int y, int z) const
+  {
+    return ((c * (int64_t) n[0] + (x - lo[0])) * n[1] + (y - lo[1])) * n[2] + (z - lo[2]);
+  }
+};
+
+// Gradient of one reverse step (adj_grad): the design voxels, E on the trace box after and before it.
+template <typename T>
+struct GradArgs
+{
+  TraceBox tb;
+  const T *cur, *prev;        // null: no gradient
+  int lo[3], n[3];
+  double *grad;
+};
+
+// (x, y, z) of element u of a box of n cells (32-bit division where it is enough).
+__device__ __forceinline__ void box_cell (const int n[3], int64_t u, int &x, int &y, int &z)
+{
+  if ((int64_t) n[0] * n[1] * n[2] <= (int64_t) INT32_MAX)
+  {
+    const uint32_t v = (uint32_t) u, r = v / (uint32_t) n[2];
+    z = (int) (v - r * (uint32_t) n[2]);
+    x = (int) (r / (uint32_t) n[1]);
+    y = (int) (r - (uint32_t) x * (uint32_t) n[1]);
+    return;
+  }
+  z = (int) (u % n[2]);
+  y = (int) ((u / n[2]) % n[1]);
+  x = (int) (u / ((int64_t) n[2] * n[1]));
+}
 
 // The adjoint D/B and PML coefficients of a special cell, loaded before any store of the
 // thread (the state pointers may alias as far as the compiler knows), so that every load of a
@@ -94,12 +133,59 @@ __device__ __forceinline__ T adj_cell (const AdjArgs<T> &g, int64_t q, T av, T m
   return w;
 }
 
+// grad(v) += sum over the six E cells whose material average contains voxel v of
+// aE(c) * (-(E'(c) - E(c)) / m(c)) / 2, for design voxel u.
+template <typename T>
+__device__ __forceinline__ void grad_voxel (const AdjArgs<T> &g, const GradArgs<T> &d, int64_t u)
+{
+  if (u >= (int64_t) d.n[0] * d.n[1] * d.n[2]) return;
+  const StepArgs<T> &a = g.a;
+  int vx, vy, vz;
+  box_cell (d.n, u, vx, vy, vz);
+  vx += d.lo[0];
+  vy += d.lo[1];
+  vz += d.lo[2];
+  const int64_t sx = a.sx;
+  const int sy = a.sy;
+  double acc = 0;
+  // (component, cell offset along that component's axis): cells c = v and c = v - e_axis
+#pragma unroll
+  for (int comp = 0; comp < 3; ++comp)
+  {
+#pragma unroll
+    for (int back = 0; back < 2; ++back)
+    {
+      const int cx = vx - (comp == 0 ? back : 0), cy = vy - (comp == 1 ? back : 0), cz = vz - (comp == 2 ? back : 0);
+      const int64_t qc = (int64_t) cx * sx + (int64_t) cy * sy + cz;
+      const int64_t step = comp == 0 ? sx : (comp == 1 ? (int64_t) sy : 1);
+      const T m = avg2 (a.eps[qc], a.eps[qc + step]);
+      const int64_t tix = d.tb.at (comp, cx, cy, cz);
+      const T de = d.cur[tix] - d.prev[tix];
+      acc += (double) g.af[comp][qc] * (-(double) de / (double) m) * 0.5;
+    }
+  }
+  d.grad[u] += acc;
+}
+
+template <typename T>
+__global__ __launch_bounds__ (256) void adj_grad (AdjArgs<T> g, GradArgs<T> d)
+{
+  grad_voxel (g, d, (int64_t) blockIdx.x * 256 + (int) threadIdx.x);
+}
+
 // aH -= curl_H(w_E) of the previous reverse step (the transpose of the E curl that read H;
 // w_E is zero before the first one), then the transpose of this step's H update (H cells of
-// [1, N-1)^3; tiles as half_cell).
+// [1, N-1)^3; tiles as half_cell).  The blocks past the tiles' nblk add the gradient of the reverse
+// step before, which reads aE (this kernel does not touch it): a launch of its own took 5 us of the
+// 59 us of a 128^3 FP32 reverse step, as did one for the monitor's source (now in adj_e).
 template <typename T, int MODE>
-__global__ __launch_bounds__ (256) void adj_h (AdjArgs<T> g)
+__global__ __launch_bounds__ (256) void adj_h (AdjArgs<T> g, GradArgs<T> d, int nblk)
 {
+  if ((int) blockIdx.x >= nblk)
+  {
+    grad_voxel (g, d, (int64_t) ((int) blockIdx.x - nblk) * 256 + (int) (threadIdx.y * 64 + threadIdx.x));
+    return;
+  }
   const StepArgs<T> &a = g.a;
   int i, j, k;
   if (!half_cell (a, i, j, k)) return;
@@ -131,7 +217,8 @@ __global__ __launch_bounds__ (256) void adj_h (AdjArgs<T> g)
   g.w[5][q] = adj_cell<T, 5> (g, q, a5, mz, special, o5);
 }
 
-// aE -= curl_E(w_H), then the transpose of the E update (E cells of [1, N-1)^3).
+// aEz += 2 Ez on the monitor rectangle (interior cells), aE -= curl_E(w_H), then the transpose of the
+// E update (E cells of [1, N-1)^3).
 template <typename T, int MODE>
 __global__ __launch_bounds__ (256) void adj_e (AdjArgs<T> g)
 {
@@ -160,33 +247,14 @@ __global__ __launch_bounds__ (256) void adj_e (AdjArgs<T> g)
   adj_load<T, 0> (g, q, p, special, o0);
   adj_load<T, 1> (g, q, p, special, o1);
   adj_load<T, 2> (g, q, p, special, o2);
-  const T a0 = g.af[0][q] - curl (vx), a1 = g.af[1][q] - curl (vy), a2 = g.af[2][q] - curl (vz);
+  T az = g.af[2][q];
+  const int mi = i - g.mx0, mj = j - g.my0;
+  if (g.mon && k == g.mz && mi >= 0 && mi < g.mnx && mj >= 0 && mj < g.mny) az += (T) 2 * g.mon[mi * g.mny + mj];
+  const T a0 = g.af[0][q] - curl (vx), a1 = g.af[1][q] - curl (vy), a2 = az - curl (vz);
   g.w[0][q] = adj_cell<T, 0> (g, q, a0, ex, special, o0);
   g.w[1][q] = adj_cell<T, 1> (g, q, a1, ey, special, o1);
   g.w[2][q] = adj_cell<T, 2> (g, q, a2, ez, special, o2);
 }
-
-// aEz += 2 Ez on the monitor rectangle (mon: that step's recorded Ez, [x][y]).
-template <typename T>
-__global__ void adj_source (T *aez, const T *mon, int64_t sx, int sy, int64_t mz, int mx0, int my0, int mnx, int mny)
-{
-  const int u = (int) (blockIdx.x * blockDim.x + threadIdx.x);
-  if (u >= mnx * mny) return;
-  const int x = mx0 + u / mny, y = my0 + u % mny;
-  const int64_t q = (int64_t) x * sx + (int64_t) y * sy + mz;
-  aez[q] += (T) 2 * mon[u];
-}
-
-// Trace box geometry: E cells [lo, lo + n) of the three components, [comp][x][y][z].
-struct TraceBox
-{
-  int lo[3], n[3];
-  __host__ __device__ int64_t cells () const { return (int64_t) n[0] * n[1] * n[2]; }
-  __host__ __device__ int64_t at (int c, int x, int y, int z) const
-  {
-    return ((c * (int64_t) n[0] + (x - lo[0])) * n[1] + (y - lo[1])) * n[2] + (z - lo[2]);
-  }
-};
 
 // Copies E of the trace box (and Ez of the monitor rectangle when mon != null).
 template <typename T>
@@ -195,9 +263,11 @@ __global__ void adj_record (const T *Ex, const T *Ey, const T *Ez, int64_t sx, i
   const int64_t u = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t nc = tb.cells ();
   if (u >= nc) return;
-  const int z = tb.lo[2] + (int) (u % tb.n[2]);
-  const int y = tb.lo[1] + (int) ((u / tb.n[2]) % tb.n[1]);
-  const int x = tb.lo[0] + (int) (u / ((int64_t) tb.n[2] * tb.n[1]));
+  int x, y, z;
+  box_cell (tb.n, u, x, y, z);
+  x += tb.lo[0];
+  y += tb.lo[1];
+  z += tb.lo[2];
   const int64_t q = (int64_t) x * sx + (int64_t) y * sy + z;
   slot[u] = Ex[q];
   slot[nc + u] = Ey[q];
@@ -211,40 +281,6 @@ __global__ void adj_monitor (const T *Ez, int64_t sx, int sy, int64_t mz, int mx
   if (u >= mnx * mny) return;
   const int x = mx0 + u / mny, y = my0 + u % mny;
   out[u] = Ez[(int64_t) x * sx + (int64_t) y * sy + mz];
-}
-
-// grad(v) += sum over the six E cells whose material average contains voxel v of
-// aE(c) * (-(E'(c) - E(c)) / m(c)) / 2, for the design voxels [dlo, dhi).
-template <typename T>
-__global__ void adj_grad (AdjArgs<T> g, TraceBox tb, const T *cur, const T *prev, int dlo0, int dlo1, int dlo2,
-                          int dn0, int dn1, int dn2, double *grad)
-{
-  const StepArgs<T> &a = g.a;
-  const int64_t u = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= (int64_t) dn0 * dn1 * dn2) return;
-  const int vz = dlo2 + (int) (u % dn2);
-  const int vy = dlo1 + (int) ((u / dn2) % dn1);
-  const int vx = dlo0 + (int) (u / ((int64_t) dn2 * dn1));
-  const int64_t sx = a.sx;
-  const int sy = a.sy;
-  double acc = 0;
-  // (component, cell offset along that component's axis): cells c = v and c = v - e_axis
-#pragma unroll
-  for (int comp = 0; comp < 3; ++comp)
-  {
-#pragma unroll
-    for (int back = 0; back < 2; ++back)
-    {
-      const int cx = vx - (comp == 0 ? back : 0), cy = vy - (comp == 1 ? back : 0), cz = vz - (comp == 2 ? back : 0);
-      const int64_t qc = (int64_t) cx * sx + (int64_t) cy * sy + cz;
-      const int64_t step = comp == 0 ? sx : (comp == 1 ? (int64_t) sy : 1);
-      const T m = avg2 (a.eps[qc], a.eps[qc + step]);
-      const int64_t tix = tb.at (comp, cx, cy, cz);
-      const T de = cur[tix] - prev[tix];
-      acc += (double) g.af[comp][qc] * (-(double) de / (double) m) * 0.5;
-    }
-  }
-  grad[u] += acc;
 }
 
 // Writes the design-box values into the eps grid.
@@ -373,8 +409,12 @@ int snapshot (yee_handle *h, int k, bool restore)
   return YEE_OK;
 }
 
+int64_t grad_blocks (const AdjointState *s) { return (s->dn[0] * s->dn[1] * s->dn[2] + 255) / 256; }
+
+// One reverse step.  d: the gradient that the reverse step before left to do (none: cur null), done in
+// this step's H launch; on return the gradient of this step.
 template <typename T>
-int reverse_step (yee_handle *h, int32_t t, int slot_cur, int slot_prev)
+int reverse_step (yee_handle *h, int32_t t, int slot_cur, int slot_prev, GradArgs<T> &d)
 {
   AdjointState *s = h->adj;
   AdjArgs<T> g = adj_args<T> (h);
@@ -390,28 +430,48 @@ int reverse_step (yee_handle *h, int32_t t, int slot_cur, int slot_prev)
   const int W = s->sp.window;
   if (t >= s->T - W)
   {
-    const int nm = s->mnx * s->mny;
-    hipLaunchKernelGGL ((adj_source<T>), dim3 ((unsigned) ((nm + 255) / 256)), dim3 (256), 0, h->stream, g.af[2],
-                       (const T *) s->mon + (size_t) (t - (s->T - W)) * nm, h->n[1] * h->n[2], (int) h->n[2],
-                       s->sp.monitor_z, (int) s->sp.monitor_lo[0], (int) s->sp.monitor_lo[1], s->mnx, s->mny);
+    g.mon = (const T *) s->mon + (size_t) (t - (s->T - W)) * s->mnx * s->mny;
+    g.mx0 = (int) s->sp.monitor_lo[0];
+    g.my0 = (int) s->sp.monitor_lo[1];
+    g.mnx = s->mnx;
+    g.mny = s->mny;
+    g.mz = (int) s->sp.monitor_z;
   }
+  dim3 hgrid = grid;
+  if (d.cur) hgrid.x += (unsigned) grad_blocks (s);
   if (h->mode == 1)
   {
-    hipLaunchKernelGGL ((adj_h<T, 1>), grid, block, 0, h->stream, g);
+    hipLaunchKernelGGL ((adj_h<T, 1>), hgrid, block, 0, h->stream, g, d, (int) grid.x);
     hipLaunchKernelGGL ((adj_e<T, 1>), grid, block, 0, h->stream, g);
   }
   else
   {
-    hipLaunchKernelGGL ((adj_h<T, 0>), grid, block, 0, h->stream, g);
+    hipLaunchKernelGGL ((adj_h<T, 0>), hgrid, block, 0, h->stream, g, d, (int) grid.x);
     hipLaunchKernelGGL ((adj_e<T, 0>), grid, block, 0, h->stream, g);
   }
-  const int64_t nd = s->dn[0] * s->dn[1] * s->dn[2];
   const int64_t nc = s->tb.cells ();
-  hipLaunchKernelGGL ((adj_grad<T>), dim3 ((unsigned) ((nd + 255) / 256)), dim3 (256), 0, h->stream, g, s->tb,
-                     (const T *) s->trace + (size_t) slot_cur * 3 * nc, (const T *) s->trace + (size_t) slot_prev * 3 * nc,
-                     (int) s->sp.design_lo[0], (int) s->sp.design_lo[1], (int) s->sp.design_lo[2], (int) s->dn[0],
-                     (int) s->dn[1], (int) s->dn[2], s->grad);
+  d.tb = s->tb;
+  d.cur = (const T *) s->trace + (size_t) slot_cur * 3 * nc;
+  d.prev = (const T *) s->trace + (size_t) slot_prev * 3 * nc;
+  for (int ax = 0; ax < 3; ++ax)
+  {
+    d.lo[ax] = (int) s->sp.design_lo[ax];
+    d.n[ax] = (int) s->dn[ax];
+  }
+  d.grad = s->grad;
   HIP_TRY (hipGetLastError ());
+  return YEE_OK;
+}
+
+// The gradient that the last reverse step of a segment left, before the trace is written again or read
+// out (aE is the one of that step until then).
+template <typename T>
+int last_gradient (yee_handle *h, GradArgs<T> &d)
+{
+  if (!d.cur) return YEE_OK;
+  hipLaunchKernelGGL ((adj_grad<T>), dim3 ((unsigned) grad_blocks (h->adj)), dim3 (256), 0, h->stream, adj_args<T> (h), d);
+  HIP_TRY (hipGetLastError ());
+  d.cur = nullptr;
   return YEE_OK;
 }
 
@@ -500,10 +560,12 @@ int backward_impl (yee_handle *h, double dJ, double *grad)
   HIP_TRY (hipMemsetAsync (s->grad, 0, (size_t) nd * sizeof (double), h->stream));
   HIP_TRY (hipEventRecord (h->ev[0], h->stream));
   const int K = s->sp.checkpoint_every;
+  GradArgs<T> grad_d {};
   if (K == 0)
   {
     for (int32_t t = s->T - 1; t >= 1; --t)
-      if ((rc = reverse_step<T> (h, t, t, t - 1))) return rc;
+      if ((rc = reverse_step<T> (h, t, t, t - 1, grad_d))) return rc;
+    if ((rc = last_gradient (h, grad_d))) return rc;
   }
   else
   {
@@ -522,7 +584,8 @@ int backward_impl (yee_handle *h, double dJ, double *grad)
         }
       }
       for (int32_t t = t1; t >= t0 + 1; --t)
-        if ((rc = reverse_step<T> (h, t, t - t0, t - t0 - 1))) return rc;
+        if ((rc = reverse_step<T> (h, t, t - t0, t - t0 - 1, grad_d))) return rc;
+      if ((rc = last_gradient (h, grad_d))) return rc;
     }
     s->last_traced = false;   // the trace now holds segment 0
   }

@@ -236,3 +236,28 @@ def test_sweep_and_half_steps_meet(z, y, precision, engine_lib, monkeypatch):
     for n, v in ref.items():
         assert np.array_equal(got[n], v), n
     assert np.abs(ref["Ez"]).max() > 0
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (16, 16, 1), (1, 1, 17), (8, 4, 8), (7, 6, 7)])
+def test_gradient_in_the_next_reverse_step(dims, precision, engine_lib):
+    """A reverse step's gradient is added in the next one's H launch (1 to 294 voxels: one block, one
+    full block, a block of rest): bit-identical to the gradient in a launch of its own, which segments
+    of one step take, with the monitor rectangle through the design box."""
+    args = "--3d --size x:28,y:27,z:29 --use-pml --pml-size x:3,y:3,z:3 --point-source x:5,y:6,z:7 --point-source-ez " \
+           "--wavelength 0.004 --time-steps 24"
+    print(f"[gpu] gradient in the next reverse step, design {dims}, precision {precision}", flush=True)
+    rng = np.random.default_rng(6)
+    eps = rng.uniform(1.0, 4.0, size=(28, 27, 29))
+    design = rng.uniform(1.0, 4.0, size=dims)
+    out = []
+    for every in (0, 1, 5):
+        eng = Engine(parse_args(args.split(), precision=precision))
+        eng.set_material("eps", eps)
+        eng.prepare()
+        eng.adjoint_setup((5, 5, 6), tuple(lo + n for lo, n in zip((5, 5, 6), dims)), 6, (4, 4), (20, 19), 9, every)
+        out.append((eng.forward(design), eng.backward(1.0)))
+        eng.close()
+    for J, g in out[1:]:
+        assert J == out[0][0] and np.array_equal(g, out[0][1])
+    assert np.abs(out[0][1]).max() > 0
