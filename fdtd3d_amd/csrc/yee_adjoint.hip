@@ -235,22 +235,32 @@ __global__ __launch_bounds__ (256) void adj_e (AdjArgs<T> g)
   const T vx[4] = { wz[q - sy], wz[q], wy[q - 1], wy[q] };
   const T vy[4] = { wx[q - 1], wx[q], wz[q - sx], wz[q] };
   const T vz[4] = { wy[q - sx], wy[q], wx[q - sy], wx[q] };
-  T ex = a.eps_u, ey = a.eps_u, ez = a.eps_u;
+  // (averaged after the last load: averages here would wait for every load before them; backward of
+  // 128^3, 160 steps: FP32 17.8 ms so, 17.6 now, FP64 37.6 and 37.1)
+  T m0, mx, my, mz;
   if (a.eps)
   {
-    const T e = a.eps[q];
-    ex = avg2 (e, a.eps[q + sx]);
-    ey = avg2 (e, a.eps[q + sy]);
-    ez = avg2 (e, a.eps[q + 1]);
+    m0 = a.eps[q];
+    mx = a.eps[q + sx];
+    my = a.eps[q + sy];
+    mz = a.eps[q + 1];
   }
   AdjOld<T> o0 {}, o1 {}, o2 {};
   adj_load<T, 0> (g, q, p, special, o0);
   adj_load<T, 1> (g, q, p, special, o1);
   adj_load<T, 2> (g, q, p, special, o2);
+  const T f0 = g.af[0][q], f1 = g.af[1][q];
   T az = g.af[2][q];
+  T ex = a.eps_u, ey = a.eps_u, ez = a.eps_u;
+  if (a.eps)
+  {
+    ex = avg2 (m0, mx);
+    ey = avg2 (m0, my);
+    ez = avg2 (m0, mz);
+  }
   const int mi = i - g.mx0, mj = j - g.my0;
   if (g.mon && k == g.mz && mi >= 0 && mi < g.mnx && mj >= 0 && mj < g.mny) az += (T) 2 * g.mon[mi * g.mny + mj];
-  const T a0 = g.af[0][q] - curl (vx), a1 = g.af[1][q] - curl (vy), a2 = az - curl (vz);
+  const T a0 = f0 - curl (vx), a1 = f1 - curl (vy), a2 = az - curl (vz);
   g.w[0][q] = adj_cell<T, 0> (g, q, a0, ex, special, o0);
   g.w[1][q] = adj_cell<T, 1> (g, q, a1, ey, special, o1);
   g.w[2][q] = adj_cell<T, 2> (g, q, a2, ez, special, o2);
