@@ -413,9 +413,16 @@ int snapshot (yee_handle *h, int k, bool restore)
     if ((rc = move (h->f[h->cur][c], grid))) return rc;
     if ((rc = move (h->d[h->cur][c], grid))) return rc;
   }
-  if (restore) h->inc_t = h->hist_t = h->t;   // the next step restarts the incident rows
   if ((rc = move (h->einc[h->inc_cur], inc))) return rc;
   if ((rc = move (h->hinc[h->inc_cur], inc))) return rc;
+  if (restore)
+  {
+    h->inc_t = h->hist_t = h->t;   // the next step restarts the incident rows
+    // the other buffer holds the wave of later steps, and a launch of incident_steps writes it only
+    // as far as the wave of its own steps reaches: the launch after that would read the rest as zeros
+    for (void *p : { h->einc[1 - h->inc_cur], h->hinc[1 - h->inc_cur] })
+      if (p) HIP_TRY (hipMemsetAsync (p, 0, inc, h->stream));
+  }
   return YEE_OK;
 }
 

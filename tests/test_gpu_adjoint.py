@@ -122,3 +122,26 @@ def test_fp32_gradient_vs_fp64(engine_lib):
         g.append(e.backward(1.0))
         e.close()
     assert rel_l2(g[1], g[0]) <= 1e-3
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("every", [50, 150, 200])
+def test_long_checkpoint_intervals_with_tfsf(every, precision, engine_lib):
+    """A re-run segment starts from the incident wave of its snapshot, not from what later steps left
+    behind: several launches of 32 incident steps in a segment, and a wave that has passed the cells
+    of the first one (192 cells for the 161-cell rows of this box) before the segment is run again.
+    J and gradient are those of the traced pass, bit for bit."""
+    args = "--3d --size x:20,y:20,z:160 --use-pml --pml-size x:3,y:3,z:3 --use-tfsf --tfsf-size-left x:6,y:6,z:6 " \
+           "--tfsf-size-right x:6,y:6,z:6 --angle-teta 0 --angle-phi 0 --angle-psi 0 --time-steps 400"
+    say(f"[gpu] checkpoints every {every} steps with TF/SF, precision {precision}")
+    dlo, dhi = (8, 8, 136), (12, 12, 146)
+    design = np.random.default_rng(5).uniform(1.5, 2.5, size=(4, 4, 10))
+    out = []
+    for k in (0, every):
+        cfg = parse_args(args.split())
+        e = _engine(cfg, _eps(cfg, 9), dlo, dhi, 148, (5, 5), (15, 15), 60, precision, k)
+        out.append((e.forward(design), e.backward(1.0)))
+        e.close()
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1])
+    assert np.abs(out[0][1]).max() > 0
