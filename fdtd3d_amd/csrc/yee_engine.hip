@@ -403,13 +403,13 @@ bool exp_has (const yee_handle *h, int comp)
   return h->fn_exact >= YEE_FN_EXP1 && (comp == kE[h->exp_pair] || comp == kH[h->exp_pair]);
 }
 
-// Records an event pair around the next launch when kernel timing is on.
+// Records an event pair around the next launch, which takes `steps` steps, when kernel timing is on.
 struct ProfScope
 {
   yee_handle *h;
-  int kind;
+  int kind, steps;
   bool on;
-  ProfScope (yee_handle *hh, int k) : h (hh), kind (k), on (hh->prof_events != nullptr)
+  ProfScope (yee_handle *hh, int k, int n = 1) : h (hh), kind (k), steps (n), on (hh->prof_events != nullptr)
   {
     if (on) record ();
   }
@@ -424,7 +424,7 @@ struct ProfScope
     {
       (void) hipEventRecord (e, h->stream);
       h->prof_events->push_back (e);
-      h->prof_kinds->push_back (kind);
+      h->prof_kinds->push_back ({ kind, steps });
     }
   }
 };
@@ -719,7 +719,7 @@ int incident_ahead (yee_handle *h, int32_t ahead)
   // cells the wave can have reached, and the rows' length
   const int64_t cells = std::max (std::min (h->inc_len, (int64_t) h->t + n + 2), h->hist_len);
   const int b = h->inc_cur;
-  ProfScope ps (h, 0);
+  ProfScope ps (h, 0, n);
   hipLaunchKernelGGL ((incident_steps<T>), dim3 ((unsigned) ((cells + kIncTile - 1) / kIncTile)), dim3 (64), 0, h->stream,
                      (const T *) h->einc[b], (const T *) h->hinc[b], (T *) h->einc[1 - b], (T *) h->hinc[1 - b],
                      h->inc_len, n, modE, modH, src, (T *) h->hist_e, (T *) h->hist_h, h->hist_len);
@@ -1142,7 +1142,7 @@ int plane_advance (yee_handle *h, int32_t ahead, int32_t &done)
   {
     LineSource src {};
     sources (src.v);
-    ProfScope ps (h, 3);
+    ProfScope ps (h, 3, n);
     launch_line<T> (h->cfg.scheme, a, n, src, h->stream);
   }
   else
@@ -1152,7 +1152,7 @@ int plane_advance (yee_handle *h, int32_t ahead, int32_t &done)
     const int ma = missing_axis (h->cfg), ra = ma == 0 ? 1 : 0, ca = ma == 2 ? 1 : 2;
     const PlaneGrid g = plane_grid<T> (h->n[ra], h->n[ca], n, h->ncu);
     if (g.ntile < 0) return fail (YEE_EINVAL, "grid too large for one launch");
-    ProfScope ps (h, 3);
+    ProfScope ps (h, 3, n);
     launch_plane<T> (h->cfg.scheme, a, g, src, h->stream);
   }
   HIP_TRY (hipGetLastError ());
@@ -1663,7 +1663,7 @@ int yee_profile_steps (yee_handle *h, int32_t n, double out[5])
   if (!h->prepared) return fail (YEE_ESTATE, "yee_prepare has not been called");
   if (n <= 0) return fail (YEE_EINVAL, "step count must be positive");
   std::vector<hipEvent_t> events;
-  std::vector<int> kinds;
+  std::vector<std::pair<int, int>> kinds;
   events.reserve ((size_t) n * 6);
   kinds.reserve ((size_t) n * 6);
   h->prof_events = &events;
@@ -1672,19 +1672,19 @@ int yee_profile_steps (yee_handle *h, int32_t n, double out[5])
   h->prof_events = nullptr;
   h->prof_kinds = nullptr;
   double sum[4] = { 0, 0, 0, 0 };
-  int cnt[4] = { 0, 0, 0, 0 };
+  int steps[4] = { 0, 0, 0, 0 };   // a launch of the incident grid or of a 1D or 2D run takes several
   for (size_t e = 0; rc == YEE_OK && e + 1 < events.size (); e += 2)
   {
     float ms = 0;
     if (hipEventElapsedTime (&ms, events[e], events[e + 1]) == hipSuccess)
     {
-      sum[kinds[e]] += ms;
-      cnt[kinds[e]]++;
+      sum[kinds[e].first] += ms;
+      steps[kinds[e].first] += kinds[e].second;
     }
   }
   for (hipEvent_t e : events) (void) hipEventDestroy (e);
   if (rc) return rc;
-  for (int k = 0; k < 4; ++k) out[k] = cnt[k] ? sum[k] / cnt[k] : 0.0;
+  for (int k = 0; k < 4; ++k) out[k] = steps[k] ? sum[k] / steps[k] : 0.0;
   out[4] = h->last_ms;
   return YEE_OK;
 }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/yee.h"
@@ -94,9 +95,10 @@ struct yee_handle
   int32_t t = 0;
   bool prepared = false;
   double last_ms = 0;
-  // kernel timing (yee_profile_steps): events recorded around each launch when set
+  // kernel timing (yee_profile_steps): events recorded around each launch when set, with its group
+  // and the steps it takes
   std::vector<hipEvent_t> *prof_events = nullptr;
-  std::vector<int> *prof_kinds = nullptr;
+  std::vector<std::pair<int, int>> *prof_kinds = nullptr;
 
   bool fp32 () const { return wsize == 4; }
   bool use_pml () const { return (cfg.flags & YEE_USE_PML) != 0; }

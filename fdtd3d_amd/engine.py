@@ -287,7 +287,7 @@ class Engine:
         return ms.value
 
     def profile_steps(self, n: int) -> dict:
-        """Runs n steps with per-kernel HIP events; average ms per launch of each kernel."""
+        """Runs n steps with HIP events around the launches; average ms per step of each group of kernels."""
         out = np.zeros(5, dtype=np.float64)
         _check(load_library().yee_profile_steps(self.h, int(n), out.ctypes.data))
         return {"incident_ms": float(out[0]), "e_half_ms": float(out[1]), "h_half_ms": float(out[2]),

@@ -362,11 +362,12 @@ int yee_last_step_ms (yee_handle *h, double *ms);
 
 /*
  * Runs `n` steps like yee_step with a HIP event pair around every group of kernel launches
- * and returns average device milliseconds per step of each group: out[0] incident 1D
- * update, out[1] E half-step (with the fused step: the E update of the PML slabs), out[2]
- * H half-step (fused: the H update of the PML slabs), out[3] fused E+H step kernel of the
- * PML-free box (0 when not used), out[4] whole step (yee_last_step_ms of the run).
- * Benchmark hook; the extra events cost a few microseconds per step.
+ * and returns average device milliseconds per step of each group, whatever the steps of one
+ * launch: out[0] incident 1D update, out[1] E half-step (with the fused step: the E update of
+ * the boxes around it), out[2] H half-step (fused: the H update of those boxes), out[3] kernels
+ * that take E and H in one launch: the fused step of 3D runs, the several steps a launch of 1D
+ * and 2D runs (0 when neither is used), out[4] whole step (yee_last_step_ms of the run).
+ * Benchmark hook; the extra events cost a few microseconds per launch.
  */
 int yee_profile_steps (yee_handle *h, int32_t n, double out[5]);
 

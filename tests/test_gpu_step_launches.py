@@ -261,3 +261,27 @@ def test_gradient_in_the_next_reverse_step(dims, precision, engine_lib):
     for J, g in out[1:]:
         assert J == out[0][0] and np.array_equal(g, out[0][1])
     assert np.abs(out[0][1]).max() > 0
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("args,one_launch", [
+    ("--1d-exhy --size z:600 --use-pml --pml-size z:50 --use-tfsf --tfsf-size-left z:150 --tfsf-size-right z:0 --angle-teta 0 "
+     "--angle-phi 0", True),
+    ("--2d-tmz --size x:160,y:140 --use-pml --pml-size x:6,y:6 --use-tfsf --tfsf-size-left x:12,y:12 --tfsf-size-right "
+     "x:12,y:12 --angle-teta 90 --angle-phi 30", True),
+    ("--3d --size x:40,y:40,z:40 --use-pml --pml-size x:5,y:5,z:5 --use-tfsf --tfsf-size-left x:9,y:9,z:9 --tfsf-size-right "
+     "x:9,y:9,z:9 --angle-teta 30 --angle-phi 45 --angle-psi 90", False),
+])
+def test_profile_is_per_step(args, one_launch, precision, engine_lib):
+    """The groups of yee_profile_steps are milliseconds per step however many steps a launch takes:
+    their intervals follow one another on one stream inside the measured run, so their sum is at most
+    the step's own time (5 % for the resolution of the time stamps)."""
+    eng = Engine(parse_args((args + " --time-steps 300").split(), precision=precision))
+    eng.prepare()
+    eng.step(70)
+    p = eng.profile_steps(70)
+    eng.close()
+    groups = [p[k] for k in ("incident_ms", "e_half_ms", "h_half_ms", "fused_ms")]
+    print(f"[gpu] profile {args.split()[0]} precision {precision}: {p}", flush=True)
+    assert p["incident_ms"] > 0 and (p["fused_ms"] > 0) == one_launch and (p["e_half_ms"] > 0) != one_launch
+    assert sum(groups) <= 1.05 * p["step_ms"]
