@@ -1377,12 +1377,19 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   // are disjoint, face boxes are clipped to the fused box), so they update in place: the second
   // buffer's views alias the first's.  The Drude box overlaps slab and face boxes, so Drude
   // runs keep two buffers.
-  // 1D and 2D runs keep two buffers of every array too when they fit (a tile's margin reads old values)
+  // 1D and 2D runs keep two buffers of every array too (a tile's margin reads old values), and 2D runs
+  // with PML six words a cell of factors.  What that adds may take a quarter of the free memory: the
+  // materials and what else the program allocates need the rest, and the half-step kernels do
+  // without (8 words a cell of TMz with PML, eps and mu, against 20).
+  const int present = (int) std::count (h->present, h->present + 6, true);
   {
     int active = 0;
     for (int ax = 0; ax < 3; ++ax) active += axis_active (*cfg, ax) ? 1 : 0;
+    const int words = present * (h->mode >= 1 ? 2 : 1) + (h->mode >= 1 && line < 0 ? 6 : 0);
+    size_t mem_free = 0, mem_total = 0;
     h->plane = active <= 2 && h->mode <= 1 && cfg->layout == 0 && want_fused
-               && 36.0 * (double) h->ncell * (double) h->wsize < 200e9;
+               && hipMemGetInfo (&mem_free, &mem_total) == hipSuccess
+               && (double) words * (double) h->ncell * (double) h->wsize <= 0.25 * (double) mem_free;
   }
   const int nbuf = h->fused || h->plane ? 2 : 1;
   // the arrays of a 1D or 2D run in one allocation (each costs about 10 us, and its clearing a launch)
@@ -1390,7 +1397,6 @@ int yee_create (const yee_config *cfg, yee_handle **out)
   const size_t each = ((size_t) (kPadFront + h->ncell + pad_back (h)) * h->wsize + 255) / 256 * 256;
   if (h->plane && each <= (size_t) 1 << 26)
   {
-    const int present = (int) std::count (h->present, h->present + 6, true);
     void *all = nullptr;
     rc = alloc_zero (h, &all, (size_t) (present * nbuf * (h->mode >= 1 ? 2 : 1)) * each);
     if (all) h->grids.push_back (all);
@@ -1608,15 +1614,22 @@ int yee_prepare (yee_handle *h)
   }
   if (h->plane && h->use_pml () && line_axis (h->cfg) < 0)
   {
-    // (one allocation: pairs for each of the scheme's three components)
+    // (one allocation: pairs for each of the scheme's three components; half steps without it)
     void *p = nullptr;
-    HIP_TRY (hipMalloc (&p, 6 * (size_t) h->ncell * h->wsize));
-    h->grids.push_back (p);
-    for (int c = 0, k = 0; c < 6; ++c)
-      if (h->exposed[c]) h->pfac[c] = (char *) p + 2 * k++ * (size_t) h->ncell * h->wsize;
-    if (h->fp32 ()) launch_plane_factors<float> (h->cfg.scheme, make_args<float> (h), h->stream);
-    else launch_plane_factors<double> (h->cfg.scheme, make_args<double> (h), h->stream);
-    HIP_TRY (hipGetLastError ());
+    if (hipMalloc (&p, 6 * (size_t) h->ncell * h->wsize) != hipSuccess)
+    {
+      (void) hipGetLastError ();
+      h->plane = false;
+    }
+    else
+    {
+      h->grids.push_back (p);
+      for (int c = 0, k = 0; c < 6; ++c)
+        if (h->exposed[c]) h->pfac[c] = (char *) p + 2 * k++ * (size_t) h->ncell * h->wsize;
+      if (h->fp32 ()) launch_plane_factors<float> (h->cfg.scheme, make_args<float> (h), h->stream);
+      else launch_plane_factors<double> (h->cfg.scheme, make_args<double> (h), h->stream);
+      HIP_TRY (hipGetLastError ());
+    }
   }
   if (h->fn_start)
   {
