@@ -79,6 +79,7 @@ struct yee_batch
   std::vector<std::vector<BatchGroup>> groupings;   // [grouping][group], one per cache budget
   int *state = nullptr;                 // device: [sim] steps done, buffer of the newest fields
   bool two_ok = true;                   // two-step launches allowed (no mu grid in the batch)
+  bool plane_ok = true;                 // register tiles allowed (memory for their PML factors)
   int *all = nullptr;                   // 0 .. nsim-1 in device memory
   void *src_tab = nullptr;              // [sim][src_len][2] source values
   int src_len = 0;
@@ -289,10 +290,10 @@ int cand_stride (const yee_batch *b, const Cand &c)
   return c.two == 2 ? (b->wsize == 4 ? BATCH_STEPS (float) : BATCH_STEPS (double)) : (c.two ? 2 : 1);
 }
 
-// A mu grid rules out the two-step kernel.
+// A mu grid rules out the two-step kernel, short memory the register tiles.
 bool cand_ok (const yee_batch *b, const Cand &c)
 {
-  return c.two != 1 || b->two_ok;
+  return c.two == 2 ? b->plane_ok : (c.two == 0 || b->two_ok);
 }
 
 // `k` steps of group g with candidate c's tiles: one launch where k is at most the candidate's
@@ -406,7 +407,8 @@ int step_impl (yee_batch *b, int32_t n)
     (void) hipEventDestroy (e0);
     (void) hipEventDestroy (e1);
   }
-  if (b->cand < 0) b->cand = kPlaneCand;   // too few steps to tune
+  // too few steps to tune (without the register tiles: one group, 64-row tiles)
+  if (b->cand < 0) b->cand = b->plane_ok ? kPlaneCand : 2;
   const Cand &c = kCands[b->cand];
   const char *use_graph = std::getenv ("YEE_BATCH_GRAPH");
   // (a launch of the register tiles covers enough steps by itself)
@@ -463,7 +465,8 @@ int prepare_impl (yee_batch *b)
 {
   int rc;
   std::vector<StepArgs<T>> args (2 * (size_t) b->nsim);
-  // the D/B -> field factors of the register tiles' PML cells (pairs for Ez, Hx, Hy), in one allocation
+  // the D/B -> field factors of the register tiles' PML cells (pairs for Ez, Hx, Hy), in one allocation,
+  // if it takes no more than a quarter of the free memory (six words a cell beside 12 of state)
   std::vector<size_t> pf_at ((size_t) b->nsim);
   size_t pf_bytes = 0;
   for (int s = 0; s < b->nsim; ++s)
@@ -475,8 +478,11 @@ int prepare_impl (yee_batch *b)
   void *pf = nullptr;
   if (pf_bytes)
   {
-    BHIP (hipMalloc (&pf, pf_bytes));
-    b->grids.push_back (pf);
+    size_t mem_free = 0, mem_total = 0;
+    b->plane_ok = hipMemGetInfo (&mem_free, &mem_total) == hipSuccess && pf_bytes <= mem_free / 4
+                  && hipMalloc (&pf, pf_bytes) == hipSuccess;
+    if (b->plane_ok) b->grids.push_back (pf);
+    else (void) hipGetLastError ();
   }
   for (int s = 0; s < b->nsim; ++s)
   {
@@ -491,9 +497,12 @@ int prepare_impl (yee_batch *b)
       BHIP (hipMemcpyAsync (p, tv.data (), tv.size () * sizeof (T), hipMemcpyHostToDevice, b->stream));
       BHIP (hipStreamSynchronize (b->stream));
       b->pml[s] = p;
-      b->pfac[s] = (char *) pf + pf_at[s];
-      launch_plane_factors<T> (YEE_SCHEME_TMZ, sim_args<T> (b, s, 0), b->stream);
-      BHIP (hipGetLastError ());
+      if (b->plane_ok)
+      {
+        b->pfac[s] = (char *) pf + pf_at[s];
+        launch_plane_factors<T> (YEE_SCHEME_TMZ, sim_args<T> (b, s, 0), b->stream);
+        BHIP (hipGetLastError ());
+      }
     }
     args[2 * s] = sim_args<T> (b, s, 0);
     args[2 * s + 1] = sim_args<T> (b, s, 1);

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from fdtd3d_amd.config import parse_args
-from fdtd3d_amd.engine import Engine, load_library
+from fdtd3d_amd.engine import Batch, Engine, load_library
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +65,24 @@ def test_2d_run_in_short_memory(engine_lib):
     for c, v in ref.items():
         assert np.array_equal(got[c], v), c
     assert np.abs(ref["Ez"]).max() > 0
+
+
+def test_batch_in_short_memory(engine_lib):
+    """17 words a cell free: the batch's two buffers and the materials fit (14), the factors of the
+    register tiles do not (6 more).  The batch goes on with its other launches, long enough to tune
+    them, with the fields of a single run."""
+    eps = np.random.default_rng(2).uniform(1.0, 3.0, size=(3600, 3500))
+    ref = _fields(eps, [70])
+    with only(17 * WORD):
+        b = Batch([parse_args(ARGS.split(), precision=8)])
+        try:
+            b.set_material(0, "eps", eps)
+            b.set_material(0, "mu", eps)
+            b.prepare()
+            b.step(3)
+            b.step(67)
+            got = {c: b.field(0, c) for c in ref}
+        finally:
+            b.close()
+    for c, v in ref.items():
+        assert np.array_equal(got[c], v), c
