@@ -11,6 +11,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <mutex>
 #include <thread>
@@ -40,10 +41,18 @@ struct Pool
   int round = 0, want = 0, left = 0;
   bool stop = false;
 
+  // Up to n - 1 threads: where the process may start no more, run goes on with fewer.
   void start (int n)
   {
     stop = false;
-    for (int t = 1; t < n; ++t) threads.emplace_back ([this, t, seen = round] { serve (t, seen); });
+    try
+    {
+      threads.reserve ((size_t) n);
+      for (int t = 1; t < n; ++t) threads.emplace_back ([this, t, seen = round] { serve (t, seen); });
+    }
+    catch (const std::exception &)
+    {
+    }
   }
 
   void serve (int t, int seen)
