@@ -110,15 +110,16 @@ struct Staging
   Pool pool;
 
   // Buffers, events and threads for reads on `dev`; false if they are another device's or cannot
-  // be had.
+  // be had (the next check of a launch must not find that error).
   bool open (int dev)
   {
     if (buf) return dev == device;
-    for (hipEvent_t &e : ev)
-      if (!e && hipEventCreateWithFlags (&e, hipEventDisableTiming) != hipSuccess) return false;
-    if (hipHostMalloc ((void **) &buf, 2 * kThreads * kChunk, hipHostMallocDefault) != hipSuccess)
+    bool ok = true;
+    for (hipEvent_t &e : ev) ok = ok && (e || hipEventCreateWithFlags (&e, hipEventDisableTiming) == hipSuccess);
+    if (!ok || hipHostMalloc ((void **) &buf, 2 * kThreads * kChunk, hipHostMallocDefault) != hipSuccess)
     {
       buf = nullptr;
+      (void) hipGetLastError ();
       return false;
     }
     device = dev;

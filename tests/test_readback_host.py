@@ -98,6 +98,12 @@ int main (int argc, char **argv)
     threads_left = -1;
     CHECK (read_ramp (0, large + 3) == 0);
   }
+  else if (what == "pinned")
+  {
+    no_pinned = true;
+    CHECK (read_ramp (0, large + 3) == 0);
+    CHECK (hipGetLastError () == hipSuccess);
+  }
   else CHECK (!"a known case");
   yee::readback_unref ();
   CHECK (pinned == 0);
@@ -130,3 +136,9 @@ def test_read_with_fewer_threads_than_asked_for(program, allowed):
     """std::thread throws where the process may start no more threads: the read goes on with those
     that started, none at worst, and leaves no exception for a C caller."""
     run(program, "threads", str(allowed))
+
+
+def test_no_error_left_where_pinned_memory_cannot_be_had(program):
+    """The read then takes plain copies, and the error of the attempt is not left for the next
+    check of a kernel launch."""
+    run(program, "pinned")
