@@ -101,6 +101,21 @@ struct Pool
   }
 };
 
+// The current device of the thread is `device` while this lives.
+struct OnDevice
+{
+  int before = -1;
+  bool ok;
+  explicit OnDevice (int device)
+  {
+    ok = hipGetDevice (&before) == hipSuccess && (before == device || hipSetDevice (device) == hipSuccess);
+  }
+  ~OnDevice ()
+  {
+    if (before >= 0) (void) hipSetDevice (before);
+  }
+};
+
 struct Staging
 {
   std::mutex mu;   // held by the one read that uses the buffers and threads
@@ -109,7 +124,7 @@ struct Staging
   hipEvent_t ev[2 * kThreads] = {};
   Pool pool;
 
-  // Buffers, events and threads for reads on `dev`; false if they are another device's or cannot
+  // Buffers, events and threads for reads on `dev`, the current device; false if they are another device's or cannot
   // be had (the next check of a launch must not find that error).
   bool open (int dev)
   {
@@ -119,6 +134,7 @@ struct Staging
     if (!ok || hipHostMalloc ((void **) &buf, 2 * kThreads * kChunk, hipHostMallocDefault) != hipSuccess)
     {
       buf = nullptr;
+      close ();   // (events made before the failure are of this device)
       (void) hipGetLastError ();
       return false;
     }
@@ -177,6 +193,8 @@ hipError_t read_back (int device, hipStream_t stream, const void *src, int64_t n
 {
   const int64_t bytes = n * (int64_t) wsize;
   const int64_t grow = widen ? 2 : 1;
+  const OnDevice on (device);   // (the events and the stream must be of one device)
+  if (!on.ok) return hipErrorInvalidDevice;
   std::unique_lock<std::mutex> use (g_staging.mu, std::try_to_lock);
   // small reads, and reads while another thread holds the buffers: one plain copy
   if (bytes * grow < kLeast || !use.owns_lock () || !g_staging.open (device))
@@ -200,7 +218,7 @@ hipError_t read_back (int device, hipStream_t stream, const void *src, int64_t n
       if (e != hipSuccess) err = e;
       return e != hipSuccess;
     };
-    if (fail (hipSetDevice (device))) return;
+    if (t > 0 && fail (hipSetDevice (device))) return;
     auto queue = [&] (int64_t c, int slot) {
       const int64_t at = c * chunk, len = std::min (chunk, bytes - at);
       hipError_t e = hipMemcpyAsync (g_staging.buf + slot * kChunk, (const char *) src + at, (size_t) len,

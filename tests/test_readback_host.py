@@ -20,7 +20,7 @@ HIP = r"""
 typedef int hipError_t;
 typedef struct stream { int device; } *hipStream_t;
 typedef struct event { int device; } *hipEvent_t;
-enum { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorInvalidHandle = 400 };
+enum { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorInvalidDevice = 101, hipErrorInvalidHandle = 400 };
 enum { hipMemcpyDeviceToHost, hipEventDisableTiming, hipHostMallocDefault };
 inline thread_local int cur_dev = 0;
 inline thread_local hipError_t last = hipSuccess;
@@ -104,6 +104,13 @@ int main (int argc, char **argv)
     CHECK (read_ramp (0, large + 3) == 0);
     CHECK (hipGetLastError () == hipSuccess);
   }
+  else if (what == "device")
+  {
+    hipSetDevice (1);   // another one than the handle's
+    CHECK (read_ramp (0, large + 3) == 0);
+    CHECK (cur_dev == 1);
+    CHECK (hipGetLastError () == hipSuccess);
+  }
   else CHECK (!"a known case");
   yee::readback_unref ();
   CHECK (pinned == 0);
@@ -142,3 +149,9 @@ def test_no_error_left_where_pinned_memory_cannot_be_had(program):
     """The read then takes plain copies, and the error of the attempt is not left for the next
     check of a kernel launch."""
     run(program, "pinned")
+
+
+def test_handle_of_another_device_than_the_current_one(program):
+    """The events belong to the handle's device, as its stream does, and the caller's current
+    device stays as it was."""
+    run(program, "device")
