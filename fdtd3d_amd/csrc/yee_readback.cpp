@@ -27,8 +27,14 @@ namespace {
 constexpr int64_t kChunk = 2 << 20;
 constexpr int64_t kLeastChunk = 256 << 10;
 constexpr int kThreads = 8;
-// Below this one hipMemcpy is as fast.
+// Below this one hipMemcpy is as fast (3.2 MB into pages in use: 175 us, 184 in chunks; 5.5 MB 304
+// and 226; into fresh pages 3.2 MB 749 and 299).
 constexpr int64_t kLeast = 3 << 20;
+// Opening and closing the pool (pinning 32 MB, starting threads) costs 1 to 2.5 ms, chunks gain 25 us
+// a MB in pages in use and 75 us in fresh ones.  So the first reads after the pool was closed are plain
+// copies until this much has been read: a run that reads 8 MB once takes 0.47 ms of 1.37, one
+// that reads 24 MB 1.4 of 3.9, and 48 MB at once take 4.2 ms through the pool, 4.6 plain.
+constexpr int64_t kOpen = 48 << 20;
 
 // Threads that wait for a read between reads (starting eight takes 100 us, as long as 1 MB takes
 // to arrive on the plain path).
@@ -120,9 +126,18 @@ struct Staging
 {
   std::mutex mu;   // held by the one read that uses the buffers and threads
   char *buf = nullptr;
+  int64_t plain = 0;   // bytes that plain copies of kLeast or more have put in place since the last close
   int device = -1;
   hipEvent_t ev[2 * kThreads] = {};
   Pool pool;
+
+  // Whether a read that puts `bytes` in place goes through the buffers.
+  bool wanted (int64_t bytes)
+  {
+    if (buf || plain + bytes >= kOpen) return true;
+    plain += bytes;
+    return false;
+  }
 
   // Buffers, events and threads for reads on `dev`, the current device; false if they are another device's or cannot
   // be had (the next check of a launch must not find that error).
@@ -146,6 +161,7 @@ struct Staging
   void close ()
   {
     pool.join ();
+    plain = 0;
     if (buf) (void) hipHostFree (buf);
     buf = nullptr;
     for (hipEvent_t &e : ev)
@@ -196,8 +212,8 @@ hipError_t read_back (int device, hipStream_t stream, const void *src, int64_t n
   const OnDevice on (device);   // (the events and the stream must be of one device)
   if (!on.ok) return hipErrorInvalidDevice;
   std::unique_lock<std::mutex> use (g_staging.mu, std::try_to_lock);
-  // small reads, and reads while another thread holds the buffers: one plain copy
-  if (bytes * grow < kLeast || !use.owns_lock () || !g_staging.open (device))
+  // small reads, the first ones, and reads while another thread holds the buffers: one plain copy
+  if (bytes * grow < kLeast || !use.owns_lock () || !g_staging.wanted (bytes * grow) || !g_staging.open (device))
   {
     hipError_t e = hipStreamSynchronize (stream);
     if (e != hipSuccess || !widen) return e != hipSuccess ? e : hipMemcpy (out, src, (size_t) bytes, hipMemcpyDeviceToHost);

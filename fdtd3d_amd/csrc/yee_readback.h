@@ -9,7 +9,7 @@
 namespace yee {
 
 // Every handle and batch holds one reference from its creation to its destruction; the pinned
-// buffers of read_back are allocated by the first large read and freed with the last reference.
+// buffers of read_back are allocated once enough has been read (kOpen) and freed with the last reference.
 void readback_ref ();
 void readback_unref ();
 

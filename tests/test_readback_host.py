@@ -111,6 +111,24 @@ int main (int argc, char **argv)
     CHECK (cur_dev == 1);
     CHECK (hipGetLastError () == hipSuccess);
   }
+  else if (what == "few")
+  {
+    // 4 MB and 8 MB of output a call: the fourth reaches 48
+    for (int k = 0; k < 3; ++k)
+    {
+      CHECK (read_ramp (0, 1 << 20) == 0);
+      CHECK (pinned == 0 && threads_started == 0);
+    }
+    CHECK (read_ramp (0, 1 << 20) == 0);
+    CHECK (pinned == 1 && threads_started > 0);
+    yee::readback_unref ();
+    CHECK (pinned == 0);
+    yee::readback_ref ();
+    CHECK (read_ramp (0, 1 << 20) == 0);   // counted from the start again
+    CHECK (pinned == 0);
+    CHECK (read_ramp (0, large) == 0);     // one large read is enough
+    CHECK (pinned == 1);
+  }
   else CHECK (!"a known case");
   yee::readback_unref ();
   CHECK (pinned == 0);
@@ -155,3 +173,9 @@ def test_handle_of_another_device_than_the_current_one(program):
     """The events belong to the handle's device, as its stream does, and the caller's current
     device stays as it was."""
     run(program, "device")
+
+
+def test_a_few_small_reads_open_no_pool(program):
+    """Pinned buffers and threads cost more than they gain until 48 MB have been read: a run that
+    reads a few small fields takes plain copies."""
+    run(program, "few")
