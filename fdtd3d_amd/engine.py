@@ -436,7 +436,7 @@ class Batch:
         _bcheck(load_library().yee_batch_last_step_ms(self.h, ctypes.byref(ms)))
         return ms.value
 
-    def tuning(self, ncand: int = 12):
+    def tuning(self, ncand: int = 13):   # the candidates of yee_batch.hip (kCands)
         out = np.zeros(3, dtype=np.int32)
         ms = np.zeros(ncand, dtype=np.float64)
         _bcheck(load_library().yee_batch_tuning(self.h, out.ctypes.data, ms.ctypes.data, ncand))

@@ -178,3 +178,16 @@ def test_batch_launch_shapes_match_single_runs(precision, cand, engine_lib, monk
                 assert np.array_equal(b.field(s, f), e.field(f)), f"sim {s} {f}"
         e.close()
     b.close()
+
+
+def test_every_candidate_is_reported(engine_lib):
+    """The tuner's times of all its launch shapes, the register tiles among them, are in the default
+    report: as many as a caller with room for more gets."""
+    say("[gpu] batch tuner report")
+    b = Batch(make(4, 70))
+    b.prepare()
+    b.step(70)
+    ms = b.tuning()["candidate_ms"]
+    more = b.tuning(64)["candidate_ms"]
+    b.close()
+    assert all(v > 0 for v in ms) and sum(v > 0 for v in more) == len(ms)
