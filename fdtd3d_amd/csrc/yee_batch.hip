@@ -343,10 +343,73 @@ int build_graph (yee_batch *b, BatchGroup &grp, const Cand &c)
 }
 
 
+// `left` steps of every simulation with candidate c: each group runs all of them before the next one
+// starts.
+template <typename T>
+int run_steps (yee_batch *b, const Cand &c, int32_t left)
+{
+  int rc;
+  const char *use_graph = std::getenv ("YEE_BATCH_GRAPH");
+  // (a launch of the register tiles covers enough steps by itself)
+  const bool graphs = !(use_graph && std::strcmp (use_graph, "0") == 0) && c.two != 2;
+  for (BatchGroup &g : b->groupings[c.grouping])
+  {
+    if (graphs && !g.graph && left >= kGraphSteps && (rc = build_graph<T> (b, g, c))) return rc;
+    int32_t k = 0;
+    while (k < left)
+    {
+      if (graphs && g.graph && left - k >= b->graph_steps)
+      {
+        BHIP (hipGraphLaunch (g.graph, b->stream));
+        k += b->graph_steps;
+      }
+      else
+      {
+        // (the register tiles' launches share one advance)
+        const int kk = std::min (c.two == 2 ? kPlaneRun : cand_stride (b, c), left - k);
+        if ((rc = enqueue_steps<T> (b, g, c, kk))) return rc;
+        k += kk;
+      }
+    }
+  }
+  return YEE_OK;
+}
+
+// Of `left` steps with the register tiles, those past the last full launch that another candidate takes
+// in less time: how many, and the candidate.  The margin of a tile is that of a full launch, so
+// one of a single step takes 0.72 to 0.80 of a full launch's time in FP32 (8 steps) and 0.84 to 0.88 in FP64
+// (4): 64 simulations of 5.7e7 cells in FP32 1194 us, a full launch 1508, where the marching kernels take
+// 515 for one step and 538 for two.  The tuner's times decide where there are any.  Without, the
+// marching kernels take up to two steps of more than 3e6 cells (us for 1, 2, 3 steps, tiles and two
+// steps a launch: 3.9e6 cells FP32 85, 89, 93 and 63, 80, 128, FP64 113, 119, 125 and 103, 116, 205; 1.9e6
+// cells FP32 55, 57, 59 and 58, 72, 116).
+int32_t rest_steps (const yee_batch *b, int32_t left, int &cand)
+{
+  if (kCands[b->cand].two != 2) return 0;
+  const int full = cand_stride (b, kCands[b->cand]);
+  const int32_t rest = left % full;
+  if (b->tune_ms.empty ())
+  {
+    double cells = 0;
+    for (const yee_config &c : b->cfg) cells += (double) c.size[0] * (double) c.size[1];
+    cand = b->two_ok ? 5 : 2;
+    return cells > 3e6 && rest <= (b->two_ok ? 2 : 1) ? rest : 0;
+  }
+  int best = -1;
+  for (int c = 0; c < kNumCands; ++c)
+    if (kCands[c].two != 2 && b->tune_ms[c] > 0 && (best < 0 || b->tune_ms[c] < b->tune_ms[best])) best = c;
+  if (best < 0) return 0;
+  cand = best;
+  // (one step of a two-step candidate takes as long as two)
+  const int32_t paid = kCands[best].two == 1 ? rest + rest % 2 : rest;
+  return paid * b->tune_ms[best] < 0.8 * full * b->tune_ms[b->cand] ? rest : 0;
+}
+
 template <typename T>
 int step_impl (yee_batch *b, int32_t n)
 {
   int rc = YEE_OK;
+  bool forced = false;
   if (b->t + n > b->src_len && (rc = upload_sources<T> (b, std::max (b->t + n, 2 * b->src_len)))) return rc;
   // device pointers inside StepArgs do not change, but the source table may have moved
   BHIP (hipEventRecord (b->ev[0], b->stream));
@@ -368,6 +431,7 @@ int step_impl (yee_batch *b, int32_t n)
     if (b->cand != ci) rc = drop_graphs (b);
     if (rc) return rc;
     b->cand = ci;
+    forced = true;
   }
   // tuner: kTuneSteps ordinary steps of every simulation per candidate, timed, on the first
   // call that has room
@@ -409,32 +473,10 @@ int step_impl (yee_batch *b, int32_t n)
   }
   // too few steps to tune (without the register tiles: one group, 64-row tiles)
   if (b->cand < 0) b->cand = b->plane_ok ? kPlaneCand : 2;
-  const Cand &c = kCands[b->cand];
-  const char *use_graph = std::getenv ("YEE_BATCH_GRAPH");
-  // (a launch of the register tiles covers enough steps by itself)
-  const bool graphs = !(use_graph && std::strcmp (use_graph, "0") == 0) && c.two != 2;
-  // each group runs all the remaining steps before the next one starts
   const int32_t left = n - done;
-  for (BatchGroup &g : b->groupings[c.grouping])
-  {
-    if (graphs && !g.graph && left >= kGraphSteps && (rc = build_graph<T> (b, g, c))) return rc;
-    int32_t k = 0;
-    while (k < left)
-    {
-      if (graphs && g.graph && left - k >= b->graph_steps)
-      {
-        BHIP (hipGraphLaunch (g.graph, b->stream));
-        k += b->graph_steps;
-      }
-      else
-      {
-        // (the register tiles' launches share one advance)
-        const int kk = std::min (c.two == 2 ? kPlaneRun : cand_stride (b, c), left - k);
-        if ((rc = enqueue_steps<T> (b, g, c, kk))) return rc;
-        k += kk;
-      }
-    }
-  }
+  int other = b->cand;
+  const int32_t rest = forced ? 0 : rest_steps (b, left, other);
+  if ((rc = run_steps<T> (b, kCands[b->cand], left - rest)) || (rc = run_steps<T> (b, kCands[other], rest))) return rc;
   b->t += left;
   BHIP (hipEventRecord (b->ev[1], b->stream));
   BHIP (hipEventSynchronize (b->ev[1]));

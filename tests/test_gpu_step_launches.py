@@ -285,3 +285,40 @@ def test_profile_is_per_step(args, one_launch, precision, engine_lib):
     print(f"[gpu] profile {args.split()[0]} precision {precision}: {p}", flush=True)
     assert p["incident_ms"] > 0 and (p["fused_ms"] > 0) == one_launch and (p["e_half_ms"] > 0) != one_launch
     assert sum(groups) <= 1.05 * p["step_ms"]
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("mu", [False, True])
+def test_batch_steps_past_a_full_launch(mu, precision, engine_lib, monkeypatch):
+    """The steps of a call past the last full launch of the register tiles may take another launch
+    shape: 3.3e6 cells (where one or two steps do without the tuner's times), calls of every remainder of
+    4 and 8 steps before the tuner has run and after it, against single runs, bit for bit."""
+    calls = [1, 1, 2, 3, 4, 5, 6, 7, 9, 10, 62, 1, 2, 3, 4, 5, 6, 7, 9]
+    sims = [f"--2d-tmz --size x:{a},y:{b} --use-pml --pml-size x:6,y:7 --point-source x:{a // 2},y:{b // 2} --point-source-ez "
+            f"--time-steps {sum(calls)}" for a, b in ((1303, 1250), (1290, 1301))]
+    cfgs = [parse_args(s.split(), precision=precision) for s in sims]
+    print(f"[gpu] batch remainders, mu {mu}, precision {precision}", flush=True)
+    rng = np.random.default_rng(23)
+    eps = [rng.uniform(1.0, 5.0, size=c.shape) for c in cfgs]
+    mus = [rng.uniform(1.0, 2.0, size=c.shape) for c in cfgs]
+    b = Batch(cfgs)
+    for s in range(2):
+        b.set_material(s, "eps", eps[s])
+        if mu:
+            b.set_material(s, "mu", mus[s])
+    b.prepare()
+    for n in calls:
+        b.step(n)
+    assert b.time == sum(calls)
+    monkeypatch.setenv("YEE_KERNEL", "split")
+    for s, c in enumerate(cfgs):
+        e = Engine(c)
+        e.set_material("eps", eps[s])
+        if mu:
+            e.set_material("mu", mus[s])
+        e.prepare()
+        e.step(sum(calls))
+        for f in ("Ez", "Hx", "Hy", "Dz", "Bx", "By"):
+            assert np.array_equal(b.field(s, f), e.field(f)), f"sim {s} {f}"
+        e.close()
+    b.close()
