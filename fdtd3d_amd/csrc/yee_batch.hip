@@ -290,6 +290,13 @@ int cand_stride (const yee_batch *b, const Cand &c)
   return c.two == 2 ? (b->wsize == 4 ? BATCH_STEPS (float) : BATCH_STEPS (double)) : (c.two ? 2 : 1);
 }
 
+// The candidate of a step: the tuner's, or, before a call with steps enough to tune, the register tiles
+// (without them: one group, 64-row tiles).
+int current_cand (const yee_batch *b)
+{
+  return b->cand >= 0 ? b->cand : (b->plane_ok ? kPlaneCand : 2);
+}
+
 // A mu grid rules out the two-step kernel, short memory the register tiles.
 bool cand_ok (const yee_batch *b, const Cand &c)
 {
@@ -375,8 +382,8 @@ int run_steps (yee_batch *b, const Cand &c, int32_t left)
   return YEE_OK;
 }
 
-// Of `left` steps with the register tiles, those past the last full launch that another candidate takes
-// in less time: how many, and the candidate.  The margin of a tile is that of a full launch, so
+// Of `left` steps with candidate `cand`, the register tiles, those past the last full launch that another
+// takes in less time: how many, and that candidate in `cand`.  The margin of a tile is that of a full launch, so
 // one of a single step takes 0.72 to 0.80 of a full launch's time in FP32 (8 steps) and 0.84 to 0.88 in FP64
 // (4): 64 simulations of 5.7e7 cells in FP32 1194 us, a full launch 1508, where the marching kernels take
 // 515 for one step and 538 for two.  The tuner's times decide where there are any.  Without, the
@@ -385,8 +392,9 @@ int run_steps (yee_batch *b, const Cand &c, int32_t left)
 // cells FP32 55, 57, 59 and 58, 72, 116).
 int32_t rest_steps (const yee_batch *b, int32_t left, int &cand)
 {
-  if (kCands[b->cand].two != 2) return 0;
-  const int full = cand_stride (b, kCands[b->cand]);
+  const int tiles = cand;
+  if (kCands[tiles].two != 2) return 0;
+  const int full = cand_stride (b, kCands[tiles]);
   const int32_t rest = left % full;
   if (b->tune_ms.empty ())
   {
@@ -402,7 +410,7 @@ int32_t rest_steps (const yee_batch *b, int32_t left, int &cand)
   cand = best;
   // (one step of a two-step candidate takes as long as two)
   const int32_t paid = kCands[best].two == 1 ? rest + rest % 2 : rest;
-  return paid * b->tune_ms[best] < 0.8 * full * b->tune_ms[b->cand] ? rest : 0;
+  return paid * b->tune_ms[best] < 0.8 * full * b->tune_ms[tiles] ? rest : 0;
 }
 
 template <typename T>
@@ -437,6 +445,7 @@ int step_impl (yee_batch *b, int32_t n)
   // call that has room
   if (b->cand < 0 && n - done >= kTuneTotal)
   {
+    if ((rc = drop_graphs (b))) return rc;   // those of the steps before
     b->tune_ms.assign (kNumCands, 0.0);
     hipEvent_t e0, e1;
     BHIP (hipEventCreate (&e0));
@@ -471,12 +480,11 @@ int step_impl (yee_batch *b, int32_t n)
     (void) hipEventDestroy (e0);
     (void) hipEventDestroy (e1);
   }
-  // too few steps to tune (without the register tiles: one group, 64-row tiles)
-  if (b->cand < 0) b->cand = b->plane_ok ? kPlaneCand : 2;
   const int32_t left = n - done;
-  int other = b->cand;
+  const int main = current_cand (b);
+  int other = main;
   const int32_t rest = forced ? 0 : rest_steps (b, left, other);
-  if ((rc = run_steps<T> (b, kCands[b->cand], left - rest)) || (rc = run_steps<T> (b, kCands[other], rest))) return rc;
+  if ((rc = run_steps<T> (b, kCands[main], left - rest)) || (rc = run_steps<T> (b, kCands[other], rest))) return rc;
   b->t += left;
   BHIP (hipEventRecord (b->ev[1], b->stream));
   BHIP (hipEventSynchronize (b->ev[1]));
@@ -806,9 +814,9 @@ int yee_batch_last_step_ms (yee_batch *b, double *ms)
 int yee_batch_tuning (yee_batch *b, int32_t out[3], double *cand_ms, int32_t ncand)
 {
   if (!b || !out) return batch_fail (YEE_EINVAL, "null argument");
-  if (b->cand >= 0)
+  if (b->cand >= 0 || b->t > 0)
   {
-    const Cand &c = kCands[b->cand];
+    const Cand &c = kCands[current_cand (b)];
     const std::vector<BatchGroup> &gs = b->groupings[c.grouping];
     out[0] = kLx[c.sel];
     out[1] = gs.empty () ? 0 : (c.two == 2 ? gs[0].nplane : (gs[0].ntiles[c.two][c.sel] + 3) / 4);

@@ -191,3 +191,17 @@ def test_every_candidate_is_reported(engine_lib):
     more = b.tuning(64)["candidate_ms"]
     b.close()
     assert all(v > 0 for v in ms) and sum(v > 0 for v in more) == len(ms)
+
+
+def test_tuner_runs_on_the_first_call_with_room(engine_lib):
+    """Short calls before it do not keep the tuner off, and their launch shape is reported until then."""
+    say("[gpu] batch tuner after short calls")
+    b = Batch(make(4, 120))
+    b.prepare()
+    b.step(5)
+    b.step(20)
+    t = b.tuning()
+    assert t["workgroups"] > 0 and not any(t["candidate_ms"])
+    b.step(70)
+    assert all(v > 0 for v in b.tuning()["candidate_ms"])
+    b.close()
