@@ -1113,11 +1113,17 @@ int get_field (yee_handle *h, int32_t comp, void *out, bool widen)
 
 // The next steps of a 1D or 2D run in one launch (yee_plane.hip), at most `ahead`.  t = 0 (which only
 // fires the sources), Drude media, test functions, current sources and a hard source outside the
-// updated cells take the half-step kernels.
-bool plane_runs (const yee_handle *h)
+// updated cells take the half-step kernels, and so does a single step of a 2D run with TF/SF (the
+// corrections of eight steps are read before the first) or with two buffers of E and H that the
+// last-level cache does not hold, where the half steps, in place, touch one.  us of a call of one step,
+// tiles and half steps: FP32 with TF/SF 100^2 29 and 25, 2000x1500 57 and 52, 5000x4000 292 and 189;
+// FP64 without 2000x1500 57 and 57, 2500x2000 110 and 83, 3000x2500 153 and 112; FP32 without 2000x1500
+// 41 and 48, 3000x2500 82 and 82, 5000x4000 204 and 179.  (FP64 with TF/SF 1403x977 43 and 48.)
+bool plane_runs (const yee_handle *h, int32_t ahead)
 {
+  const bool single = ahead == 1 && line_axis (h->cfg) < 0 && (h->use_tfsf () || 6.0 * (double) h->ncell * (double) h->wsize > 200e6);
   return h->plane && h->t > 0 && !h->fn_any () && !(h->cfg.current_source & 0x3fu)
-         && (!(h->cfg.point_source & 0x3fu) || source_in_update (h));
+         && (!(h->cfg.point_source & 0x3fu) || source_in_update (h)) && !single;
 }
 
 template <typename T>
@@ -1168,7 +1174,7 @@ namespace yee {
 
 int engine_steps (yee_handle *h, int32_t ahead, int32_t &done)
 {
-  if (plane_runs (h)) return h->fp32 () ? plane_advance<float> (h, ahead, done) : plane_advance<double> (h, ahead, done);
+  if (plane_runs (h, ahead)) return h->fp32 () ? plane_advance<float> (h, ahead, done) : plane_advance<double> (h, ahead, done);
   done = 1;
   return engine_step_once (h, ahead);
 }

@@ -322,3 +322,31 @@ def test_batch_steps_past_a_full_launch(mu, precision, engine_lib, monkeypatch):
             assert np.array_equal(b.field(s, f), e.field(f)), f"sim {s} {f}"
         e.close()
     b.close()
+
+
+@pytest.mark.parametrize("precision,nb", [(4, 2886), (8, 2041)])
+@pytest.mark.parametrize("fits", [True, False])
+def test_single_steps_of_2d_runs(fits, precision, nb, engine_lib, monkeypatch):
+    """A single step takes the tiles where two buffers of E and H fill at most 200 MB and half steps in
+    place above; both sides of that line, mixed with calls of several steps: the half-step kernels'
+    fields and D / B, bit for bit."""
+    na = int(200e6 / (6 * precision) / nb) + (0 if fits else 1)
+    assert (6 * precision * na * nb <= 200e6) == fits
+    cfg = parse_args(f"--2d-tmz --size x:{na},y:{nb} --use-pml --pml-size x:7,y:6 --point-source x:{na // 2},y:{nb // 2} "
+                     "--point-source-ez --time-steps 60".split(), precision=precision)
+    eps = np.random.default_rng(29).uniform(1.0, 5.0, size=cfg.shape)
+    calls = [1, 1, 1, 9, 1, 2, 17, 1]
+    print(f"[gpu] single steps {na}x{nb} precision {precision}", flush=True)
+    out = []
+    for kernel in ("split", ""):
+        monkeypatch.setenv("YEE_KERNEL", kernel)
+        eng = Engine(cfg)
+        eng.set_material("eps", eps)
+        eng.prepare()
+        for n in calls:
+            eng.step(n)
+        out.append({c: eng.field_raw(c) for c in ("Ez", "Hx", "Hy", "Dz", "Bx", "By")})
+        eng.close()
+    for c, v in out[0].items():
+        assert np.array_equal(out[1][c], v), c
+    assert np.abs(out[0]["Ez"]).max() > 0
