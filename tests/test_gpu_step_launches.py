@@ -350,3 +350,39 @@ def test_single_steps_of_2d_runs(fits, precision, nb, engine_lib, monkeypatch):
     for c, v in out[0].items():
         assert np.array_equal(out[1][c], v), c
     assert np.abs(out[0]["Ez"]).max() > 0
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("args", [
+    "--2d-tmz --size x:98,y:67 --use-pml --pml-size x:6,y:5 --use-tfsf --tfsf-size-left x:12,y:12 --tfsf-size-right x:12,y:12 "
+    "--angle-teta 90 --angle-phi 30",
+    "--2d-tex --size y:51,z:99 --use-pml --pml-size y:5,z:6 --point-source y:25,z:50 --point-source-ey",
+    "--2d-tmy --size x:66,z:52 --point-source x:30,z:20 --point-source-ey",
+    "--1d-exhy --size z:421 --use-pml --pml-size z:9 --use-tfsf --tfsf-size-left z:60 --tfsf-size-right z:0 --angle-teta 0 "
+    "--angle-phi 0",
+    "--1d-eyhz --size x:195 --point-source x:90 --point-source-ey",
+])
+def test_double_material_precision_in_one_launch(args, precision, engine_lib, monkeypatch):
+    """Runs with double material precision take the tiles and lines as well, with the 8-cell averages
+    of each component: the half-step kernels' fields and D / B, bit for bit."""
+    cfg = parse_args((args + " --use-double-material-precision --time-steps 70").split(), precision=precision)
+    assert cfg.double_material
+    rng = np.random.default_rng(31)
+    eps, mu = rng.uniform(1.0, 5.0, size=cfg.material_shape), rng.uniform(1.0, 2.0, size=cfg.material_shape)
+    print(f"[gpu] double material precision {args.split()[0]} precision {precision}", flush=True)
+    out = []
+    for kernel, calls in (("split", [70]), ("", [70]), ("", [1, 2, 7, 33, 27])):
+        monkeypatch.setenv("YEE_KERNEL", kernel)
+        eng = Engine(cfg)
+        eng.set_material("eps", eps)
+        eng.set_material("mu", mu)
+        eng.prepare()
+        for n in calls:
+            eng.step(n)
+        names = list(cfg.components) + ([("D" if c[0] == "E" else "B") + c[1] for c in cfg.components] if cfg.use_pml else [])
+        out.append({c: eng.field_raw(c) for c in names})
+        eng.close()
+    for c, v in out[0].items():
+        assert np.array_equal(out[1][c], v), c
+        assert np.array_equal(out[2][c], v), c
+    assert any(np.abs(v).max() > 0 for v in out[0].values())
