@@ -1340,17 +1340,24 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     // x chunks: a CU holds 16 waves of this kernel (<= 128 VGPRs each), i.e. 16 / (waves per
     // row) workgroups.  The chunk count minimises rounds of resident workgroups x planes per
     // chunk (+1 for the chunk's first plane, read twice): enough workgroups to fill every CU,
-    // and no last round left mostly empty.  Rows of five waves put two on one SIMD, and a third
-    // workgroup (15 of the 16 waves) measures as not resident: counted as two a CU, with a fifth
-    // added for more than one round, 251x187x301 FP32 takes 157 us of 192 (6 chunks of 9),
-    // 320^3 392 of 450 (3 of 5), 220x260x300 193 of 230 (4 of 13) and FP64 458 of 512 (2 of 13).
+    // and no last round left mostly empty.  Rows of five waves put two on one SIMD: in FP32 a plane takes
+    // 1, 1.4 and 2.5 times as long with one, two and three workgroups a CU, so that one round of two is the
+    // best there is and a round of three costs 1.8 of it.  Sweep with the count of these weights, and of
+    // whole rounds of three: 251x187x301 157 us of 192 (6 chunks of 9), 256x256x264 219 of 253 (4 of 13),
+    // 400x150x320 223 of 266 (7 of 11), 118x380x264 153 of 162 (7 of 4), 397x363x267 522 of 552 (7 of 13),
+    // 298x233x284 264 of 284 (12 of 7; 259 with 4), 120x400x264 168 (4 of both).  FP64 is counted as two a CU
+    // with a fifth added for more than one round: 256x256x264 536 of 635 (2 of 3), 220x260x300 458 of 512 (2
+    // of 13), 400x150x257 524 of 539 (19 of 11), 282x386x303 1035 of 1090 (7 of 2; the weights choose 2 too).
     // (Other row lengths gain nothing from either: 256^3 FP64 400 us, 412 with one round.)
     const int64_t waves = (h->n[2] + 63) / 64;
-    const bool five = waves == 5;
-    const int64_t slots = (int64_t) h->ncu * (five ? 2 : std::max<int64_t> (1, 16 / waves));
+    const bool five32 = waves == 5 && h->fp32 (), five64 = waves == 5 && !h->fp32 ();
+    const int64_t slots = (int64_t) h->ncu * (five64 ? 2 : std::max<int64_t> (1, 16 / waves));
     auto chunk_cost = [&] (int64_t c) {
-      const int64_t rounds = (h->fused_nstrips * c + slots - 1) / slots;
-      return (five && rounds > 1 ? 1.2 : 1.0) * (double) rounds * (double) ((planes + c - 1) / c + 1);
+      const int64_t full = h->fused_nstrips * c / slots, rest = h->fused_nstrips * c % slots;
+      double rounds = (double) full + (rest > 0 ? 1.0 : 0.0);
+      if (five32) rounds = 2.5 * (double) full + (rest > 2 * h->ncu ? 2.5 : (rest > h->ncu ? 1.4 : (rest > 0 ? 1.0 : 0.0)));
+      if (five64 && rounds > 1) rounds *= 1.2;
+      return rounds * (double) ((planes + c - 1) / c + 1);
     };
     double best = 1e300;
     for (int64_t c = 1; c <= planes; ++c) best = std::min (best, chunk_cost (c));
@@ -1360,9 +1367,13 @@ int yee_create (const yee_config *cfg, yee_handle **out)
     // workgroups that run together stay on the same planes, unless one round fills the chip.  Sweep of
     // 384^3 630 us of 657 (11 chunks before), 448^3 970 of 1006 (7), 512^3 1410 of 1457 (2; the same
     // order on a faster card, 1196 of 1270), 512x300x420 735 of 768; 360^3 545 of 536 (3, which fill it).
-    // Longer rows lose (200x500x640 725 of 660), as do short sweeps (100x400x400 147 of 142).
+    // Longer rows lose (200x500x640 725 of 660), as do short sweeps (100x400x400 147 of 142); from 200
+    // planes on 222x300x330 takes 291 of 318, x384 309 of 341, x448 343 of 337, x512 374 of 379.  One round
+    // fills the chip with 95 % of its workgroups, 93 % in rows of six waves (240 strips in two chunks, 94 %:
+    // 260x500x330 562 of 517, x384 585 of 585, but x448 648 of 661 and x512 705 of 726).
+    const int64_t filled = slots * (waves == 6 ? 93 : 95) / 100;
     if (h->fp32 () && waves >= 6 && waves <= 8 && planes >= 200
-        && !(h->fused_nstrips * nch <= slots && h->fused_nstrips * nch > slots * 95 / 100))
+        && !(h->fused_nstrips * nch <= slots && h->fused_nstrips * nch > filled))
       nch = std::max (nch, std::min<int64_t> (32, planes / 10));
     if (const char *e = std::getenv ("YEE_FUSED_CHUNKS")) nch = std::max (1, std::atoi (e));
     nch = std::min (nch, planes);

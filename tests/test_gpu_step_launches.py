@@ -386,3 +386,19 @@ def test_double_material_precision_in_one_launch(args, precision, engine_lib, mo
         assert np.array_equal(out[1][c], v), c
         assert np.array_equal(out[2][c], v), c
     assert any(np.abs(v).max() > 0 for v in out[0].values())
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+@pytest.mark.parametrize("x,y,z", [(31, 40, 257), (24, 560, 260), (12, 1100, 320), (203, 30, 330)])
+def test_sweep_chunks_of_long_rows(x, y, z, precision, engine_lib, monkeypatch):
+    """Rows of five and six waves with fewer strips than compute units, one to two strips a unit and
+    more than two: however the sweep is cut into chunks, the half steps' fields, bit for bit."""
+    args = f"--3d --size x:{x},y:{y},z:{z} --use-pml --pml-size x:3,y:4,z:5 --point-source x:{x // 2},y:{y // 2},z:{z // 2} " \
+           "--point-source-ez --time-steps 12"
+    print(f"[gpu] chunks {x}x{y}x{z} precision {precision}", flush=True)
+    eps = np.random.default_rng(37).uniform(1.0, 4.0, size=(x, y, z))
+    ref = _run(args, precision, monkeypatch, "split", eps, 12)
+    got = _run(args, precision, monkeypatch, "fused", eps, 12)
+    for n, v in ref.items():
+        assert np.array_equal(got[n], v), n
+    assert np.abs(ref["Ez"]).max() > 0
