@@ -1654,6 +1654,8 @@ int yee_prepare (yee_handle *h)
     if (rc) return rc;
   }
   HIP_TRY (hipStreamSynchronize (h->stream));
+  // the two parts of complex fields take the same steps in one launch (yee_step)
+  if (h->imag) h->plane = h->imag->plane = h->plane && h->imag->plane;
   h->prepared = true;
   return YEE_OK;
 }

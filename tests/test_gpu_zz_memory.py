@@ -86,3 +86,28 @@ def test_batch_in_short_memory(engine_lib):
             b.close()
     for c, v in ref.items():
         assert np.array_equal(got[c], v), c
+
+
+def test_factors_for_one_part_of_complex_fields(engine_lib):
+    """9 words a cell free at yee_prepare: the imaginary part, prepared first, gets its factors (6) and
+    the real part does not.  Both parts then take half steps, step for step."""
+    eps = np.random.default_rng(2).uniform(1.0, 3.0, size=(3600, 3500))
+
+    def fields(ctx):
+        cfg = parse_args(ARGS.split(), precision=8)
+        cfg.complex_fields = True
+        eng = Engine(cfg)
+        try:
+            eng.set_material("eps", eps)
+            with ctx:
+                eng.prepare()
+                eng.step(12)
+            return {f"{part} {c}": e.field_raw(c) for part, e in (("real", eng), ("imag", eng.imag())) for c in ("Ez", "Hx", "Dz")}
+        finally:
+            eng.close()
+
+    ref = fields(contextlib.nullcontext())
+    got = fields(only(9 * WORD))
+    for c, v in ref.items():
+        assert np.array_equal(got[c], v), c
+    assert min(np.abs(ref["real Ez"]).max(), np.abs(ref["imag Ez"]).max()) > 0
