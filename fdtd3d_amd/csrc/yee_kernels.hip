@@ -1079,20 +1079,20 @@ __global__ __launch_bounds__ (64 * MAXW) void step_3d_fused (StepArgs<T> a)
 // TMz half-steps (Ez; Hx, Hy) on [1, N-1)^2; one thread per cell, y lane-contiguous
 // ---------------------------------------------------------------------------------------
 template <typename T, int MODE>
-__device__ __forceinline__ void tmz_e_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
+__device__ __forceinline__ void tmz_e_cell (const StepArgs<T> &a, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;   // == 1
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = special_cell<T, MODE> (a, fl, p, 2);
+  const bool special = special_cell<T, MODE> (a, 0u, p, 2);
   T fo;
   Old<T> dold;
   PmlCoef<T> pc2;
   load_old<T, MODE, 2> (a, q, p, special, fo, dold, pc2);
   const T *Hx = a.f[3], *Hy = a.f[4];
   T v[4] = { Hy[q - sx], Hy[q], Hx[q - sy], Hx[q] };
-  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 2, 2> (a, i, j, 0, v);
+  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 2, 2> (a, i, j, 0, v);
   // Ez sits on the eps point: the 2-cell average reads the same cell twice
   const T e = a.eps ? a.eps[q] : a.eps_u;
   const T mat = a.matc[2] ? a.matc[2][q] : avg2 (e, e);
@@ -1103,17 +1103,17 @@ __device__ __forceinline__ void tmz_e_cell (const StepArgs<T> &a, uint32_t fl, i
     om = avg2 (o, o);
     ga = avg2 (g, g);
   }
-  update_cell<T, MODE, 2> (a, fl, q, p, fo, dold, curl_rhs<T, 2> (a, v, p), mat, special, om, ga, pc2);
+  update_cell<T, MODE, 2> (a, 0u, q, p, fo, dold, curl_rhs<T, 2> (a, v, p), mat, special, om, ga, pc2);
 }
 
 template <typename T, int MODE>
-__device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
+__device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = special_cell<T, MODE> (a, fl, p, 2);
+  const bool special = special_cell<T, MODE> (a, 0u, p, 2);
   T fo3, fo4;
   Old<T> do3, do4;
   PmlCoef<T> pc3, pc4;
@@ -1124,7 +1124,7 @@ __device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, uint32_t fl, i
   // Hx: Ey operands absent (0), Ez at (i, j) and (i, j+1); Hy: Ez at (i, j) and (i+1, j), Ex absent
   T vx[4] = { (T) 0, (T) 0, ez, Ez[q + sy] };
   T vy[4] = { ez, Ez[q + sx], (T) 0, (T) 0 };
-  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0))
+  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0))
   {
     tfsf_apply<T, 3, 2> (a, i, j, 0, vx);
     tfsf_apply<T, 4, 2> (a, i, j, 0, vy);
@@ -1160,8 +1160,8 @@ __device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, uint32_t fl, i
       gmy = sum4 (g[q], g[q], g[q + sx], g[q + sx]);
     }
   }
-  update_cell<T, MODE, 3> (a, fl, q, p, fo3, do3, curl_rhs<T, 3> (a, vx, p), mx, special, omx, gmx, pc3);
-  update_cell<T, MODE, 4> (a, fl, q, p, fo4, do4, curl_rhs<T, 4> (a, vy, p), my, special, omy, gmy, pc4);
+  update_cell<T, MODE, 3> (a, 0u, q, p, fo3, do3, curl_rhs<T, 3> (a, vx, p), mx, special, omx, gmx, pc3);
+  update_cell<T, MODE, 4> (a, 0u, q, p, fo4, do4, curl_rhs<T, 4> (a, vy, p), my, special, omy, gmy, pc4);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1169,13 +1169,13 @@ __device__ __forceinline__ void tmz_h_cell (const StepArgs<T> &a, uint32_t fl, i
 // (Hy for Ex, Hx for Ey) read as 0, as for TMz; y lane-contiguous, updated in place
 // ---------------------------------------------------------------------------------------
 template <typename T, int MODE>
-__device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
+__device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;   // == 1
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = special_cell<T, MODE> (a, fl, p, 2);
+  const bool special = special_cell<T, MODE> (a, 0u, p, 2);
   T fo0, fo1;
   Old<T> do0, do1;
   PmlCoef<T> pc0, pc1;
@@ -1186,7 +1186,7 @@ __device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, uint32_t fl, i
   // Ex: Hz at (i, j-1) and (i, j), Hy absent; Ey: Hx absent, Hz at (i-1, j) and (i, j)
   T vx[4] = { Hz[q - sy], hz, (T) 0, (T) 0 };
   T vy[4] = { (T) 0, (T) 0, Hz[q - sx], hz };
-  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0))
+  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0))
   {
     tfsf_apply<T, 0, 2> (a, i, j, 0, vx);
     tfsf_apply<T, 1, 2> (a, i, j, 0, vy);
@@ -1218,18 +1218,18 @@ __device__ __forceinline__ void tez_e_cell (const StepArgs<T> &a, uint32_t fl, i
       gym = avg2 (a.ge[q], a.ge[q + sy]);
     }
   }
-  update_cell<T, MODE, 0> (a, fl, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm, pc0);
-  update_cell<T, MODE, 1> (a, fl, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym, pc1);
+  update_cell<T, MODE, 0> (a, 0u, q, p, fo0, do0, curl_rhs<T, 0> (a, vx, p), ex_m, special, oxm, gxm, pc0);
+  update_cell<T, MODE, 1> (a, 0u, q, p, fo1, do1, curl_rhs<T, 1> (a, vy, p), ey_m, special, oym, gym, pc1);
 }
 
 template <typename T, int MODE>
-__device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, uint32_t fl, int i, int j)
+__device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, int i, int j)
 {
   const int64_t sx = a.sx;
   const int sy = a.sy;
   const int64_t q = (int64_t) i * sx + (int64_t) j * sy;
   const int p[3] = { i, j, 0 };
-  const bool special = special_cell<T, MODE> (a, fl, p, 2);
+  const bool special = special_cell<T, MODE> (a, 0u, p, 2);
   T fo5;
   Old<T> do5;
   PmlCoef<T> pc5;
@@ -1237,7 +1237,7 @@ __device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, uint32_t fl, i
   const T *Ex = a.f[0], *Ey = a.f[1];
   // Hz: Ex at (i, j) and (i, j+1), Ey at (i, j) and (i+1, j)
   T vz[4] = { Ex[q], Ex[q + sy], Ey[q], Ey[q + sx] };
-  if (a.tfsf && !(fl & kNoTfsf) && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 5, 2> (a, i, j, 0, vz);
+  if (a.tfsf && tfsf_near<T, 2> (a, i, j, 0)) tfsf_apply<T, 5, 2> (a, i, j, 0, vz);
   // 4-cell transverse average
   T hz_m = a.mu_u;
   if (a.matc[5])
@@ -1256,7 +1256,7 @@ __device__ __forceinline__ void tez_h_cell (const StepArgs<T> &a, uint32_t fl, i
     if (o) ozm = sum4 (o[q], o[q + sy], o[q + sx], o[q + sx + sy]);
     if (g) gzm = sum4 (g[q], g[q + sy], g[q + sx], g[q + sx + sy]);
   }
-  update_cell<T, MODE, 5> (a, fl, q, p, fo5, do5, curl_rhs<T, 5> (a, vz, p), hz_m, special, ozm, gzm, pc5);
+  update_cell<T, MODE, 5> (a, 0u, q, p, fo5, do5, curl_rhs<T, 5> (a, vz, p), hz_m, special, ozm, gzm, pc5);
 }
 
 template <typename T, int MODE>
@@ -1267,8 +1267,8 @@ __global__ __launch_bounds__ (256) void e_half_tez (StepArgs<T> a)
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
   // outside the Drude box: the PML update (see e_half_3d)
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_e_cell<T, 1> (a, 0u, i, j);
-  else tez_e_cell<T, MODE> (a, 0u, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_e_cell<T, 1> (a, i, j);
+  else tez_e_cell<T, MODE> (a, i, j);
 }
 
 template <typename T, int MODE>
@@ -1278,8 +1278,8 @@ __global__ __launch_bounds__ (256) void h_half_tez (StepArgs<T> a)
   const int i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_h_cell<T, 1> (a, 0u, i, j);
-  else tez_h_cell<T, MODE> (a, 0u, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tez_h_cell<T, 1> (a, i, j);
+  else tez_h_cell<T, MODE> (a, i, j);
 }
 
 template <typename T, int MODE>
@@ -1290,8 +1290,8 @@ __global__ __launch_bounds__ (256) void e_half_tmz (StepArgs<T> a)
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
   // outside the Drude box: the PML update (see e_half_3d)
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_e_cell<T, 1> (a, 0u, i, j);
-  else tmz_e_cell<T, MODE> (a, 0u, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_e_cell<T, 1> (a, i, j);
+  else tmz_e_cell<T, MODE> (a, i, j);
 }
 
 template <typename T, int MODE>
@@ -1301,8 +1301,8 @@ __global__ __launch_bounds__ (256) void h_half_tmz (StepArgs<T> a)
   const int i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i < 1 || i >= a.nx - 1 || j < 1 || j >= a.ny - 1) return;
   const int p[3] = { i, j, 0 };
-  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_h_cell<T, 1> (a, 0u, i, j);
-  else tmz_h_cell<T, MODE> (a, 0u, i, j);
+  if (MODE == 2 && !in_drude_box (a, p, 2)) tmz_h_cell<T, 1> (a, i, j);
+  else tmz_h_cell<T, MODE> (a, i, j);
 }
 
 // ---------------------------------------------------------------------------------------

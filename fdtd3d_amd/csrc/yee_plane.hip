@@ -152,7 +152,7 @@ __device__ __forceinline__ void tile_load (const StepArgs<T> &a, int i0, int j, 
 
 template <typename T, class S, int RW, int COMP, bool PML>
 __device__ __forceinline__ void tile_factors (const StepArgs<T> &a, const bool (&in)[RW], const bool (&sp)[RW],
-                                              TileComp<T, RW> &x,                                              const TileRaw<T, RW> &w)
+                                              TileComp<T, RW> &x, const TileRaw<T, RW> &w)
 {
   const T modc = COMP >= 3 ? a.mu0 : a.eps0;
 #pragma unroll
