@@ -1,5 +1,5 @@
 // Batched TMz sweep: many independent TMz simulations (different grid sizes, materials and
-// sources) advanced together, two launches per time step for the whole batch.
+// sources) advanced together, a launch for one, two or several time steps of the whole batch.
 //
 // The reference runs one simulation per process (Source/main.cpp); this has no counterpart
 // there.  Every simulation is exactly what a single yee_handle with the same configuration
@@ -10,10 +10,10 @@
 // Infinity Cache of the MI355X sits in front of HBM): a call of yee_batch_step advances one
 // group by all its steps before the next group starts, so after the first step a group's
 // fields are read from the cache rather than from HBM.  Per step of a group: batch_tmz_step
-// (E and H fused, double-buffered state) over the group's tile table, then batch_advance of
-// its simulations' step counters.  The counters live in device memory (one per simulation),
+// (E and H fused, double-buffered state; batch_tmz_step2 takes two steps, batch_plane_steps up to
+// eight) over the group's tile table, then batch_advance of its simulations' step counters.  The counters live in device memory (one per simulation),
 // so a graph captured over several steps of a group is replayed as often as needed.  The
-// grouping budget and the tile length (x rows per tile) are picked by a short timing of the
+// grouping budget, the tile length (x rows per tile) and the kernel are picked by a short timing of the
 // first steps (every candidate computes the same values, so the tuning steps are ordinary
 // steps).
 #include <hip/hip_runtime.h>

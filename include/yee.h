@@ -404,10 +404,10 @@ int yee_adjoint_timing (yee_handle *h, double out[2]);
 /*
  * Batched TMz sweep: `nsim` independent TMz simulations (each its own yee_config: size, PML,
  * point source; one precision for the batch; no TF/SF, no metamaterials) advanced together,
- * two launches per time step for the whole batch, replayed from a captured HIP graph.  The
- * reference runs one simulation per process (Source/main.cpp); the batch has no counterpart
- * there and replaces running the same simulations one by one.  Every member computes exactly
- * what a yee_handle with its configuration computes.  Errors: yee_batch_last_error().
+ * a launch covering one, two or several time steps of the whole batch.  The reference runs one
+ * simulation per process (Source/main.cpp); the batch has no counterpart there and replaces
+ * running the same simulations one by one.  Every member computes exactly what a yee_handle
+ * with its configuration computes.  Errors: yee_batch_last_error().
  */
 typedef struct yee_batch yee_batch;
 
