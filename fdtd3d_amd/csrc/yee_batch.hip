@@ -481,10 +481,10 @@ int step_impl (yee_batch *b, int32_t n)
     (void) hipEventDestroy (e1);
   }
   const int32_t left = n - done;
-  const int main = current_cand (b);
-  int other = main;
+  const int cand = current_cand (b);
+  int other = cand;
   const int32_t rest = forced ? 0 : rest_steps (b, left, other);
-  if ((rc = run_steps<T> (b, kCands[main], left - rest)) || (rc = run_steps<T> (b, kCands[other], rest))) return rc;
+  if ((rc = run_steps<T> (b, kCands[cand], left - rest)) || (rc = run_steps<T> (b, kCands[other], rest))) return rc;
   b->t += left;
   BHIP (hipEventRecord (b->ev[1], b->stream));
   BHIP (hipEventSynchronize (b->ev[1]));

@@ -139,8 +139,8 @@ struct Staging
     return false;
   }
 
-  // Buffers, events and threads for reads on `dev`, the current device; false if they are another device's or cannot
-  // be had (the next check of a launch must not find that error).
+  // Buffers, events and threads for reads on `dev`, the current device; false if they are another
+  // device's or cannot be had (the next check of a launch must not find that error).
   bool open (int dev)
   {
     if (buf) return dev == device;
